@@ -11,14 +11,15 @@
 //                 applied to q and k (model/block.rs:128-146)
 // so the activation between a GEMM and its elementwise op never crosses HBM.
 //
-// Fast path (f16, N % kBN == 0, K % kBK == 0): matrix-core GEMM. A workgroup
-// of kWaves waves computes a 256 (rows) x kBN (columns) tile of out, K in
-// steps of kBK staged through LDS (double-buffered; the next step's tiles go straight
-// from global memory into LDS with buffer_load_dwordx4 ... lds while the
-// current one computes, with no registers in between). Both operands are K-contiguous
-// rows (x rows, w rows), which is exactly the operand layout of
-// v_mfma_f32_32x32x16_f16, so both come from LDS with 16-byte reads. Each
-// wave owns 128 rows x 64 columns and computes the transposed tile
+// Fast path (f16, N % 256 == 0, K % kBK == 0): matrix-core GEMM. A workgroup
+// computes one tile of out in a shape chosen by the tile count (256 x 256 down
+// to 64 x 64, F16Tile), K in steps of kBK staged through a ring in LDS (the
+// coming steps' tiles go straight from global memory into LDS with
+// buffer_load_dwordx4 ... lds while the current one computes, with no
+// registers in between). Both operands are K-contiguous rows (x rows, w rows),
+// which is exactly the operand layout of v_mfma_f32_32x32x16_f16, so both come
+// from LDS with 16-byte reads. Each wave owns 32, 96 or 128 rows x 64 columns
+// and computes the transposed tile
 // out^T = w x^T: its accumulators then hold, per lane, 4 consecutive output
 // columns of one output row. The epilogue adds the bias (and applies GELU)
 // there, stages the f16 results through LDS, and then streams whole rows:
@@ -77,23 +78,21 @@ struct LnArgs {
 // ---------------------------------------------------------------------------
 // matrix-core path
 
-#ifndef HS_GEMM_WAVES
-#define HS_GEMM_WAVES 8  // waves per workgroup: 2 row groups x (waves / 2) column groups
-#endif
-#ifndef HS_GEMM_BK
-#define HS_GEMM_BK 64  // K per LDS stage
-#endif
 #ifndef HS_GEMM_XCD
 #define HS_GEMM_XCD 1  // XCD-aware tile order
 #endif
-constexpr int kWaves = HS_GEMM_WAVES;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kBM = 256;               // output rows per workgroup (2 x 128)
-constexpr int kBN = 64 * (kWaves / 2);  // output columns per workgroup
-constexpr int kBK = HS_GEMM_BK;
+constexpr int kBK = 64;                  // K per LDS stage
 constexpr int kRowChunks = kBK / 8;      // 16-byte chunks per LDS row
 constexpr int kRowsPerInstr = 64 / kRowChunks;
 constexpr int kRowsPer256B = 128 / kBK;  // LDS rows per 64-bank period
+static_assert((kBK / 16) % 2 == 0, "operand register sets alternate within a stage");
+// Epilogue staging: each wave's block of 64 columns as f16 rows of kEpiPitch
+// halves (144 B: 16-byte aligned rows, spread over the banks).
+constexpr int kEpiPitch = 64 + 8;
+
+// A tile shape: WM x WN waves of 32 RB rows x 64 columns each, a ring of ST
+// stages in LDS, the refill of a freed stage issued in SP parts.
+//
 // Stages are filled by buffer_load_dwordx4 ... lds (LDS-DMA): one wave
 // instruction puts its 64 lanes' 16-byte chunks into 1 KiB of LDS in lane
 // order, i.e. kRowsPerInstr unpadded rows. Lane L of instruction j supplies
@@ -106,29 +105,38 @@ constexpr int kRowsPer256B = 128 / kBK;  // LDS rows per 64-bank period
 // instruction per load, and unlike the global (FLAT-encoded) form it lets
 // the compiler wait for the operand reads of one k-slice with lgkmcnt(n)
 // while the next slice's reads are in flight.
-constexpr int kXInstr = kBM * kBK / 8 / 64;  // wave instructions per x stage
-constexpr int kWInstr = kBN * kBK / 8 / 64;  // per w stage
-constexpr int kLoads = kXInstr / kWaves + kWInstr / kWaves;  // per wave and stage
-static_assert(kXInstr % kWaves == 0 && kWInstr % kWaves == 0, "stage split");
-static_assert((kBK / 16) % 2 == 0, "operand register sets alternate within a stage");
-
-struct GemmSmem {
-    f16 x[2][kBM * kBK];
-    f16 w[2][kBN * kBK];
+template <int WM, int WN, int RB_, int ST_, int SP_>
+struct F16Tile {
+    static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
+    static constexpr int kWN = WN, kRB = RB_, kST = ST_, kSP = SP_;
+    static constexpr int kBM = 32 * RB_ * WM;  // output rows per workgroup
+    static constexpr int kBN = 64 * WN;        // output columns per workgroup
+    static constexpr int kXL = kBM * kBK / 8 / 64 / kWaves;  // stage loads per wave, x
+    static constexpr int kWL = kBN * kBK / 8 / 64 / kWaves;  // w
+    static_assert(kXL * 64 * kWaves == kBM * kBK / 8 && kWL * 64 * kWaves == kBN * kBK / 8, "stage split");
+    struct Smem {
+        f16 x[ST_][kBM * kBK];
+        f16 w[ST_][kBN * kBK];
+    };
+    // With the LayerNorm prologue, x stages land in `raw` one stage ahead of
+    // their use and are normalised from there into x[]: raw follows Smem.
+    static constexpr size_t kRawBytes = size_t{2} * kBM * kBK;
+    static constexpr int kEpiWave = 32 * RB_ * kEpiPitch;  // halves per wave
+    static constexpr size_t smem_bytes(bool ln) {
+        const size_t loop = sizeof(Smem) + (ln ? kRawBytes : 0);
+        const size_t epi = size_t{2} * kWaves * kEpiWave;
+        return loop > epi ? loop : epi;
+    }
+    // waves per SIMD that the LDS lets a CU hold
+    static constexpr int kGroups = 160 * 1024 / static_cast<int>(sizeof(Smem));
+    static constexpr int kWavesPerEu = kGroups * kWaves >= 8 ? kGroups * kWaves / 4 : 1;
 };
-// With the LayerNorm prologue, x stages land in `raw` one stage ahead of
-// their use and are normalised from there into x[]: raw follows GemmSmem.
-constexpr size_t kRawBytes = size_t{2} * kBM * kBK;
-// Epilogue staging: each wave's 128 x 64 output block as f16 rows of
-// kEpiPitch halves (144 B: 16-byte aligned rows, spread over the banks).
-constexpr int kEpiPitch = 64 + 8;
-constexpr int kEpiWave = 128 * kEpiPitch;  // halves per wave
-constexpr size_t smem_bytes(bool ln) {
-    const size_t loop = sizeof(GemmSmem) + (ln ? kRawBytes : 0);
-    const size_t epi = size_t{2} * kWaves * kEpiWave;
-    return loop > epi ? loop : epi;
-}
-static_assert(smem_bytes(true) <= 160 * 1024, "gfx950 has 160 KiB of LDS per workgroup");
+using F16Big = F16Tile<2, 4, 4, 2, 1>;    // 256 x 256, 8 waves, one workgroup per CU
+using F16Mid = F16Tile<2, 4, 3, 2, 1>;    // 192 x 256, 8 waves, one per CU
+using F16Pair = F16Tile<4, 2, 1, 2, 1>;   // 128 x 128, 8 waves, two per CU
+using F16Solo = F16Tile<4, 2, 1, 4, 4>;   // 128 x 128, 8 waves, one per CU, four stages
+using F16Small = F16Tile<2, 1, 1, 4, 4>;  // 64 x 64, 2 waves, two per CU, four stages
+static_assert(F16Big::smem_bytes(true) <= 160 * 1024, "gfx950 has 160 KiB of LDS per workgroup");
 
 __device__ __forceinline__ h8 as_h8(u32x4 v) { return __builtin_bit_cast(h8, v); }
 
@@ -138,51 +146,34 @@ __device__ __forceinline__ int swz(int row) { return (row / kRowsPer256B) % kRow
 
 // Per-lane byte offsets of this wave's stage loads within the tile's x and
 // w row blocks; x rows past M read row M - 1 (their outputs are masked).
+template <typename P>
 struct StageOffsets {
-    uint32_t x[kXInstr / kWaves];
-    uint32_t w[kWInstr / kWaves];
+    uint32_t x[P::kXL];
+    uint32_t w[P::kWL];
 };
 
-__device__ __forceinline__ StageOffsets stage_offsets(int64_t m0, int M, int K, int wave,
-                                                     int lane) {
-    StageOffsets o;
+template <typename P>
+__device__ __forceinline__ StageOffsets<P> stage_offsets(int64_t m0, int M, int K, int wave, int lane) {
+    StageOffsets<P> o;
     const int prow = lane / kRowChunks, pc = lane % kRowChunks;
 #pragma unroll
-    for (int i = 0; i < kXInstr / kWaves; i++) {
-        const int row = kRowsPerInstr * (wave + kWaves * i) + prow;
+    for (int i = 0; i < P::kXL; i++) {
+        const int row = kRowsPerInstr * (wave + P::kWaves * i) + prow;
         const int lrow = static_cast<int>(min(m0 + row, static_cast<int64_t>(M) - 1) - m0);
         o.x[i] = static_cast<uint32_t>(lrow * K * 2 + 16 * (pc ^ swz(row)));
     }
 #pragma unroll
-    for (int i = 0; i < kWInstr / kWaves; i++) {
-        const int row = kRowsPerInstr * (wave + kWaves * i) + prow;
+    for (int i = 0; i < P::kWL; i++) {
+        const int row = kRowsPerInstr * (wave + P::kWaves * i) + prow;
         o.w[i] = static_cast<uint32_t>(row * K * 2 + 16 * (pc ^ swz(row)));
     }
     return o;
 }
 
-// Issue this wave's LDS-DMA loads of one stage's x (or w) rows from the
-// buffer resource covering the tile's rows into dst; koff = the stage's
-// first column, in bytes.
-__device__ __forceinline__ void issue_x(f16* dst, __amdgpu_buffer_rsrc_t xr, int koff,
-                                        const StageOffsets& o, int wave) {
-#pragma unroll
-    for (int i = 0; i < kXInstr / kWaves; i++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            xr, (lds_void*)(dst + (wave + kWaves * i) * 512), 16, o.x[i], koff, 0, 0);
-}
-__device__ __forceinline__ void issue_w(f16* dst, __amdgpu_buffer_rsrc_t wr, int koff,
-                                        const StageOffsets& o, int wave) {
-#pragma unroll
-    for (int i = 0; i < kWInstr / kWaves; i++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            wr, (lds_void*)(dst + (wave + kWaves * i) * 512), 16, o.w[i], koff, 0, 0);
-}
-__device__ __forceinline__ void issue_stage(GemmSmem& sm, int buf, __amdgpu_buffer_rsrc_t xr,
-                                            __amdgpu_buffer_rsrc_t wr, int koff,
-                                            const StageOffsets& o, int wave) {
-    issue_x(sm.x[buf], xr, koff, o, wave);
-    issue_w(sm.w[buf], wr, koff, o, wave);
+// One LDS-DMA wave instruction: each lane's 16 bytes at voff + koff of the
+// buffer into the 1 KiB at dst, in lane order.
+__device__ __forceinline__ void lds_load(f16* dst, __amdgpu_buffer_rsrc_t src, uint32_t voff, int koff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)dst, 16, voff, koff, 0, 0);
 }
 
 // The LayerNorm prologue. Lane L of a wave normalises exactly the 16-byte
@@ -193,8 +184,9 @@ __device__ __forceinline__ void issue_stage(GemmSmem& sm, int buf, __amdgpu_buff
 // loads to have landed (vmcnt, no barrier), its rows' statistics stay in
 // registers for the whole product, and each stage's parameters are the 8
 // columns 8 lc of that stage.
-constexpr int kLnRows = kXInstr / kWaves;  // x pieces per lane and stage
-static_assert((kRowsPerInstr * kWaves / kRowsPer256B) % kRowChunks == 0,
+constexpr int kLnWaves = F16Big::kWaves;  // the prologue runs in F16Big tiles
+constexpr int kLnRows = F16Big::kXL;     // x pieces per lane and stage
+static_assert((kRowsPerInstr * kLnWaves / kRowsPer256B) % kRowChunks == 0,
               "a lane's x pieces share one logical chunk");
 constexpr int kLnParamLoads = 4;            // 16-byte loads of ln_w / ln_b per stage
 #ifndef HS_GEMM_LN_SLICES
@@ -225,7 +217,7 @@ __device__ __forceinline__ LnLane ln_lane(const LnArgs& la, int64_t m0, int M, i
     LnLane ll;
 #pragma unroll
     for (int i = 0; i < kLnRows; i++) {
-        const int row = kRowsPerInstr * (wave + kWaves * i) + lane / kRowChunks;
+        const int row = kRowsPerInstr * (wave + kLnWaves * i) + lane / kRowChunks;
         // rows past M were loaded from row M - 1 and are normalised with its
         // statistics (their products are masked)
         const int64_t r = min(m0 + row, static_cast<int64_t>(M) - 1);
@@ -245,7 +237,7 @@ __device__ __forceinline__ void ln_params(const LnArgs& la, const LnLane& ll, in
 
 // Halves offset of the lane's piece i within an x stage.
 __device__ __forceinline__ int ln_off(int i, int wave, int lane) {
-    return (wave + kWaves * i) * 512 + 8 * lane;
+    return (wave + kLnWaves * i) * 512 + 8 * lane;
 }
 
 // One normalised piece: the 8 f16 values of v, with the row's (mean, rstd)
@@ -283,14 +275,14 @@ __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
     return h22u(h);
 }
 
-// Phase 2 of the q|k|v epilogue: the wave's staged block is 128 token rows
+// Phase 2 of the q|k|v epilogue: the wave's staged block is `rows` token rows
 // of one head of q, k or v (its 64 columns). 8 lanes per row hold the head
 // vector in the lane layout of qk_norm_rope_vec (the QK-norm / RoPE fused
 // op's), so each head vector is normalised, rotated and rounded by the same
 // code as there; each row's 128 bytes go to (frame, head, token) of the
 // head-major output.
 __device__ __forceinline__ void qkv_heads_out(const f16* stage, const QkvArgs& qa, int64_t row0,
-                                              int M, int64_t col, int lane) {
+                                              int M, int64_t col, int lane, int rows) {
     const int hd = qa.heads * 64;
     const int which = static_cast<int>(col / hd);            // 0 q, 1 k, 2 v: wave-uniform
     const int head = static_cast<int>(col - int64_t{which} * hd) / 64;
@@ -317,7 +309,7 @@ __device__ __forceinline__ void qkv_heads_out(const f16* stage, const QkvArgs& q
     int64_t m = row0 + (lane >> 3);
     uint32_t s = static_cast<uint32_t>(m) / static_cast<uint32_t>(qa.seq);
     int t = static_cast<int>(static_cast<uint32_t>(m) - s * static_cast<uint32_t>(qa.seq));
-    for (int rr = 0; rr < 128; rr += 8) {
+    for (int rr = 0; rr < rows; rr += 8) {
         if (m >= M) break;  // rows grow with rr: the rest are past M too
         float f[8];
         unpack(ld16(stage + (rr + (lane >> 3)) * kEpiPitch + ch), f, f16{});
@@ -345,14 +337,16 @@ __device__ __forceinline__ void qkv_heads_out(const f16* stage, const QkvArgs& q
 
 // Grid: tiles_m * tiles_n workgroups, column tiles fastest, so workgroups
 // running together share their x rows.
-template <int EPI, bool LN>
-__global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
+template <int EPI, typename P, bool LN>
+__global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f16_kernel(
     const f16* __restrict__ x, const f16* __restrict__ w, const float* __restrict__ bias,
     const float* __restrict__ gamma, const f16* res, f16* out, int M, int N, int K,
     int tiles_n, int ntiles, QkvArgs qa, LnArgs la) {
-    __shared__ __align__(16) unsigned char smem_raw[smem_bytes(LN)];
-    GemmSmem& sm = *reinterpret_cast<GemmSmem*>(smem_raw);
-    f16* const raw = reinterpret_cast<f16*>(smem_raw + sizeof(GemmSmem));  // LN only
+    static_assert(!LN || std::is_same_v<P, F16Big>, "the LayerNorm prologue runs in F16Big tiles");
+    constexpr int kRB = P::kRB, kST = P::kST, kBM = P::kBM, kBN = P::kBN;
+    __shared__ __align__(16) unsigned char smem_raw[P::smem_bytes(LN)];
+    typename P::Smem& sm = *reinterpret_cast<typename P::Smem*>(smem_raw);
+    f16* const raw = reinterpret_cast<f16*>(smem_raw + sizeof(typename P::Smem));  // LN only
     const int tid = threadIdx.x;
     const int lane = lane_id();
     const int wave = tid >> 6;
@@ -370,26 +364,51 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
 #endif
     const int64_t m0 = static_cast<int64_t>(tile / tiles_n) * kBM;
     const int64_t n0 = static_cast<int64_t>(tile % tiles_n) * kBN;
-    const int wm = (wave / (kWaves / 2)) * 128;  // wave's rows within the tile
-    const int wn = (wave % (kWaves / 2)) * 64;   // wave's columns within the tile
+    const int wm = (wave / P::kWN) * (32 * kRB);  // wave's rows within the tile
+    const int wn = (wave % P::kWN) * 64;   // wave's columns within the tile
 
     // acc[a][b]: out^T block of columns wn + 32 a .. + 32 (MFMA rows) and
     // rows wm + 32 b .. + 32 (MFMA columns); register r of lane (l32, hh)
     // is column 8 (r / 4) + 4 hh + r % 4, row l32 of the block.
-    f32x16 acc[2][4];
+    f32x16 acc[2][kRB];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = f32x16{};
+        for (int b = 0; b < kRB; b++) acc[a][b] = f32x16{};
 
     const int nsteps = K / kBK;
     const int wv = wave_in_block();
-    const StageOffsets so = stage_offsets(m0, M, K, wv, lane);
+    const StageOffsets<P> so = stage_offsets<P>(m0, M, K, wv, lane);
     const int xrows = static_cast<int>(min(static_cast<int64_t>(kBM), M - m0));
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<f16*>(x + m0 * K), 0, xrows * K * 2, kRawBufferFlags);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<f16*>(w + n0 * K), 0, kBN * K * 2, kRawBufferFlags);
+    // Issue this wave's LDS-DMA loads of one stage's x (or w) rows into dst;
+    // koff = the stage's first column, in bytes.
+    auto issue_x = [&](f16* dst, int koff) {
+#pragma unroll
+        for (int i = 0; i < P::kXL; i++)
+            lds_load(dst + (wv + P::kWaves * i) * 512, xr, so.x[i], koff);
+    };
+    auto issue_w = [&](f16* dst, int koff) {
+#pragma unroll
+        for (int i = 0; i < P::kWL; i++)
+            lds_load(dst + (wv + P::kWaves * i) * 512, wr, so.w[i], koff);
+    };
+    // Loads [from, to) of a stage's kL per wave, x first.
+    constexpr int kL = P::kXL + P::kWL, kPart = kL / P::kSP;
+    static_assert(kPart * P::kSP == kL && P::kSP <= kBK / 16, "a stage's loads in equal parts, one per slice");
+    auto issue_part = [&](int buf, int koff, int from, int to) {
+#pragma unroll
+        for (int i = 0; i < kL; i++) {
+            if (i < from || i >= to) continue;
+            if (i < P::kXL)
+                lds_load(sm.x[buf] + (wv + P::kWaves * i) * 512, xr, so.x[i < P::kXL ? i : 0], koff);
+            else
+                lds_load(sm.w[buf] + (wv + P::kWaves * (i - P::kXL)) * 512, wr, so.w[i < P::kXL ? 0 : i - P::kXL], koff);
+        }
+    };
     // Both buffers start filled (stages 0 and 1). The waits below are
     // explicit: vmcnt counts this wave's loads, which complete in order, and
     // the barrier then covers every wave's.
@@ -399,20 +418,20 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
     // by its own lanes during step s - 1, beside that step's multiplies; w
     // keeps the schedule above. Per wave, in issue order: params(s + 2),
     // x(s + 2) in the middle of step s, w(s + 2) after its closing barrier.
-    constexpr int kXL = kXInstr / kWaves, kWL = kWInstr / kWaves;
+    constexpr int kXL = P::kXL, kWL = P::kWL;
     LnLane ll;
     float4 gb[kLnParamLoads];
     if constexpr (LN) {
         ll = ln_lane(la, m0, M, wv, lane);
         ln_params(la, ll, 0, gb);
-        issue_x(raw, xr, 0, so, wv);
-        issue_w(sm.w[0], wr, 0, so, wv);
+        issue_x(raw, 0);
+        issue_w(sm.w[0], 0);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWL) : "memory");  // params(0), x(0)
         ln_stage(raw, sm.x[0], ll, gb, wv, lane);
         if (nsteps > 1) {
             ln_params(la, ll, kBK, gb);
-            issue_x(raw, xr, 2 * kBK, so, wv);
-            issue_w(sm.w[1], wr, 2 * kBK, so, wv);
+            issue_x(raw, 2 * kBK);
+            issue_w(sm.w[1], 2 * kBK);
             // w(0) landed; x[0]'s normalised pieces written
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLnParamLoads + kXL + kWL)
                          : "memory");
@@ -420,21 +439,27 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
     } else {
-        issue_stage(sm, 0, xr, wr, 0, so, wv);
-        if (nsteps > 1) {
-            issue_stage(sm, 1, xr, wr, 2 * kBK, so, wv);
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLoads) : "memory");
-        } else {
+#pragma unroll
+        for (int i = 0; i + 1 < kST; i++)
+            if (i < nsteps) issue_part(i, 2 * i * kBK, 0, kL);
+        if (kST - 1 < nsteps) issue_part(kST - 1, 2 * (kST - 1) * kBK, 0, kPart);
+        if (nsteps >= kST)
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kST - 2) * kL + kPart) : "memory");
+        else
             asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-        }
     }
     // Operand registers in two sets: the next 16-wide k slice is read from
     // LDS while the current one multiplies, across stage boundaries too.
-    h8 A[2][2], B[2][4];
+    constexpr int kSl = kBK / 16;
+    h8 A[2][2], B[2][kRB];
+    auto read_slice = [&](int set, int buf, int ks) {
+        const int kc = 2 * ks + hh;
 #pragma unroll
-    for (int a = 0; a < 2; a++) A[0][a] = ld_op(sm.w[0], wn + 32 * a + l32, hh);
+        for (int a = 0; a < 2; a++) A[set][a] = ld_op(sm.w[buf], wn + 32 * a + l32, kc);
 #pragma unroll
-    for (int b = 0; b < 4; b++) B[0][b] = ld_op(sm.x[0], wm + 32 * b + l32, hh);
+        for (int b = 0; b < kRB; b++) B[set][b] = ld_op(sm.x[buf], wm + 32 * b + l32, kc);
+    };
+    read_slice(0, 0, 0);
     if constexpr (LN) {
         // One step of the product with the prologue: the multiplies of stage
         // s and, beside them, NORM: stage s + 1's LayerNorm from raw into
@@ -458,7 +483,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
                         // the lane's raw pieces (read at slice 0) are in
                         // registers: refill raw with x(s + 2)
                         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                        issue_x(raw, xr, 2 * (s + 2) * kBK, so, wv);
+                        issue_x(raw, 2 * (s + 2) * kBK);
                     }
                 }
                 if (ks + 1 < kBK / 16) {
@@ -466,7 +491,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
 #pragma unroll
                     for (int a = 0; a < 2; a++) A[p ^ 1][a] = ld_op(sm.w[cur], wn + 32 * a + l32, kc);
 #pragma unroll
-                    for (int b = 0; b < 4; b++) B[p ^ 1][b] = ld_op(sm.x[cur], wm + 32 * b + l32, kc);
+                    for (int b = 0; b < kRB; b++) B[p ^ 1][b] = ld_op(sm.x[cur], wm + 32 * b + l32, kc);
                 }
                 if constexpr (NORM) {
                     if (ks == 0) {
@@ -495,18 +520,18 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
                     else
                         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
                     // w[cur] is free: refill it with stage s + 2
-                    if constexpr (ISSUE) issue_w(sm.w[cur], wr, 2 * (s + 2) * kBK, so, wv);
+                    if constexpr (ISSUE) issue_w(sm.w[cur], 2 * (s + 2) * kBK);
                     if constexpr (NORM) {
 #pragma unroll
                         for (int a = 0; a < 2; a++) A[p ^ 1][a] = ld_op(sm.w[cur ^ 1], wn + 32 * a + l32, hh);
 #pragma unroll
-                        for (int b = 0; b < 4; b++) B[p ^ 1][b] = ld_op(sm.x[cur ^ 1], wm + 32 * b + l32, hh);
+                        for (int b = 0; b < kRB; b++) B[p ^ 1][b] = ld_op(sm.x[cur ^ 1], wm + 32 * b + l32, hh);
                     }
                 }
 #pragma unroll
                 for (int a = 0; a < 2; a++)
 #pragma unroll
-                    for (int b = 0; b < 4; b++)
+                    for (int b = 0; b < kRB; b++)
                         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[p][a], B[p][b], acc[a][b], 0, 0, 0);
                 if (NORM && !kLnHints) {
                     // the scheduler's own order
@@ -533,40 +558,64 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
         if (s + 1 < nsteps) step(s++, std::true_type{}, std::false_type{});
         step(s, std::false_type{}, std::false_type{});
     } else {
-    for (int s = 0; s < nsteps; s++) {
-        const int cur = s & 1;
+        // One stage's multiplies. The refill of a freed buffer goes out behind
+        // the next slice's operand reads and between multiplies (ahead of
+        // the reads, its burst kept them waiting: fc1 at S=32 442 us against
+        // 414): part 0 behind the barrier that frees the buffer, parts 1 .. in
+        // the next step's slices. MORE: parts 1 .. of stage s + kST - 1 are
+        // issued; NEXT: part 0 of stage s + kST is.
+        int cur = 0;
+        auto step = [&](int s, auto more_c, auto next_c) {
+            constexpr bool MORE = decltype(more_c)::value, NEXT = decltype(next_c)::value;
+            const int nxt = cur + 1 == kST ? 0 : cur + 1;
+            const int prv = cur == 0 ? kST - 1 : cur - 1;
 #pragma unroll
-        for (int ks = 0; ks < kBK / 16; ks++) {
-            const int p = ks & 1;  // kBK / 16 is even: set 0 holds slice 0 of every stage
-            if (ks + 1 < kBK / 16) {
-                const int kc = 2 * (ks + 1) + hh;
+            for (int ks = 0; ks < kSl; ks++) {
+                const int p = ks & 1;
+                int loads = 0;
+                if (ks + 1 < kSl) {
+                    read_slice(p ^ 1, cur, ks + 1);
+                    if (MORE && ks + 1 < P::kSP) {
+                        issue_part(prv, 2 * (s + kST - 1) * kBK, (ks + 1) * kPart, (ks + 2) * kPart);
+                        loads = kPart;
+                    }
+                } else {
+                    // every wave's reads of stage s are done and stage s + 1
+                    // has landed (stages s + 2 .. s + kST - 1 may be in flight)
+                    if constexpr (NEXT || MORE)
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kST - 2) * kL) : "memory");
+                    else
+                        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    read_slice(p ^ 1, nxt, 0);  // (past the last stage: stale, not used)
+                    if constexpr (NEXT) {
+                        issue_part(cur, 2 * (s + kST) * kBK, 0, kPart);
+                        loads = kPart;
+                    }
+                }
 #pragma unroll
-                for (int a = 0; a < 2; a++) A[p ^ 1][a] = ld_op(sm.w[cur], wn + 32 * a + l32, kc);
+                for (int a = 0; a < 2; a++)
 #pragma unroll
-                for (int b = 0; b < 4; b++) B[p ^ 1][b] = ld_op(sm.x[cur], wm + 32 * b + l32, kc);
-            } else {
-                // every wave's reads of stage s are done and stage s + 1
-                // (the only load in flight) has landed
-                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                // buffer cur is free: refill it with stage s + 2
-                if (s + 2 < nsteps) issue_stage(sm, cur, xr, wr, 2 * (s + 2) * kBK, so, wv);
-                if (s + 1 < nsteps) {
+                    for (int b = 0; b < kRB; b++)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[p][a], B[p][b], acc[a][b], 0, 0, 0);
+                // the reads ahead of the multiplies, the loads between them
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 + kRB, 0);  // LDS reads
+                if (loads) {
+                    constexpr int per = (kPart + 2 * kRB - 1) / (2 * kRB);
 #pragma unroll
-                    for (int a = 0; a < 2; a++) A[p ^ 1][a] = ld_op(sm.w[cur ^ 1], wn + 32 * a + l32, hh);
-#pragma unroll
-                    for (int b = 0; b < 4; b++) B[p ^ 1][b] = ld_op(sm.x[cur ^ 1], wm + 32 * b + l32, hh);
+                    for (int q = 0; q < 2 * kRB; q++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // an MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x010, per, 0);  // loads
+                    }
+                } else {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2 * kRB, 0);  // MFMAs
                 }
             }
-#pragma unroll
-            for (int a = 0; a < 2; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[p][a], B[p][b], acc[a][b], 0, 0, 0);
-            // keep the reads above ahead of these multiplies
-            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);  // LDS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);  // MFMAs
-        }
-    }
+            cur = nxt;
+        };
+        int s = 0;
+        for (; s + kST < nsteps; s++) step(s, std::true_type{}, std::true_type{});
+        if (s + kST == nsteps) step(s++, std::true_type{}, std::false_type{});
+        for (; s < nsteps; s++) step(s, std::false_type{}, std::false_type{});
     }
 
     // Epilogue, in two phases so that global memory sees whole rows.
@@ -575,7 +624,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
     //    f16(acc + bias) (for GELU: f16(gelu(acc + bias))), and writes it
     //    to the wave's staging block in LDS (free once every wave has left
     //    the main loop).
-    f16* stage = reinterpret_cast<f16*>(smem_raw) + wave * kEpiWave;
+    f16* stage = reinterpret_cast<f16*>(smem_raw) + wave * P::kEpiWave;
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
@@ -583,7 +632,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
             const int cl = 32 * a + 8 * r4 + 4 * hh;  // column within the wave's block
             const float4 bv = bias ? ld_f32x4(bias + n0 + wn + cl) : float4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
+            for (int b = 0; b < kRB; b++) {
                 float v[4];
                 v[0] = acc[a][b][4 * r4] + bv.x, v[1] = acc[a][b][4 * r4 + 1] + bv.y;
                 v[2] = acc[a][b][4 * r4 + 2] + bv.z, v[3] = acc[a][b][4 * r4 + 3] + bv.w;
@@ -601,7 +650,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if constexpr (EPI == EPI_QKV) {
-        qkv_heads_out(stage, qa, m0 + wm, M, n0 + wn, lane);
+        qkv_heads_out(stage, qa, m0 + wm, M, n0 + wn, lane, 32 * kRB);
         return;
     }
     // 2. 8 lanes per 128-byte row piece, 8 rows per instruction: 16-byte
@@ -611,7 +660,7 @@ __global__ __launch_bounds__(kThreads, 8 / kWaves) void gemm_f16_kernel(
     float4 g0 = {0.0f, 0.0f, 0.0f, 0.0f}, g1 = g0;
     if constexpr (EPI == EPI_LS) g0 = ld_f32x4(gamma + n), g1 = ld_f32x4(gamma + n + 4);
 #pragma unroll 4
-    for (int rr = 0; rr < 128; rr += 8) {
+    for (int rr = 0; rr < 32 * kRB; rr += 8) {
         const int rl = rr + (lane >> 3);
         const int64_t m = m0 + wm + rl;
         if (m >= M) break;  // rows grow with rr: the rest are past M too
@@ -1075,7 +1124,7 @@ bool fast_shape(hs_dtype dt, int N, int K, const void* x, const void* w, const f
     // K == 0 takes the generic kernel (out = bias): the fast path's first
     // stage would read K-tiles that do not exist
     // K <= 2^20 keeps a tile's byte offsets (256 rows x K x 2) in 32 bits
-    return dt == HS_F16 && N % kBN == 0 && K > 0 && K % kBK == 0 && K <= (1 << 20) && aligned16(x) && aligned16(w) &&
+    return dt == HS_F16 && N % F16Big::kBN == 0 && K > 0 && K % kBK == 0 && K <= (1 << 20) && aligned16(x) && aligned16(w) &&
            (!bias || aligned16(bias)) && (!gamma || aligned16(gamma)) && aligned16(out) &&
            (!res || aligned16(res));
 }
@@ -1113,6 +1162,18 @@ void launch_f32(hipStream_t st, const void* x, const void* w, const float* bias,
         static_cast<int>(ntiles), la, qa);
 }
 
+template <int EPI, typename P, bool LN>
+void launch_f16(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
+                const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
+    const int tiles_n = N / P::kBN;
+    const int64_t ntiles = ceil_div(M, P::kBM) * tiles_n;
+    const int64_t blocks = HS_GEMM_XCD ? ceil_div(ntiles, 8) * 8 : ntiles;
+    gemm_f16_kernel<EPI, P, LN><<<dim3(static_cast<uint32_t>(blocks)), dim3(P::kThreads), 0, st>>>(
+        static_cast<const f16*>(x), static_cast<const f16*>(w), bias, gamma,
+        static_cast<const f16*>(res), static_cast<f16*>(out), M, N, K, tiles_n,
+        static_cast<int>(ntiles), qa, la);
+}
+
 template <int EPI, bool LN = false>
 hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, const float* bias,
                  const float* gamma, const void* res, void* out, int M, int N, int K,
@@ -1126,13 +1187,36 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
         return check_launch(op);
     }
     if (takes_fast_path<LN>(dt, N, K, x, w, bias, gamma, out, res, la)) {
-        const int tiles_n = N / kBN;
-        const int64_t ntiles = ceil_div(M, kBM) * tiles_n;
-        const int64_t blocks = HS_GEMM_XCD ? ceil_div(ntiles, 8) * 8 : ntiles;
-        gemm_f16_kernel<EPI, LN><<<dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, st>>>(
-            static_cast<const f16*>(x), static_cast<const f16*>(w), bias, gamma,
-            static_cast<const f16*>(res), static_cast<f16*>(out), M, N, K, tiles_n,
-            static_cast<int>(ntiles), qa, la);
+        // The tile shape. Every shape sums k in the same order, so the choice
+        // changes no bit of the result (the LayerNorm prologue exists for
+        // F16Big). Times in us for the q|k|v / proj / fc1 / fc2 shapes, Small
+        // / Solo / Pair / Mid / Big:
+        //   64 x 64 while two per CU hold them all (S=1, 1386 rows: proj
+        //     8.6 / 10 / 11 / 20 / 24, fc2 23 / 28 / 43 / 66 / 78);
+        //   then 128 x 128 with four stages while one per CU does (S=2: proj
+        //     16 / 11.4 / 12.7 / 21 / 26, fc2 49 / 31 / 44 / 66 / 78), or
+        //     with two stages while two per CU do (S=4 proj 27 / 24 / 20 / 24
+        //     / 29, S=1 q|k|v 25 / 22 / 16 / 21 / 24);
+        //   beyond, the fewer rounds of the chip in rows, with a tenth on Mid
+        //     for its larger share of LDS reads (S=2 q|k|v - / 36 / 31 / 23 /
+        //     26, S=8 q|k|v Mid 76, Big 87; fc1 at 11088 rows 119, 111).
+        if constexpr (LN) {
+            launch_f16<EPI, F16Big, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        } else {
+            const int64_t cus = num_cus();
+            auto tiles = [&](int bm, int bn) { return ceil_div(M, bm) * (N / bn); };
+            const int64_t t128 = tiles(128, 128);
+            if (tiles(64, 64) <= 2 * cus)
+                launch_f16<EPI, F16Small, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+            else if (t128 <= cus)
+                launch_f16<EPI, F16Solo, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+            else if (t128 <= 2 * cus)
+                launch_f16<EPI, F16Pair, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+            else if (ceil_div(tiles(192, 256), cus) * 192 * 11 < ceil_div(tiles(256, 256), cus) * 256 * 10)
+                launch_f16<EPI, F16Mid, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+            else
+                launch_f16<EPI, F16Big, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        }
         return check_launch(op);
     }
     if constexpr (EPI == EPI_QKV) {
@@ -1246,7 +1330,7 @@ hs_status qkv_setup(const char* op, hs_dtype dt, const void* x, const void* w_qk
     // The fused epilogue needs one head per wave (64 columns) and whole
     // column tiles (256 in f16, 128 in f32); other shapes run linear then
     // qknorm_rope.
-    const int64_t tile_n = dt == HS_F16 ? kBN : F32Shape::kBN;
+    const int64_t tile_n = dt == HS_F16 ? F16Big::kBN : F32Shape::kBN;
     if (d != 64 || N % tile_n != 0)
         return fail(HS_EUNSUPPORTED, "%s: needs head dim 64 and 3*H*64 %% %lld == 0", op,
                     static_cast<long long>(tile_n));

@@ -399,3 +399,28 @@ def test_linear_qkv_heads_fallback_f32(ctx):
             torch.cuda.current_stream().cuda_stream, _lib.HS_F32, x.data_ptr(), w.data_ptr(),
             None, None, None, None, None, None, None, got[0].data_ptr(), got[1].data_ptr(),
             got[2].data_ptr(), 2, 41, 3, 64, 64, 0, 1e-5), "linear_qkv_heads")
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 1024])
+@pytest.mark.parametrize("n", [256, 1024])
+def test_linear_f16_tile_shapes_agree(ctx, n, k):
+    """The tile shape follows the tile count (64 x 64, 128 x 128 with four
+    and two stages, 192 x 256, 256 x 256 at 256 CUs and n = 1024) and sums k
+    in one order: rows of a call of any size equal the same rows of a larger
+    one, at the edges and remainders of every shape and with fewer k stages
+    than a shape has buffers. The largest is checked against the float64
+    product: f32 sums of k f16 products and one f16 rounding (2^-11)."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    m_max = 12290 * 1024 // n if n < 1024 else 12290
+    x = torch.randn((m_max, k), generator=g, device="cuda").half()
+    w = (torch.randn((n, k), generator=g, device="cuda") / k ** 0.5).half()
+    b = torch.randn(n, generator=g, device="cuda") * 0.02
+    big = ctx.linear(x, w, b)
+    want = x.double() @ w.double().t().contiguous() + b.double()
+    err = (big.double() - want).abs()
+    assert bool((err <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * (1.0 + want.abs())).all())
+    scale = 1024 // n
+    for m in (1, 63, 65, 2048 * scale, 2049 * scale, 4097 * scale, 8191 * scale, 8193 * scale,
+              8192 * scale + 193):
+        assert torch.equal(ctx.linear(x[:m], w, b), big[:m]), m
