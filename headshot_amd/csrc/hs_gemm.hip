@@ -32,7 +32,8 @@
 // f32 (N % 128 == 0, K % 32 == 0; every epilogue but the q|k|v split, with
 // or without the LayerNorm prologue): the same arrangement on the f32
 // matrix cores in 128 x 128 tiles, the epilogue stored straight from the
-// accumulators.
+// accumulators. Up to 128 rows a kernel that splits K over the waves and
+// streams the weights straight into registers (gemm_skinny_kernel).
 //
 // Generic path (the shapes neither covers): a tiled scalar kernel, f32
 // accumulation in K order.
@@ -1057,6 +1058,162 @@ __global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f32_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// few rows (f32, N % 128 == 0, K % 32 == 0, M <= kSkinnyRows):
+// what such a call cannot do without is the weights' way from memory, so the
+// work is split until every CU streams some of them. A workgroup of 16 waves
+// takes 16 CB output columns x 16 RB rows; its waves share K, wave v taking
+// the 128-byte pieces v, v + 16, .. of every row straight from memory into
+// operand registers (16 rows x 128 bytes per pair of loads, no LDS stage, no
+// barrier), and the 16 partial tiles are summed in wave order through LDS.
+// v_mfma_f32_16x16x4_f32 computes out^T = w x^T: lane (r, g) holds row r's 4
+// floats at chunk g of the piece's half and MFMA j takes element j of both
+// operands; its accumulators are columns 4 g .. + 4 of output row r. The
+// order of the sum depends on K only.
+//
+// At 8 rows (us, beside the 64 x 128 tiles): 2048 x 2048 8.4 (72.7), 8192 x
+// 2048 14.2 (74.7), 2048 x 8192 26 (279), i.e. 2.0-4.7 TB/s of weights; at 100
+// rows 18 (74), 65 (75), 62 (280); above 128 rows wide outputs are faster in
+// tiles (200 rows, 8192 x 2048: 110 against 80).
+constexpr int kSkinnyRows = 128;
+constexpr int kSkWaves = 16, kSkThreads = 64 * kSkWaves;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 sk_mfma(u32x4 a, u32x4 b, f32x4 c) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(u2f(a[j]), u2f(b[j]), c, 0, 0, 0);
+    return c;
+}
+
+// 4 floats of an x row at column k, normalised as hs_layernorm stores them.
+__device__ __forceinline__ u32x4 sk_ln(u32x4 v, f32x2 st, const LnArgs& la, int k) {
+    const float4 g = ld_f32x4(la.ln_w + k), b = ld_f32x4(la.ln_b + k);
+    u32x4 o;
+    o[0] = f2u(ln_affine(u2f(v[0]), st[0], st[1], g.x, b.x));
+    o[1] = f2u(ln_affine(u2f(v[1]), st[0], st[1], g.y, b.y));
+    o[2] = f2u(ln_affine(u2f(v[2]), st[0], st[1], g.z, b.z));
+    o[3] = f2u(ln_affine(u2f(v[3]), st[0], st[1], g.w, b.w));
+    return o;
+}
+
+template <int EPI, int CB, int RB, bool LN>
+__global__ __launch_bounds__(kSkThreads) void gemm_skinny_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    const float* __restrict__ gamma, const float* res, float* out, int M, int N, int K, int row_groups,
+    int ngroups, QkvArgs qa, LnArgs la) {
+    constexpr int kPiece = 32;                   // floats per 128 bytes
+    constexpr int kTile = 256 * CB * RB;          // floats per partial tile
+    constexpr int kStage = EPI == EPI_QKV ? 16 * RB * kQkvPitch : 0;
+    static_assert(EPI != EPI_QKV || CB == 4, "a head is 64 columns");
+    __shared__ __align__(16) float sm[kSkWaves * kTile + kStage];
+    const int lane = lane_id(), wave = wave_in_block();
+    const int r = lane & 15, g = lane >> 4;
+    // an XCD takes a contiguous range, the row groups of one column group
+    // (which share its weights) first; the grid is padded to 8
+    const int per = static_cast<int>(gridDim.x / 8);
+    const int grp = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (grp >= ngroups) return;  // before any barrier
+    const int64_t n0 = static_cast<int64_t>(grp / row_groups) * (16 * CB);
+    const int64_t m0 = static_cast<int64_t>(grp % row_groups) * (16 * RB);
+
+    const float* wp[CB];
+    const float* xp[RB];
+    f32x2 st[RB];
+#pragma unroll
+    for (int c = 0; c < CB; c++) wp[c] = w + (n0 + 16 * c + r) * K + g * 4;
+#pragma unroll
+    for (int b = 0; b < RB; b++) {
+        // rows past M read row M - 1 (not stored)
+        const int64_t m = min(m0 + 16 * b + r, static_cast<int64_t>(M) - 1);
+        xp[b] = x + m * K + g * 4;
+        if constexpr (LN) st[b] = *reinterpret_cast<const f32x2*>(la.stats + 2 * m);
+    }
+    f32x4 acc[CB][RB];
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+        for (int b = 0; b < RB; b++) acc[c][b] = f32x4{};
+    u32x4 A[2][CB], B[2][RB];  // the piece's two halves
+    auto load = [&](int k) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int c = 0; c < CB; c++) A[h][c] = ld16(wp[c] + k + 16 * h);
+#pragma unroll
+            for (int b = 0; b < RB; b++) B[h][b] = ld16(xp[b] + k + 16 * h);
+        }
+    };
+    const int step = kSkWaves * kPiece;
+    int k = wave * kPiece;
+    if (k < K) load(k);
+    while (k < K) {
+        u32x4 a[2][CB], b[2][RB];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int c = 0; c < CB; c++) a[h][c] = A[h][c];
+#pragma unroll
+            for (int i = 0; i < RB; i++) b[h][i] = B[h][i];
+        }
+        const int kc = k;
+        k += step;
+        if (k < K) load(k);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if constexpr (LN) {
+#pragma unroll
+                for (int i = 0; i < RB; i++) b[h][i] = sk_ln(b[h][i], st[i], la, kc + 16 * h + 4 * g);
+            }
+#pragma unroll
+            for (int c = 0; c < CB; c++)
+#pragma unroll
+                for (int i = 0; i < RB; i++) acc[c][i] = sk_mfma(a[h][c], b[h][i], acc[c][i]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+        for (int b = 0; b < RB; b++)
+            *reinterpret_cast<f32x4*>(sm + wave * kTile + (c * RB + b) * 256 + r * 16 + 4 * g) = acc[c][b];
+    __syncthreads();
+
+    // quad q: columns 4 (q % 4) .. + 4 of row (q / 4) % 16 of block q / 64
+    for (int q = threadIdx.x; q < kTile / 4; q += kSkThreads) {
+        const int blk = q / 64, c = blk / RB, b = blk % RB;
+        const int row = 16 * b + (q / 4) % 16, col = 16 * c + 4 * (q % 4);
+        f32x4 v = *reinterpret_cast<const f32x4*>(sm + 4 * q);
+#pragma unroll
+        for (int i = 1; i < kSkWaves; i++) v += *reinterpret_cast<const f32x4*>(sm + i * kTile + 4 * q);
+        const int64_t m = m0 + row, n = n0 + col;
+        if (m >= M && EPI != EPI_QKV) continue;
+        const float4 bv = bias ? ld_f32x4(bias + n) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        float o[4] = {v[0] + bv.x, v[1] + bv.y, v[2] + bv.z, v[3] + bv.w};
+        if constexpr (EPI == EPI_QKV) {
+            // the head vectors' rows, staged behind the partial tiles
+            *reinterpret_cast<float4*>(sm + kSkWaves * kTile + row * kQkvPitch + col) = float4{o[0], o[1], o[2], o[3]};
+            continue;
+        }
+        if constexpr (EPI == EPI_GELU) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = gelu_f(o[e]);
+        }
+        if constexpr (EPI == EPI_LS) {
+            // res + gamma * x (res may be out: each element is read and
+            // written by one thread)
+            const float4 gv = ld_f32x4(gamma + n), rv = ld_f32x4(res + m * N + n);
+            o[0] = rv.x + gv.x * o[0], o[1] = rv.y + gv.y * o[1];
+            o[2] = rv.z + gv.z * o[2], o[3] = rv.w + gv.w * o[3];
+        }
+        *reinterpret_cast<float4*>(out + m * N + n) = float4{o[0], o[1], o[2], o[3]};
+    }
+    if constexpr (EPI == EPI_QKV) {
+        __syncthreads();
+        // each wave takes 4 rows at a time in the row kernels' lane layout
+        for (int r0 = 4 * wave; r0 < 16 * RB; r0 += 4 * kSkWaves)
+            qkv_heads_out_f32(sm + kSkWaves * kTile + r0 * kQkvPitch, qa, m0 + r0, M, n0, lane, 4);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // generic path: 64 x 64 output tile per 256 threads, 4 x 4 per thread,
 // K in steps of 16 through LDS; f32 accumulation in K order.
 
@@ -1162,6 +1319,42 @@ void launch_f32(hipStream_t st, const void* x, const void* w, const float* bias,
         static_cast<int>(ntiles), la, qa);
 }
 
+template <int EPI, int CB, int RB, bool LN>
+void launch_skinny_as(hipStream_t st, const float* x, const float* w, const float* bias, const float* gamma,
+                      const float* res, float* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
+    const int row_groups = static_cast<int>(ceil_div(M, 16 * RB));
+    const int ngroups = N / (16 * CB) * row_groups;
+    const int64_t blocks = ceil_div(ngroups, 8) * 8;
+    gemm_skinny_kernel<EPI, CB, RB, LN><<<dim3(static_cast<uint32_t>(blocks)), dim3(kSkThreads), 0, st>>>(
+        x, w, bias, gamma, res, out, M, N, K, row_groups, ngroups, qa, la);
+}
+
+// The smallest tile whose workgroups the CUs hold at once (8 rows: 2048
+// columns 1 x 1 8.4 us, 2 x 1 11.9; 8192 columns 16.4, 14.2; 33 rows of 6144: 2 x 2
+// 32.9, 2 x 3 23.3), and 2 x 2 where none does (100 rows of 8192: 2 x 1 82, 2
+// x 2 65, 2 x 3 67).
+template <int EPI, bool LN>
+void launch_skinny(hipStream_t st, const void* x_, const void* w_, const float* bias, const float* gamma,
+                   const void* res_, void* out_, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
+    const float *x = static_cast<const float*>(x_), *w = static_cast<const float*>(w_);
+    const float* res = static_cast<const float*>(res_);
+    float* out = static_cast<float*>(out_);
+    if constexpr (EPI == EPI_QKV) {
+        launch_skinny_as<EPI, 4, 1, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+    } else {
+        const int64_t cus = num_cus();
+        auto groups = [&](int cb, int rb) { return N / (16 * cb) * ceil_div(M, 16 * rb); };
+        if (groups(1, 1) <= cus)
+            launch_skinny_as<EPI, 1, 1, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        else if (groups(2, 1) <= cus)
+            launch_skinny_as<EPI, 2, 1, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        else if (groups(2, 2) > cus && groups(2, 3) <= cus)
+            launch_skinny_as<EPI, 2, 3, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        else
+            launch_skinny_as<EPI, 2, 2, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+    }
+}
+
 template <int EPI, typename P, bool LN>
 void launch_f16(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
                 const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
@@ -1180,7 +1373,11 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
                  const char* op, const QkvArgs& qa = QkvArgs{}, const LnArgs& la = LnArgs{}) {
     if (f32_fast(dt, N, K, x, w, bias, gamma, out, res) &&
         (!LN || (aligned16(la.ln_w) && aligned16(la.ln_b)))) {
-        if (ceil_div(M, F32Shape::kBM) * (N / F32Shape::kBN) < HS_GEMM_F32_NARROW_TILES)
+        // (a rule on M alone, so that one product summed in parts of its
+        // columns, as q, k and v apart, takes the same order of k)
+        if (M <= kSkinnyRows)
+            launch_skinny<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+        else if (ceil_div(M, F32Shape::kBM) * (N / F32Shape::kBN) < HS_GEMM_F32_NARROW_TILES)
             launch_f32<EPI, F32Narrow, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
         else
             launch_f32<EPI, F32Shape, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);

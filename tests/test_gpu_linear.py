@@ -424,3 +424,64 @@ def test_linear_f16_tile_shapes_agree(ctx, n, k):
     for m in (1, 63, 65, 2048 * scale, 2049 * scale, 4097 * scale, 8191 * scale, 8193 * scale,
               8192 * scale + 193):
         assert torch.equal(ctx.linear(x[:m], w, b), big[:m]), m
+
+
+@pytest.mark.parametrize("n,k", [(128, 32), (256, 96), (2048, 544), (6144, 2048), (2048, 8192)])
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 48, 49, 128, 129])
+def test_linear_f32_few_rows(ctx, m, n, k):
+    """Up to 128 rows the weights stream through gemm_skinny_kernel (tiles of
+    1 to 2 x 1 to 3 blocks of 16, K over 16 waves, some without a piece at
+    small k); 129 rows take the tiles. Every epilogue against float64: f32
+    sums of k products (error below k 2^-24 of the sum of magnitudes, which
+    is about sqrt(k) of the result's scale), and the parts of a product's
+    columns equal to the whole."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x, w, b, gamma, res = r(m, k), r(n, k) / k ** 0.5, r(n) * 0.02, r(n), r(m, n)
+    lin = x.double() @ w.double().t().contiguous() + b.double()
+    mag = x.double().abs() @ w.double().abs().t().contiguous() + 1.0
+    tol = mag * (k ** 0.5 + 8) * 2.0 ** -23
+
+    out = ctx.linear(x, w, b)
+    assert bool(((out.double() - lin).abs() <= tol).all())
+    half = n // 2
+    if half % 128 == 0:
+        assert torch.equal(ctx.linear(x, w[half:], b[half:]), out[:, half:])
+    act = ctx.linear_gelu(x, w, b)
+    # A&S 7.1.26: 1.5e-7 absolute on erf, times |v| / 2
+    gel = torch.nn.functional.gelu(lin)
+    assert bool(((act.double() - gel).abs() <= 1.2 * tol + 2e-7 * (1 + lin.abs())).all())
+    want = res.double() + gamma.double() * lin
+    got = ctx.linear_ls_residual(x, w, gamma, res, b, out=res)  # res may be out
+    assert bool(((got.double() - want).abs() <= (1 + gamma.abs()) * tol).all())
+
+
+@pytest.mark.parametrize("s,t", [(1, 1), (1, 16), (3, 17), (2, 64), (1, 129)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_linear_f32_few_rows_heads_and_prologue(ctx, s, t, norm):
+    """The same kernel's q|k|v epilogue and LayerNorm prologue, bit for bit the
+    ops apart."""
+    h, k = 4, 160
+    g = torch.Generator(device="cuda")
+    g.manual_seed(s * 1000 + t)
+    r = lambda *sh: torch.randn(sh, generator=g, device="cuda")  # noqa: E731
+    x, w, b = r(s * t, k), r(3 * h * 64, k) / k ** 0.5, r(3 * h * 64) * 0.02
+    ln = (1 + 0.1 * r(k), 0.1 * r(k))
+    nrm = lambda: (1 + 0.1 * r(64), 0.1 * r(64)) if norm else None  # noqa: E731
+    qn, kn = nrm(), nrm()
+    prefix = min(5, t)
+    ang = r(max(t - prefix, 1), 64)
+    rope = (ang.sin()[:t - prefix].contiguous(), ang.cos()[:t - prefix].contiguous(), prefix) if t > prefix else None
+    got = ctx.linear_qkv_heads(x, w, b, s, t, h, qn=qn, kn=kn, rope=rope)
+    lin = ctx.linear(x, w, b)
+    for i, n in enumerate((qn, kn, None)):
+        part = lin[:, i * h * 64:(i + 1) * h * 64].contiguous()
+        want = ctx.qknorm_rope(part, s, t, h, 64, norm=n, rope=rope if i < 2 else None)
+        tol = 0 if h in (8, 16, 32) else 2e-6
+        assert bool(((got[i] - want).abs() <= tol * (1 + want.abs())).all())
+    fused = ctx.linear_ln_qkv_heads(x, ln, w, b, s, t, h, qn=qn, kn=kn, rope=rope)
+    apart = ctx.linear_qkv_heads(ctx.layernorm(x, *ln), w, b, s, t, h, qn=qn, kn=kn, rope=rope)
+    for a, c in zip(fused, apart):
+        assert torch.equal(a, c)
+    assert torch.equal(ctx.linear_ln_gelu(x, ln, w, b), ctx.linear_gelu(ctx.layernorm(x, *ln), w, b))
