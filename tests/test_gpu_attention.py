@@ -303,6 +303,32 @@ def test_attention_d128_f32(ctx):
     assert np.abs(got - naive64(q, k, v)).max() < 1e-4
 
 
+@pytest.mark.parametrize("s,h,t", [(1, 16, 1), (2, 3, 15), (1, 16, 16), (3, 2, 17), (1, 4, 63),
+                                   (1, 4, 64), (1, 2, 65), (2, 16, 200)])
+@pytest.mark.parametrize("spread", [1.0, 6.0])
+def test_attention_d128_f32_edges(ctx, s, h, t, spread):
+    """attention_d128_kernel (16-query tiles, 16-key blocks over four waves,
+    waves without keys below 49 tokens) against the float64 softmax: within
+    the error of the one-thread-per-query kernel, which unaligned buffers
+    take, and of 1e-5 (f32 scores of 128 products, |score| up to ~60 at the
+    larger spread: 60 x 2^-23 relative on a weight)."""
+    rng = np.random.default_rng(s * 100 + t)
+    q, k, v = (rng.standard_normal((s, h, t, 128)).astype(np.float32) for _ in range(3))
+    q *= np.float32(spread)
+    want = naive64(q, k, v)
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    assert np.abs(got - want).max() < 1e-5 * spread
+    merged = back(ctx.attention_merged(dev(q), dev(k), dev(v)))
+    assert_bit_exact(merged.reshape(s, t, h, 128).transpose(0, 2, 1, 3).copy(), got, "merged d128")
+
+    def odd(a):  # one float past a 16-byte boundary
+        buf = torch.empty(a.size + 1, device="cuda:0")
+        return buf[1:].view(a.shape).copy_(dev(a))
+
+    ref = back(ctx.attention(odd(q), odd(k), odd(v)))
+    assert np.linalg.norm(got - want) <= 1.25 * np.linalg.norm(ref - want) + 1e-7 * np.linalg.norm(want)
+
+
 def test_attention_unsupported_shapes(ctx):
     x16 = torch.zeros((1, 1, 8, 128), dtype=torch.float16, device="cuda:0")
     with pytest.raises(_lib.HsError) as e:
