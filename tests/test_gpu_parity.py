@@ -70,6 +70,22 @@ def test_layernorm(ctx, dtype, rows, dim):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_layernorm_eight_chunks(ctx, dtype):
+    """Rows of 8 x 64 16-byte vectors (f32 2048, the camera head; f16 4096),
+    one row per wave, at row counts around a workgroup's four."""
+    dim = 2048 if dtype == torch.float32 else 4096
+    for rows in (1, 3, 4, 5, 130):
+        x = O.normal(rows, (rows, dim)).astype(NP[dtype])
+        w, b = O.normal(2, (dim,), 1.0, 0.1), O.normal(3, (dim,), 0.0, 0.1)
+        check(back(ctx.layernorm(dev(x), dev(w), dev(b), eps=1e-5)), O.layernorm(x, w, b, 1e-5),
+              f"layernorm {dtype} {rows}x{dim}")
+        st = back(ctx.layernorm_stats(dev(x), eps=1e-5)).astype(np.float64)
+        x64 = x.astype(np.float64)
+        assert np.abs(st[:, 0] - x64.mean(1)).max() < 1e-6
+        assert np.abs(st[:, 1] * np.sqrt(x64.var(1) + 1e-5) - 1).max() < 1e-5
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_layernorm_in_place_and_empty(ctx, dtype):
     x = host(O.normal(14, (9, 1024)), dtype)
     w, b = O.normal(15, (1024,), 1.0, 0.02), O.normal(16, (1024,), 0.0, 0.02)
