@@ -29,11 +29,10 @@
 // stores drain that burst faster than write-allocating ones (fc1 + GELU at
 // S=32: 494 us against 523).
 //
-// f32 (N % 128 == 0, K % 32 == 0; every epilogue but the q|k|v split, with
-// or without the LayerNorm prologue): the same arrangement on the f32
-// matrix cores in 128 x 128 tiles, the epilogue stored straight from the
-// accumulators. Up to 128 rows a kernel that splits K over the waves and
-// streams the weights straight into registers (gemm_skinny_kernel).
+// f32 (N % 128 == 0, K % 32 == 0; every epilogue, with or without the LayerNorm
+// prologue): each operand as two f16 values on the f16 matrix cores
+// (gemm_split_kernel), or up to 128 rows a kernel that splits K over its waves
+// and streams the weights straight into registers (gemm_skinny_kernel).
 //
 // Generic path (the shapes neither covers): a tiled scalar kernel, f32
 // accumulation in K order.
@@ -682,115 +681,12 @@ __global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f16_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// f32 matrix-core path (f32, N % 128 == 0, K % 32 == 0): v_mfma_f32_32x32x2_f32
-// in the f16 kernel's arrangement. A workgroup of WAVES waves in 2 row
-// groups computes a (2 WROWS) x (32 WAVES) tile, each wave WROWS rows x 64
-// columns as out^T blocks of 32 x 32; K in stages of 32 floats through LDS,
-// double-buffered and filled by LDS-DMA. A stage row is 128 bytes (8
-// chunks of 4 floats) with the f16 kernel's swizzle: logical chunk c of row
-// r sits at physical chunk c ^ ((r / 2) % 8). In slice ks of a stage lane
-// (l32, hh) reads logical chunk 2 ks + hh (floats 8 ks + 4 hh .. + 4) of its
-// rows, and MFMA j of the slice takes element j of both operands: it sums
-// k = 8 ks + j (lanes hh = 0) and 8 ks + 4 + j (hh = 1), so the four MFMAs
-// of a slice cover its 8 k. The epilogue stores from the accumulators:
-// register quad r4 of lane (l32, hh) is 4 consecutive columns of one row
-// (16 bytes; the lane pair's quads are 32 contiguous bytes, and the wave's
-// four r4 complete the row's 128 bytes of the block).
-//
-// Shapes: F32Shape, 4 waves, 128 x 128 tiles, 64 KiB of LDS, two
-// workgroups per CU. It beats 8 waves in 256 x 256 tiles (128 KiB, one per
-// CU) at every trunk shape, by 6-9% at S=32 (43968 x 4096 x 1024: 2716 us
-// against 2873) and by 3x where 256 x 256 tiles are too few to fill the
-// chip (2748 x 1024 x 4096, 44 of them: 286 us against 925). Below 512
-// tiles of 128 x 128 (the chip's slots at two per CU) F32Narrow, 4 waves
-// of 32 x 64 in 64 x 128 tiles (48 KiB, three per CU), doubles the tile
-// count: 6-23% faster there (2748 x 1024 x 1024: 74 us against 82; 5496 x
-// 1024 x 4096: 434 against 515), within 5% either way above.
-template <int WAVES, int WROWS>
-struct F32Tile {
-    static constexpr int kWaves = WAVES, kThreads = 64 * WAVES;
-    static constexpr int kBM = 2 * WROWS, kBN = 32 * WAVES;
-    static constexpr int kBK = 32;                      // floats per stage row
-    static constexpr int kXI = kBM * 8 / 64 / WAVES;    // LDS-DMA instructions per wave, x stage
-    static constexpr int kWI = kBN * 8 / 64 / WAVES;    // w stage
-    static constexpr int kRB = WROWS / 32;              // 32-row blocks per wave
-    static constexpr int kWavesPerEu = 8 / WAVES;
-    static_assert(kXI * 64 * WAVES == kBM * 8 && kWI * 64 * WAVES == kBN * 8, "stage split");
-};
-using F32Shape = F32Tile<4, 64>;
-using F32Narrow = F32Tile<4, 32>;
-
-template <typename P>
-struct F32Smem {
-    float x[2][P::kBM * P::kBK];
-    float w[2][P::kBN * P::kBK];
-};
-static_assert(2 * sizeof(F32Smem<F32Shape>) <= 160 * 1024 && 3 * sizeof(F32Smem<F32Narrow>) <= 160 * 1024,
-              "workgroups per CU");
-
-// Per-lane byte offsets of a wave's stage loads (4 instructions each for
-// x and w): instruction i of wave wv brings rows
-// 8 (wv + waves i) .. + 8, lane L row + L / 8 at physical chunk L % 8; x
-// rows past M read row M - 1 (their outputs are masked).
-struct F32Offsets {
-    uint32_t x[4];
-    uint32_t w[4];
-};
-static_assert(F32Shape::kXI <= 4 && F32Shape::kWI <= 4 && F32Narrow::kXI <= 4 && F32Narrow::kWI <= 4,
-              "at most four stage loads per wave and operand");
-
-// xi / wi: the loads per wave of an x / w stage (compile-time after inlining)
-__device__ __forceinline__ F32Offsets f32_offsets(int64_t m0, int M, int K, int waves, int wv,
-                                                  int lane, int xi, int wi) {
-    F32Offsets o;
-    const int prow = lane / 8, pc = lane % 8;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int row = 8 * (wv + waves * i) + prow;
-        const int lrow = static_cast<int>(min(m0 + row, static_cast<int64_t>(M) - 1) - m0);
-        o.x[i] = i < xi ? static_cast<uint32_t>(lrow * K * 4 + 16 * (pc ^ swz(row))) : 0u;
-        o.w[i] = i < wi ? static_cast<uint32_t>(row * K * 4 + 16 * (pc ^ swz(row))) : 0u;
-    }
-    return o;
-}
-
-// This wave's LDS-DMA loads of one stage into xdst / wdst (1 KiB, i.e. 8
-// rows of 32 floats, per instruction); koff = the stage's first column in
-// bytes.
-__device__ __forceinline__ void f32_issue(float* xdst, float* wdst, __amdgpu_buffer_rsrc_t xr,
-                                          __amdgpu_buffer_rsrc_t wr, int koff, const F32Offsets& o,
-                                          int waves, int wv, int xi, int wi) {
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (i < xi)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(xdst + (wv + waves * i) * 256), 16,
-                                                     o.x[i], koff, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (i < wi)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(wdst + (wv + waves * i) * 256), 16,
-                                                     o.w[i], koff, 0, 0);
-}
-
-// Operand chunk c (4 floats) of LDS row `row` (rows of 32 floats).
-__device__ __forceinline__ u32x4 f32_op(const float* buf, int row, int c) {
-    return ld16(buf + row * 32 + 4 * (c ^ swz(row)));
-}
+// f32 products: shared pieces
 
 // The f32 q|k|v epilogue's staging: each wave's block (32 kRB token rows x
 // one head's 64 columns, acc + bias) in rows of kQkvPitch floats (16-byte
 // aligned, 4 banks apart), in the LDS the stages used.
 constexpr int kQkvPitch = 68;
-template <typename P>
-constexpr size_t f32_smem_bytes(int epi) {
-    const size_t loop = sizeof(F32Smem<P>);
-    const size_t qkv = epi == EPI_QKV ? size_t{4} * P::kWaves * 32 * P::kRB * kQkvPitch : 0;
-    return loop > qkv ? loop : qkv;
-}
-static_assert(2 * f32_smem_bytes<F32Shape>(EPI_QKV) <= 160 * 1024 &&
-                  3 * f32_smem_bytes<F32Narrow>(EPI_QKV) <= 160 * 1024,
-              "workgroups per CU with the q|k|v staging");
-
 // The f32 q|k|v epilogue's second phase: the wave's staged block is `rows`
 // token rows of one head of q, k or v. 16 lanes per row hold the head
 // vector in the lane layout of the standalone f32 QK-norm / RoPE op (piece
@@ -847,169 +743,23 @@ __device__ __forceinline__ void qkv_heads_out_f32(const float* stage, const QkvA
     }
 }
 
-template <int EPI, typename P, bool LN>
-__global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f32_kernel(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
-    const float* __restrict__ gamma, const float* res, float* out, int M, int N, int K,
-    int tiles_n, int ntiles, LnArgs la, QkvArgs qa) {
-    constexpr int kRB = P::kRB;
-    __shared__ __align__(16) unsigned char smem_raw[f32_smem_bytes<P>(EPI)];
-    F32Smem<P>& sm = *reinterpret_cast<F32Smem<P>*>(smem_raw);
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
+// The f32 tile kernel's epilogue, from a wave's accumulators (acc[a][b]
+// register r of lane (l32, hh): column col0 + 32 a + 8 (r / 4) + 4 hh + r % 4, row
+// row0 + 32 b + l32). For q|k|v every wave has left the main loop.
+template <int EPI, int kRB>
+__device__ __forceinline__ void f32_epilogue(const f32x16 (&acc)[2][kRB], float* smem, const float* bias,
+                                             const float* gamma, const float* res, float* out, int64_t row0,
+                                             int64_t col0, int M, int N, int wave, int lane, const QkvArgs& qa) {
     const int l32 = lane & 31, hh = lane >> 5;
-#if HS_GEMM_XCD
-    // the f16 kernel's XCD-aware tile order
-    const int per = static_cast<int>(gridDim.x / 8);
-    const int tile = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
-    if (tile >= ntiles) return;  // padding, before any barrier
-#else
-    const int tile = static_cast<int>(blockIdx.x);
-#endif
-    const int64_t m0 = static_cast<int64_t>(tile / tiles_n) * P::kBM;
-    const int64_t n0 = static_cast<int64_t>(tile % tiles_n) * P::kBN;
-    const int wm = (wave / (P::kWaves / 2)) * (32 * kRB);
-    const int wn = (wave % (P::kWaves / 2)) * 64;
-
-    // acc[a][b]: register r of lane (l32, hh) is column wn + 32 a + 8 (r / 4)
-    // + 4 hh + r % 4, row wm + 32 b + l32 of the tile
-    f32x16 acc[2][kRB];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < kRB; b++) acc[a][b] = f32x16{};
-
-    const int nsteps = K / P::kBK;
-    const int wv = wave_in_block();
-    const F32Offsets so = f32_offsets(m0, M, K, P::kWaves, wv, lane, P::kXI, P::kWI);
-    const int xrows = static_cast<int>(min(static_cast<int64_t>(P::kBM), M - m0));
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(x + m0 * K), 0, xrows * K * 4, kRawBufferFlags);
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(w + n0 * K), 0, P::kBN * K * 4, kRawBufferFlags);
-    constexpr int kStageFloats = P::kBK, kStageBytes = P::kBK * 4;
-    auto issue = [&](int buf, int koff) {
-        f32_issue(sm.x[buf], sm.w[buf], xr, wr, koff, so, P::kWaves, wv, P::kXI, P::kWI);
-    };
-    // The LayerNorm prologue (hs_linear_ln*): each lane normalises, in
-    // place, the x pieces that its own stage loads brought (instruction i:
-    // floats (wv + WAVES i) * 256 + 4 lane .. + 4 of the stage), once they
-    // have landed (vmcnt, no barrier) and before the barrier that opens the
-    // stage to every wave. The pieces' rows are fixed for the kernel, so
-    // their (mean, rstd) stay in registers; their logical chunk (lane % 8) ^
-    // swz(row) does not depend on i, so a stage needs 4 columns of ln_w and
-    // ln_b per lane, loaded one stage ahead. Each element becomes what
-    // hs_layernorm stores for it.
-    static_assert(P::kWaves % 2 == 0, "a lane's x pieces share one logical chunk");
-    f32x2 lst[4];
-    int lcol = 0;
-    float4 lw = {0.0f, 0.0f, 0.0f, 0.0f}, lb = lw;
-    if constexpr (LN) {
-#pragma unroll
-        for (int i = 0; i < P::kXI; i++) {
-            const int row = 8 * (wv + P::kWaves * i) + lane / 8;
-            // rows past M hold row M - 1 and take its statistics
-            const int64_t r = min(m0 + row, static_cast<int64_t>(M) - 1);
-            lst[i] = *reinterpret_cast<const f32x2*>(la.stats + 2 * r);
-        }
-        lcol = 4 * ((lane % 8) ^ swz(8 * wv + lane / 8));
-        lw = ld_f32x4(la.ln_w + lcol), lb = ld_f32x4(la.ln_b + lcol);
-    }
-    auto normalise = [&](int buf) {  // with the stage's parameters in lw, lb
-#pragma unroll
-        for (int i = 0; i < P::kXI; i++) {
-            float* piece = sm.x[buf] + (wv + P::kWaves * i) * 256 + 4 * lane;
-            const u32x4 v = ld16(piece);
-            u32x4 o;
-            o[0] = f2u(ln_affine(u2f(v[0]), lst[i][0], lst[i][1], lw.x, lb.x));
-            o[1] = f2u(ln_affine(u2f(v[1]), lst[i][0], lst[i][1], lw.y, lb.y));
-            o[2] = f2u(ln_affine(u2f(v[2]), lst[i][0], lst[i][1], lw.z, lb.z));
-            o[3] = f2u(ln_affine(u2f(v[3]), lst[i][0], lst[i][1], lw.w, lb.w));
-            st16(piece, o);
-        }
-    };
-    issue(0, 0);
-    if (nsteps > 1) issue(1, kStageBytes);
-    if constexpr (LN) {
-        // stage 0 landed (stage 1's loads, the last issued, may be in flight)
-        if (nsteps > 1)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P::kXI + P::kWI) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        normalise(0);
-        if (nsteps > 1) lw = ld_f32x4(la.ln_w + kStageFloats + lcol), lb = ld_f32x4(la.ln_b + kStageFloats + lcol);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    } else {
-        if (nsteps > 1)
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(P::kXI + P::kWI) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    }
-    // operand registers in two sets: the next slice is read from LDS while
-    // the current one multiplies, across stage boundaries too
-    u32x4 A[2][2], B[2][kRB];
-#pragma unroll
-    for (int a = 0; a < 2; a++) A[0][a] = f32_op(sm.w[0], wn + 32 * a + l32, hh);
-#pragma unroll
-    for (int b = 0; b < kRB; b++) B[0][b] = f32_op(sm.x[0], wm + 32 * b + l32, hh);
-    for (int s = 0; s < nsteps; s++) {
-        const int cur = s & 1;
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const int p = ks & 1;
-            if (ks + 1 < 4) {
-                const int kc = 2 * (ks + 1) + hh;
-#pragma unroll
-                for (int a = 0; a < 2; a++) A[p ^ 1][a] = f32_op(sm.w[cur], wn + 32 * a + l32, kc);
-#pragma unroll
-                for (int b = 0; b < kRB; b++) B[p ^ 1][b] = f32_op(sm.x[cur], wm + 32 * b + l32, kc);
-            } else {
-                // every wave's reads of stage s are done and stage s + 1 has
-                // landed (and, with the prologue, is normalised); buffer cur
-                // is refilled with stage s + 2
-                if constexpr (LN) {
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    if (s + 1 < nsteps) {
-                        normalise(cur ^ 1);
-                        if (s + 2 < nsteps) {
-                            const int c = (s + 2) * kStageFloats + lcol;
-                            lw = ld_f32x4(la.ln_w + c), lb = ld_f32x4(la.ln_b + c);
-                        }
-                    }
-                    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                } else {
-                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                }
-                if (s + 2 < nsteps) issue(cur, (s + 2) * kStageBytes);
-                if (s + 1 < nsteps) {
-#pragma unroll
-                    for (int a = 0; a < 2; a++) A[p ^ 1][a] = f32_op(sm.w[cur ^ 1], wn + 32 * a + l32, hh);
-#pragma unroll
-                    for (int b = 0; b < kRB; b++) B[p ^ 1][b] = f32_op(sm.x[cur ^ 1], wm + 32 * b + l32, hh);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int a = 0; a < 2; a++)
-#pragma unroll
-                    for (int b = 0; b < kRB; b++)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(A[p][a][j]), u2f(B[p][b][j]),
-                                                                         acc[a][b], 0, 0, 0);
-        }
-    }
-
     if constexpr (EPI == EPI_QKV) {
-        // every wave has left the main loop: the stages' LDS takes the
-        // waves' blocks
-        __syncthreads();
-        float* stage = reinterpret_cast<float*>(smem_raw) + wave * (32 * kRB * kQkvPitch);
+        // the stages' LDS takes the waves' blocks
+        float* stage = smem + wave * (32 * kRB * kQkvPitch);
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
                 const int cl = 32 * a + 8 * r4 + 4 * hh;
-                const float4 bv = bias ? ld_f32x4(bias + n0 + wn + cl) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+                const float4 bv = bias ? ld_f32x4(bias + col0 + cl) : float4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int b = 0; b < kRB; b++) {
                     u32x4 o;
@@ -1022,20 +772,20 @@ __global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f32_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        qkv_heads_out_f32(stage, qa, m0 + wm, M, n0 + wn, lane, 32 * kRB);
+        qkv_heads_out_f32(stage, qa, row0, M, col0, lane, 32 * kRB);
         return;
     }
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
-            const int64_t n = n0 + wn + 32 * a + 8 * r4 + 4 * hh;
+            const int64_t n = col0 + 32 * a + 8 * r4 + 4 * hh;
             const float4 bv = bias ? ld_f32x4(bias + n) : float4{0.0f, 0.0f, 0.0f, 0.0f};
             float4 gv = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (EPI == EPI_LS) gv = ld_f32x4(gamma + n);
 #pragma unroll
             for (int b = 0; b < kRB; b++) {
-                const int64_t m = m0 + wm + 32 * b + l32;
+                const int64_t m = row0 + 32 * b + l32;
                 if (m >= M) continue;
                 float v[4] = {acc[a][b][4 * r4] + bv.x, acc[a][b][4 * r4 + 1] + bv.y,
                               acc[a][b][4 * r4 + 2] + bv.z, acc[a][b][4 * r4 + 3] + bv.w};
@@ -1055,6 +805,332 @@ __global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f32_kernel(
                 st16_nt(out + m * N + n, o);
             }
         }
+}
+
+// 4 floats normalised as hs_layernorm stores them.
+__device__ __forceinline__ u32x4 ln_quad(u32x4 v, f32x2 st, float4 g, float4 b) {
+    u32x4 o;
+    o[0] = f2u(ln_affine(u2f(v[0]), st[0], st[1], g.x, b.x));
+    o[1] = f2u(ln_affine(u2f(v[1]), st[0], st[1], g.y, b.y));
+    o[2] = f2u(ln_affine(u2f(v[2]), st[0], st[1], g.z, b.z));
+    o[3] = f2u(ln_affine(u2f(v[3]), st[0], st[1], g.w, b.w));
+    return o;
+}
+
+// A wave's 32 kRB x 64 block of an f32 product on v_mfma_f32_32x32x2_f32,
+// operands straight from memory (rows past M read row M - 1): MFMA j of a
+// step takes element j of lane (l32, hh)'s 4 floats at 8 step + 4 hh of both rows.
+template <bool LN, int kRB>
+__device__ __forceinline__ void f32_block(f32x16 (&acc)[2][kRB], const float* x, const float* w, int64_t row0,
+                                       int64_t col0, int M, int K, const LnArgs& la, int l32, int hh) {
+    const float* xp[kRB];
+    f32x2 st[kRB];
+#pragma unroll
+    for (int b = 0; b < kRB; b++) {
+        const int64_t m = min(row0 + 32 * b + l32, static_cast<int64_t>(M) - 1);
+        xp[b] = x + m * K + 4 * hh;
+        if constexpr (LN) st[b] = *reinterpret_cast<const f32x2*>(la.stats + 2 * m);
+    }
+    const float* wp = w + (col0 + l32) * K + 4 * hh;
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < kRB; b++) acc[a][b] = f32x16{};
+#pragma unroll 1
+    for (int k = 0; k < K; k += 8) {
+        u32x4 av[2], bv[kRB];
+#pragma unroll
+        for (int a = 0; a < 2; a++) av[a] = ld16(wp + static_cast<int64_t>(32 * a) * K + k);
+#pragma unroll
+        for (int b = 0; b < kRB; b++) {
+            bv[b] = ld16(xp[b] + k);
+            if constexpr (LN)
+                bv[b] = ln_quad(bv[b], st[b], ld_f32x4(la.ln_w + k + 4 * hh), ld_f32x4(la.ln_b + k + 4 * hh));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int b = 0; b < kRB; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(av[a][j]), u2f(bv[b][j]), acc[a][b], 0, 0, 0);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// f32 products on the f16 matrix cores (N % 128 == 0, K % 32 == 0, more rows
+// than gemm_skinny_kernel takes). The f32 matrix instructions run at a
+// sixteenth of the f16 rate; an f32 value is, to 2^-24 of itself, the sum of
+// two f16 values, a = h + l / 2048 with h = f16(a) and l = f16((a - h) 2048),
+// so that three f16 products with f32 accumulators
+//     sum(h_x h_w)  +  (sum(h_x l_w) + sum(l_x h_w)) / 2048
+// give the f32 product but for l_x l_w / 2^22 (below 2^-24 of |a_x a_w|) and
+// the two roundings of l. Every f16 product is exact in f32, and the chain of
+// accumulations is K / 16 long instead of K / 2, so the result is nearer the
+// 64-bit product than the f32 instructions' (DINO's q|k|v: 2.2e-7 against
+// 5.7e-7, fc2's 4096 terms 3.0e-7 against 8.1e-7).
+//
+// l is held times 2048, in accumulators of its own, so both halves keep 11
+// bits for |a| from 2^-14 to 65504; smaller values lose absolute precision
+// only (2^-36). A row whose largest magnitude is above 65504 or below 2^-13
+// (all zeros apart) would lose more than 2^-23 of it: each workgroup tracks
+// its rows' maxima while it converts, and a tile with such a row (infinities
+// among them) is computed again on v_mfma_f32_32x32x2_f32.
+//
+// A workgroup of WM x WN waves computes 32 RB WM rows x 64 WN columns, a wave 32
+// RB x 64 as out^T blocks. K goes in stages of 32 through LDS, two buffers: a
+// stage row is 128 bytes, logical chunk 2 c holding h and 2 c + 1 l of floats 8
+// c .. + 8, at physical chunk ^ swz(row) (operand reads and these writes
+// conflict-free). The f32 pieces are prefetched into registers a stage ahead
+// and converted once per workgroup between the multiplies (~3 vector
+// instructions per element, 4.5 per MFMA).
+// Bounds: the sum of matrix and vector issue, which overlap little at two waves
+// per SIMD. At 10992 rows, q|k|v / proj / fc1 / fc2, us: 273 / 107 / 358 / 323
+// (242-285 TFLOP/s of f32 product) against 560 / 202 / 694 / 731 on the f32
+// matrix cores (94-133, peak 157); at 2748 rows 98 / 36 / 106 / 107 against 162 /
+// 67 / 199 / 247.
+template <int WM, int WN, int RB_>
+struct SplitTile {
+    static constexpr int kWN = WN, kWaves = WM * WN, kThreads = 64 * kWaves, kRB = RB_;
+    static constexpr int kBM = 32 * RB_ * WM, kBN = 64 * WN, kBK = 32;
+    static constexpr int kPR = kThreads / 4;                                   // rows a pass of pieces covers
+    static constexpr int kXP = kBM / kPR, kWP = kBN / kPR, kPieces = kXP + kWP;  // 8-float pieces per thread
+    static_assert(kXP * kPR == kBM && kWP * kPR == kBN && kPR % 16 == 0, "pieces");
+    struct Smem {
+        f16 x[2][kBM * 64];
+        f16 w[2][kBN * 64];
+    };
+    static constexpr size_t smem_bytes(int epi) {
+        const size_t qkv = epi == EPI_QKV ? size_t{4} * kWaves * 32 * kRB * kQkvPitch : 0;
+        return sizeof(Smem) > qkv ? sizeof(Smem) : qkv;
+    }
+};
+using SplitShape = SplitTile<2, 2, 2>;   // 128 x 128, two workgroups per CU
+using SplitEight = SplitTile<4, 2, 1>;   // 128 x 128 by 8 waves
+using SplitNarrow = SplitTile<2, 2, 1>;  // 64 x 128
+constexpr float kSplitMax = 65504.0f, kSplitMin = 0x1p-13f;
+
+// 8 floats as h and l chunks; mx gathers their largest magnitude.
+__device__ __forceinline__ void split8(const u32x4 (&v)[2], u32x4& hi, u32x4& lo, float& mx) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = u2f(v[i / 2][2 * (i % 2)]), b = u2f(v[i / 2][2 * (i % 2) + 1]);
+        uint32_t hp = pk_f16(a, b);
+        asm("" : "+v"(hp));  // converted once, as a pair
+        const f16x2 h = u2h2(hp);
+        f16x2 l;
+        // a - h is exact in f32
+        l.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, a * 2048.0f));
+        l.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, b * 2048.0f));
+        hi[i] = hp, lo[i] = h22u(l);
+        mx = fmaxf(fmaxf(mx, fabsf(a)), fabsf(b));
+    }
+}
+
+__device__ __forceinline__ u32x4 buf_ld16(__amdgpu_buffer_rsrc_t src, uint32_t voff, int soff) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
+}
+
+template <int EPI, typename P, bool LN>
+__global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    const float* __restrict__ gamma, const float* res, float* out, int M, int N, int K,
+    int tiles_n, int ntiles, LnArgs la, QkvArgs qa) {
+    constexpr int kRB = P::kRB, kXP = P::kXP, kWP = P::kWP;
+    __shared__ __align__(16) unsigned char smem_raw[P::smem_bytes(EPI)];
+    __shared__ int out_of_range;
+    typename P::Smem& sm = *reinterpret_cast<typename P::Smem*>(smem_raw);
+    const int tid = threadIdx.x;
+    const int lane = lane_id(), wave = wave_in_block();
+    const int l32 = lane & 31, hh = lane >> 5;
+#if HS_GEMM_XCD
+    // the f16 kernel's XCD-aware tile order
+    const int per = static_cast<int>(gridDim.x / 8);
+    const int tile = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (tile >= ntiles) return;  // padding, before any barrier
+#else
+    const int tile = static_cast<int>(blockIdx.x);
+#endif
+    const int64_t m0 = static_cast<int64_t>(tile / tiles_n) * P::kBM;
+    const int64_t n0 = static_cast<int64_t>(tile % tiles_n) * P::kBN;
+    const int wm = (wave / P::kWN) * (32 * kRB);
+    const int wn = (wave % P::kWN) * 64;
+    if (tid == 0) out_of_range = 0;
+
+    const int xrows = static_cast<int>(min(static_cast<int64_t>(P::kBM), M - m0));
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(x + m0 * K), 0, xrows * K * 4, kRawBufferFlags);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(w + n0 * K), 0, P::kBN * K * 4, kRawBufferFlags);
+    // Pieces 0 .. kXP of the thread are x's, the rest w's: piece i is row kPR i +
+    // tid / 4 of its operand, floats 8 (tid % 4) .. + 8 of the stage (x rows
+    // past M read row M - 1; their outputs are masked).
+    const int prow = tid / 4, pc = tid % 4;
+    uint32_t off[P::kPieces];
+    f32x2 lst[kXP];
+#pragma unroll
+    for (int i = 0; i < kXP; i++) {
+        const int row = static_cast<int>(min(m0 + P::kPR * i + prow, static_cast<int64_t>(M) - 1) - m0);
+        off[i] = static_cast<uint32_t>(row * K * 4 + 32 * pc);
+        if constexpr (LN) lst[i] = *reinterpret_cast<const f32x2*>(la.stats + 2 * (m0 + row));
+    }
+#pragma unroll
+    for (int i = 0; i < kWP; i++) off[kXP + i] = static_cast<uint32_t>((P::kPR * i + prow) * K * 4 + 32 * pc);
+    // halves offsets of a piece's h and l chunks (kPR rows on: the same swizzle)
+    const int dh = prow * 64 + 8 * ((2 * pc) ^ swz(prow)), dl = prow * 64 + 8 * ((2 * pc + 1) ^ swz(prow));
+
+    u32x4 raw[P::kPieces][2];
+    float mx[P::kPieces];
+#pragma unroll
+    for (int i = 0; i < P::kPieces; i++) mx[i] = 0.0f;
+    const int nsteps = K / P::kBK;
+    auto load_piece = [&](int i, int s) {
+        const __amdgpu_buffer_rsrc_t src = i < kXP ? xr : wr;
+        raw[i][0] = buf_ld16(src, off[i], s * 128);
+        raw[i][1] = buf_ld16(src, off[i] + 16, s * 128);
+    };
+    // Piece i of stage s into buffer buf, as h and l.
+    auto store_piece = [&](int i, int s, int buf) {
+        if constexpr (LN) {
+            if (i < kXP) {
+                // each element as hs_layernorm stores it
+                const int c = s * P::kBK + 8 * pc;
+                raw[i][0] = ln_quad(raw[i][0], lst[i < kXP ? i : 0], ld_f32x4(la.ln_w + c), ld_f32x4(la.ln_b + c));
+                raw[i][1] = ln_quad(raw[i][1], lst[i < kXP ? i : 0], ld_f32x4(la.ln_w + c + 4), ld_f32x4(la.ln_b + c + 4));
+            }
+        }
+        u32x4 h, l;
+        split8(raw[i], h, l, mx[i]);
+        f16* dst = (i < kXP ? sm.x[buf] + P::kPR * 64 * i : sm.w[buf] + P::kPR * 64 * (i - kXP));
+        st16(dst + dh, h);
+        st16(dst + dl, l);
+    };
+
+    // acc[a][b] (and the 1 / 2048 part, acl): register r of lane (l32, hh) is
+    // column wn + 32 a + 8 (r / 4) + 4 hh + r % 4, row wm + 32 b + l32
+    f32x16 acc[2][kRB], acl[2][kRB];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < kRB; b++) acc[a][b] = f32x16{}, acl[a][b] = f32x16{};
+
+    h8 Ah[2][2], Bh[2][kRB], Al[2], Bl[kRB];  // h operands of two slices, l of one
+    auto read_h = [&](int ks, int buf) {
+        const int ch = 2 * (2 * ks + hh);
+#pragma unroll
+        for (int a = 0; a < 2; a++) Ah[ks][a] = ld_op(sm.w[buf], wn + 32 * a + l32, ch);
+#pragma unroll
+        for (int b = 0; b < kRB; b++) Bh[ks][b] = ld_op(sm.x[buf], wm + 32 * b + l32, ch);
+    };
+    auto read_l = [&](int ks, int buf) {
+        const int ch = 2 * (2 * ks + hh) + 1;
+#pragma unroll
+        for (int b = 0; b < kRB; b++) Bl[b] = ld_op(sm.x[buf], wm + 32 * b + l32, ch);
+#pragma unroll
+        for (int a = 0; a < 2; a++) Al[a] = ld_op(sm.w[buf], wn + 32 * a + l32, ch);
+    };
+    // part 0 h_x h_w, 1 l_x h_w, 2 h_x l_w of slice ks
+    auto multiply = [&](int ks, int part) {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < kRB; b++) {
+                if (part == 0)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ks][a], Bh[ks][b], acc[a][b], 0, 0, 0);
+                else if (part == 1)
+                    acl[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ks][a], Bl[b], acl[a][b], 0, 0, 0);
+                else
+                    acl[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al[a], Bh[ks][b], acl[a][b], 0, 0, 0);
+            }
+    };
+#pragma unroll
+    for (int i = 0; i < P::kPieces; i++) load_piece(i, 0);
+#pragma unroll
+    for (int i = 0; i < P::kPieces; i++) store_piece(i, 0, 0);
+    if (nsteps > 1) {
+#pragma unroll
+        for (int i = 0; i < P::kPieces; i++) load_piece(i, 1);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    read_h(0, 0);
+    // A stage's six groups of multiplies. In the first five, stage s + 1 is
+    // converted into the other buffer (last read before the barrier of the
+    // step before) and stage s + 2's pieces are loaded behind it; the barrier
+    // then opens stage s + 1, and its first h operands are read under the last
+    // group. NEXT: stage s + 1 exists.
+    auto step = [&](int s, auto next_c) {
+        constexpr bool NEXT = decltype(next_c)::value;
+        const int cur = s & 1;
+        const int ld = s + 2 < nsteps ? s + 2 : s + 1;  // (past the end: not used)
+        auto convert = [&](int i) {
+            if (NEXT && i < P::kPieces) {
+                store_piece(i, s + 1, cur ^ 1);
+                load_piece(i, ld);
+            }
+        };
+        // A group's reads, then its MFMAs with the conversion's vector work
+        // between them; its loads leave with it (left to the compiler they
+        // sank to the stage's end, a group before their use: 380 us for fc1
+        // at 10992 rows against 358).
+        auto group = [&](auto reads, auto conv) {
+            if constexpr (reads.value) __builtin_amdgcn_sched_group_barrier(0x100, 2 + kRB, 0);  // LDS reads
+#pragma unroll
+            for (int q = 0; q < 2 * kRB; q++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
+                if constexpr (NEXT && conv.value) __builtin_amdgcn_sched_group_barrier(0x002, 16 / kRB, 0);  // VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr std::true_type yes;
+        constexpr std::false_type no;
+        read_l(0, cur);
+        convert(0);
+        multiply(0, 0);
+        group(yes, yes);
+        convert(1);
+        multiply(0, 1);
+        group(no, yes);
+        read_h(1, cur);
+        convert(2);
+        multiply(0, 2);
+        group(yes, yes);
+        read_l(1, cur);
+        convert(3);
+        multiply(1, 0);
+        group(yes, yes);
+        multiply(1, 1);
+        group(no, no);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (NEXT) read_h(0, cur ^ 1);
+        multiply(1, 2);
+        group(next_c, no);
+    };
+    static_assert(P::kPieces <= 4, "one piece per group of multiplies");
+    for (int s = 0; s + 1 < nsteps; s++) step(s, std::true_type{});
+    step(nsteps - 1, std::false_type{});
+
+    // a row's four threads are a quad
+    bool bad = false;
+    auto range = [&](float v) {
+        v = fmaxf(v, dpp<kQuadXor1>(v));
+        v = fmaxf(v, dpp<kQuadXor2>(v));
+        bad = bad || v > kSplitMax || (v > 0.0f && v < kSplitMin);
+    };
+#pragma unroll
+    for (int i = 0; i < P::kPieces; i++) range(mx[i]);
+    if (bad) out_of_range = 1;
+    __syncthreads();  // also: every wave has left the main loop
+    if (out_of_range == 0) {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < kRB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[a][b][r] = fmaf(acl[a][b][r], 1.0f / 2048.0f, acc[a][b][r]);
+    } else {
+        f32_block<LN, kRB>(acc, x, w, m0 + wm, n0 + wn, M, K, la, l32, hh);
+    }
+    f32_epilogue<EPI, kRB>(acc, reinterpret_cast<float*>(smem_raw), bias, gamma, res, out, m0 + wm, n0 + wn, M, N, wave, lane, qa);
 }
 
 // ---------------------------------------------------------------------------
@@ -1082,17 +1158,6 @@ __device__ __forceinline__ f32x4 sk_mfma(u32x4 a, u32x4 b, f32x4 c) {
 #pragma unroll
     for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(u2f(a[j]), u2f(b[j]), c, 0, 0, 0);
     return c;
-}
-
-// 4 floats of an x row at column k, normalised as hs_layernorm stores them.
-__device__ __forceinline__ u32x4 sk_ln(u32x4 v, f32x2 st, const LnArgs& la, int k) {
-    const float4 g = ld_f32x4(la.ln_w + k), b = ld_f32x4(la.ln_b + k);
-    u32x4 o;
-    o[0] = f2u(ln_affine(u2f(v[0]), st[0], st[1], g.x, b.x));
-    o[1] = f2u(ln_affine(u2f(v[1]), st[0], st[1], g.y, b.y));
-    o[2] = f2u(ln_affine(u2f(v[2]), st[0], st[1], g.z, b.z));
-    o[3] = f2u(ln_affine(u2f(v[3]), st[0], st[1], g.w, b.w));
-    return o;
 }
 
 template <int EPI, int CB, int RB, bool LN>
@@ -1161,7 +1226,8 @@ __global__ __launch_bounds__(kSkThreads) void gemm_skinny_kernel(
         for (int h = 0; h < 2; h++) {
             if constexpr (LN) {
 #pragma unroll
-                for (int i = 0; i < RB; i++) b[h][i] = sk_ln(b[h][i], st[i], la, kc + 16 * h + 4 * g);
+                for (int i = 0; i < RB; i++) b[h][i] = ln_quad(b[h][i], st[i], ld_f32x4(la.ln_w + kc + 16 * h + 4 * g),
+                                      ld_f32x4(la.ln_b + kc + 16 * h + 4 * g));
             }
 #pragma unroll
             for (int c = 0; c < CB; c++)
@@ -1294,29 +1360,43 @@ bool takes_fast_path(hs_dtype dt, int N, int K, const void* x, const void* w, co
            (!LN || (aligned16(la.ln_w) && aligned16(la.ln_b)));
 }
 
-#ifndef HS_GEMM_F32_NARROW_TILES
-#define HS_GEMM_F32_NARROW_TILES 512  // 128 x 128 tiles below which F32Narrow runs
-#endif
+constexpr int kF32ColTile = 128;  // columns of an f32 tile: N is a multiple of it
 
 // f32 matrix-core eligibility: shape and alignment.
 bool f32_fast(hs_dtype dt, int N, int K, const void* x, const void* w, const float* bias,
               const float* gamma, const void* out, const void* res) {
     // K <= 2^19 keeps a tile's byte offsets (128 rows x K x 4) in 32 bits
-    return dt == HS_F32 && N % F32Shape::kBN == 0 && K > 0 && K % F32Shape::kBK == 0 &&
+    return dt == HS_F32 && N % kF32ColTile == 0 && K > 0 && K % SplitShape::kBK == 0 &&
            K <= (1 << 19) && aligned16(x) && aligned16(w) && (!bias || aligned16(bias)) &&
            (!gamma || aligned16(gamma)) && aligned16(out) && (!res || aligned16(res));
 }
 
 template <int EPI, typename P, bool LN>
-void launch_f32(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
-                const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
+void launch_split_as(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
+                     const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
     const int tiles_n = N / P::kBN;
     const int64_t ntiles = ceil_div(M, P::kBM) * tiles_n;
     const int64_t blocks = HS_GEMM_XCD ? ceil_div(ntiles, 8) * 8 : ntiles;
-    gemm_f32_kernel<EPI, P, LN><<<dim3(static_cast<uint32_t>(blocks)), dim3(P::kThreads), 0, st>>>(
+    gemm_split_kernel<EPI, P, LN><<<dim3(static_cast<uint32_t>(blocks)), dim3(P::kThreads), 0, st>>>(
         static_cast<const float*>(x), static_cast<const float*>(w), bias, gamma,
         static_cast<const float*>(res), static_cast<float*>(out), M, N, K, tiles_n,
         static_cast<int>(ntiles), la, qa);
+}
+
+// 128 x 128 tiles by two 4-wave workgroups per CU; where one per CU holds
+// them all, by one of 8 waves (2748 rows, fc2: 107 us against 113), and where half
+// the CUs would, in 64 x 128 tiles (1374 rows, fc2: 85 us against 108 and 98).
+// Every shape sums k in one order.
+template <int EPI, bool LN>
+void launch_split(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
+                  const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
+    const int64_t tiles = ceil_div(M, SplitShape::kBM) * (N / SplitShape::kBN), cus = num_cus();
+    if (2 * tiles <= cus)
+        launch_split_as<EPI, SplitNarrow, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+    else if (tiles <= cus)
+        launch_split_as<EPI, SplitEight, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+    else
+        launch_split_as<EPI, SplitShape, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
 }
 
 template <int EPI, int CB, int RB, bool LN>
@@ -1377,10 +1457,8 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
         // columns, as q, k and v apart, takes the same order of k)
         if (M <= kSkinnyRows)
             launch_skinny<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
-        else if (ceil_div(M, F32Shape::kBM) * (N / F32Shape::kBN) < HS_GEMM_F32_NARROW_TILES)
-            launch_f32<EPI, F32Narrow, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
         else
-            launch_f32<EPI, F32Shape, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
+            launch_split<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
         return check_launch(op);
     }
     if (takes_fast_path<LN>(dt, N, K, x, w, bias, gamma, out, res, la)) {
@@ -1419,7 +1497,7 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
     if constexpr (EPI == EPI_QKV) {
         return fail(HS_EUNSUPPORTED,
                     "%s: needs K %% %d == 0 (f16) or %% %d == 0 (f32) and 16-byte aligned buffers", op,
-                    kBK, F32Shape::kBK);
+                    kBK, SplitShape::kBK);
     } else {
         const int tiles_n = static_cast<int>(ceil_div(N, kGT));
         const int64_t blocks = ceil_div(M, kGT) * tiles_n;
@@ -1527,7 +1605,7 @@ hs_status qkv_setup(const char* op, hs_dtype dt, const void* x, const void* w_qk
     // The fused epilogue needs one head per wave (64 columns) and whole
     // column tiles (256 in f16, 128 in f32); other shapes run linear then
     // qknorm_rope.
-    const int64_t tile_n = dt == HS_F16 ? F16Big::kBN : F32Shape::kBN;
+    const int64_t tile_n = dt == HS_F16 ? F16Big::kBN : kF32ColTile;
     if (d != 64 || N % tile_n != 0)
         return fail(HS_EUNSUPPORTED, "%s: needs head dim 64 and 3*H*64 %% %lld == 0", op,
                     static_cast<long long>(tile_n));
@@ -1662,7 +1740,7 @@ extern "C" hs_status hs_linear_ln_qkv_heads(hs_stream_t stream, hs_dtype dt, con
                                           nullptr, la))
         return fail(HS_EUNSUPPORTED,
                     "%s: needs K %% %d == 0 (f16) or %% %d == 0 (f32) and 16-byte aligned buffers", op,
-                    kBK, F32Shape::kBK);
+                    kBK, SplitShape::kBK);
     hipStream_t st = static_cast<hipStream_t>(stream);
     rc = hs_layernorm_stats(st, dt, x, workspace, M, k, eps);
     if (rc != HS_OK) return rc;

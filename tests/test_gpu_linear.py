@@ -485,3 +485,99 @@ def test_linear_f32_few_rows_heads_and_prologue(ctx, s, t, norm):
     for a, c in zip(fused, apart):
         assert torch.equal(a, c)
     assert torch.equal(ctx.linear_ln_gelu(x, ln, w, b), ctx.linear_gelu(ctx.layernorm(x, *ln), w, b))
+
+
+def _split_operands(m, n, k, seed, w_scale=1.0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.randn((m, k), generator=g, device="cuda")
+    w = torch.randn((n, k), generator=g, device="cuda") / k ** 0.5 * w_scale
+    return x, w, torch.randn(n, generator=g, device="cuda") * 0.02
+
+
+# (m, n): 64 x 128 tiles, 128 x 128 by 8 waves, 128 x 128 by 4 (256 CUs), with
+# row remainders
+@pytest.mark.parametrize("m,n", [(129, 128), (191, 1024), (2049, 1024), (2177, 2048), (4200, 1024),
+                                 (5000, 3072)])
+@pytest.mark.parametrize("k", [32, 64, 96, 1024])
+def test_linear_f32_split(ctx, m, n, k):
+    """f32 products as three f16 ones: closer to the float64 product than a
+    plain f32 chain of k / 2 terms is (relative 2-norm; 2^-24 per rounding, a
+    chain's error grows with sqrt(k)), and rows and column parts of a call
+    equal the same of a larger one."""
+    x, w, b = _split_operands(m, n, k, m + n + k)
+    out = ctx.linear(x, w, b)
+    want = x.double() @ w.double().t().contiguous() + b.double()
+    err = ((out.double() - want).norm() / want.norm()).item()
+    assert err < 2.0 ** -24 * (1.5 + 0.12 * k ** 0.5), err
+    for rows in (129, m - 1):
+        if rows > 128:
+            assert torch.equal(ctx.linear(x[:rows], w, b), out[:rows]), rows
+    if n > 1024:
+        assert torch.equal(ctx.linear(x, w[1024:], b[1024:]), out[:, 1024:])
+
+
+@pytest.mark.parametrize("xs,ws", [(1e-3, 1.0), (200.0, 1e-2), (3000.0, 100.0), (1e-9, 1.0), (1.0, 1e-12),
+                                   (1e6, 1.0), (1e20, 1e10)])
+def test_linear_f32_split_ranges(ctx, xs, ws):
+    """Magnitudes inside the f16 pair's range and, below 2^-13 or above 65504 a
+    row, outside it, where a tile is computed again in f32: the same relative
+    error everywhere."""
+    x, w, _ = _split_operands(300, 256, 512, 5)
+    x *= xs
+    w *= ws
+    want = x.double() @ w.double().t().contiguous()
+    err = ((ctx.linear(x, w).double() - want).norm() / want.norm()).item()
+    assert err < 6e-7, err
+
+
+def test_linear_f32_split_mixed_rows(ctx):
+    """Zero rows, tiny rows, huge rows, infinities and NaN beside ordinary
+    rows, in x and in w: every row as precise as alone, non-finite values only
+    where the float64 product has them."""
+    x, w, b = _split_operands(400, 384, 640, 11)
+    x[3] = 0
+    x[140] *= 1e-20
+    x[141, ::2] = 0
+    x[270] *= 1e8
+    x[271, 5] = float("inf")
+    x[272, 7] = float("nan")
+    x[399, 100] = 7e4
+    w[5] *= 1e-15
+    w[200] = 0
+    w[383, 639] = float("-inf")
+    out = ctx.linear(x, w, b).double()
+    want = x.double() @ w.double().t().contiguous() + b.double()
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(out))
+    assert torch.equal(torch.isnan(want), torch.isnan(out))
+    assert torch.equal(want[torch.isinf(want)], out[torch.isinf(want)])
+    mag = torch.nan_to_num(x.double(), 0, 0, 0).abs() @ torch.nan_to_num(w.double(), 0, 0, 0).abs().t().contiguous()
+    bound = (mag + b.abs()) * 640 ** 0.5 * 2.0 ** -23 + 1e-45
+    assert bool(((out - want).abs()[fin] <= bound[fin]).all())
+
+
+@pytest.mark.parametrize("s,t,h", [(1, 129, 4), (2, 700, 16), (3, 1400, 16)])
+def test_linear_f32_split_heads_and_prologue(ctx, s, t, h):
+    """The q|k|v epilogue and the LayerNorm prologue of the three tile
+    shapes, bit for bit the ops apart (within 2e-6 for 4 heads)."""
+    k = 256
+    x, w, b = _split_operands(s * t, 3 * h * 64, k, t)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    r = lambda *sh: torch.randn(sh, generator=g, device="cuda")  # noqa: E731
+    ln, qn, kn = ((1 + 0.1 * r(n), 0.1 * r(n)) for n in (k, 64, 64))
+    ang = r(t - 5, 64)
+    rope = (ang.sin(), ang.cos(), 5)
+    got = ctx.linear_qkv_heads(x, w, b, s, t, h, qn=qn, kn=kn, rope=rope)
+    hd = h * 64
+    for i, n in enumerate((qn, kn, None)):
+        part = ctx.linear(x, w[i * hd:(i + 1) * hd], b[i * hd:(i + 1) * hd])
+        want = ctx.qknorm_rope(part, s, t, h, 64, norm=n, rope=rope if i < 2 else None)
+        tol = 0 if h in (8, 16, 32) else 2e-6
+        assert bool(((got[i] - want).abs() <= tol * (1 + want.abs())).all())
+    xn = ctx.layernorm(x, *ln)
+    for a, c in zip(ctx.linear_ln_qkv_heads(x, ln, w, b, s, t, h, qn=qn, kn=kn, rope=rope),
+                    ctx.linear_qkv_heads(xn, w, b, s, t, h, qn=qn, kn=kn, rope=rope)):
+        assert torch.equal(a, c)
+    assert torch.equal(ctx.linear_ln_gelu(x, ln, w, b), ctx.linear_gelu(xn, w, b))
