@@ -27,7 +27,7 @@
 // XCD, so its K/V stream through that XCD's L2.
 //
 // f32, D = 64 (16-byte aligned buffers): the same transposed flash scheme
-// on v_mfma_f32_32x32x2_f32 (flash_f32_kernel).
+// with each f32 value as two f16 ones (flash_split_kernel).
 //
 // f32, D = 128 (16-byte aligned buffers): attention_d128_kernel.
 //
@@ -170,6 +170,8 @@ __device__ __forceinline__ float halves_sum(float v) {
     return __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) +
            __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
 }
+
+__device__ __forceinline__ float xor_lanes(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
 __device__ __forceinline__ void mask_tail(f32x16 (&s)[kKB], int key0, int t, int hh) {
 #pragma unroll
@@ -570,9 +572,9 @@ __global__ __launch_bounds__(256) void merge_scalar_kernel(const T* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// f32 flash attention, head_dim 64, on v_mfma_f32_32x32x2_f32. A workgroup
-// of kF32Waves waves takes kF32Q queries of one (frame, head), a wave 32 of
-// them; keys stream through LDS in tiles of kF32Keys: K row-major [key][dim]
+// f32 flash attention, head_dim 64, on v_mfma_f32_32x32x2_f32, for the
+// workgroups whose values the split kernel below does not fit. A wave takes 32
+// queries of one (frame, head); keys stream through LDS in tiles of kF32Keys: K row-major [key][dim]
 // and V transposed [dim][key], rows padded to kF32Pitch floats, written
 // from a register prefetch of the next tile issued while the current one
 // computes. Per tile and wave, in transposed form so that a lane's column is
@@ -589,48 +591,29 @@ __global__ __launch_bounds__(256) void merge_scalar_kernel(const T* __restrict__
 //     hh), element e of V^T row (dim) n's chunk at key 8 qd + 4 hh and the
 //     weight in score register j, which is that same key: the scores are
 //     the B operand as they stand.
-// The output (O / l) leaves from the accumulators: register quad r4 of lane
-// (n, hh) is dims 32 db + 8 r4 + 4 hh .. + 4 of query n, one 16-byte store.
-constexpr int kF32Waves = 4;
-constexpr int kF32Threads = 64 * kF32Waves;
-constexpr int kF32Q = 32 * kF32Waves;  // queries per workgroup
-constexpr int kF32Keys = 64;           // keys per LDS tile
-constexpr int kF32Pitch = 68;          // floats per LDS row (16-byte aligned, 4 banks apart)
-constexpr int kF32Loads = kF32Keys * kD / 4 / kF32Threads;  // 16-byte loads per thread, K or V
-static_assert(kF32Loads * kF32Threads * 4 == kF32Keys * kD, "tile split");
+// Register quad r4 of lane (n, hh) is dims 32 db + 8 r4 + 4 hh .. + 4 of query n.
+constexpr int kF32Keys = 64;   // keys per LDS tile
+constexpr int kF32Pitch = 68;  // floats per LDS row (16-byte aligned, 4 banks apart)
 
 struct alignas(16) F32FlashSmem {
     float k[kF32Keys * kF32Pitch];  // [key][dim]
     float vt[kD * kF32Pitch];       // [dim][key]
 };
 
-__global__ __launch_bounds__(kF32Threads, 2) void flash_f32_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    float* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c, int token_major) {
-    __shared__ F32FlashSmem sm;
-    // the f16 kernel's XCD-aware order: the query tiles of one (frame,
-    // head) run on one XCD and share its L2 copy of K and V
-    const int b = blockIdx.x;
-    const int slot = b / kXcds;
-    const int sh = (slot / qtiles) * kXcds + b % kXcds;
-    if (sh >= sh_count) return;  // workgroup-uniform, before any barrier
-    const int qt = slot % qtiles;
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = tid >> 6;
-    const int n = lane & 31, hh = lane >> 5;
-    const int64_t base = static_cast<int64_t>(sh) * t * kD;
-    const float* kb = k + base;
-    const float* vb = v + base;
-
-    // query n of the wave (queries past T read row T - 1; not stored)
-    const int qi = qt * kF32Q + wave * 32 + n;
-    const float* qrow = q + base + static_cast<int64_t>(min(qi, t - 1)) * kD;
+// The unnormalised output of query qi of the wave in o, returning the sum of
+// its weights; every wave of the workgroup calls it (barriers inside). q, k, v
+// are the (frame, head)'s rows; queries past T read row T - 1.
+template <int W>
+__device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm, const float* qb, const float* kb,
+                                                const float* vb, int qi, int t, float c, int tid, int n, int hh) {
+    constexpr int kF32Threads = 64 * W;
+    constexpr int kF32Loads = kF32Keys * kD / 4 / kF32Threads;  // 16-byte loads per thread, K or V
+    const float* qrow = qb + static_cast<int64_t>(min(qi, t - 1)) * kD;
     float4 qv[8];
 #pragma unroll
     for (int g = 0; g < 8; g++) qv[g] = ld_f32x4(qrow + 8 * g + 4 * hh);
 
-    f32x16 o[2] = {f32x16{}, f32x16{}};
+    o[0] = f32x16{}, o[1] = f32x16{};
     float m = -3.0e38f, l = 0.0f;
 
     // staging: load i of thread tid is float4 f = tid + kF32Threads i of the
@@ -658,6 +641,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void flash_f32_kernel(
         }
     };
     load(0);
+#pragma unroll 1
     for (int k0 = 0; k0 < t; k0 += kF32Keys) {
         __syncthreads();  // every wave's reads of the previous tile are done
         stage();
@@ -718,18 +702,299 @@ __global__ __launch_bounds__(kF32Threads, 2) void flash_f32_kernel(
                     o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, s[kb2][4 * qd + 3], o[db], 0, 0, 0);
                 }
     }
+    return l;
+}
+
+// ---------------------------------------------------------------------------
+// f32 flash attention, head_dim 64, on the f16 matrix cores. The f32 matrix
+// instructions run at a sixteenth of the f16 rate; an f32 value is, to 2^-24 of
+// itself, h + l / 2048 with h = f16(a) and l = f16((a - h) 2048), so each
+// product is three f16 products with f32 accumulators (h h in one set, h l
+// and l h in a second that counts 1 / 2048), l l (below 2^-24) left out. Queries
+// are split once, K and V as their tiles are staged, the softmax weights (f32;
+// the row sum adds them unsplit) where the f16 kernel rounds them. The rest is the f16 kernel: W waves of 32
+// queries over shared 64-key tiles, double-buffered (the next tile's rows in
+// registers while the current one computes), S^T = K Q^T, the lazy running
+// max, V^T through the transposing read, O^T += V^T P^T.
+//
+// Both halves keep 11 bits for |a| from 2^-14 to 65504, smaller values an
+// absolute 2^-36. A query or key row, or a V column, whose largest magnitude is
+// above 65504 or below 2^-13 (all zeros apart) would lose more than 2^-23 of it:
+// the workgroup then computes its queries again on the f32 matrix
+// instructions (flash_f32_body).
+//
+// Bounds: matrix and vector issue, 48 MFMAs and ~350 vector instructions per
+// wave and tile, which overlap little: two waves per SIMD in step. 16 heads of
+// 1374 tokens, us on the f32 matrix instructions and here: 1 sequence 111, 55;
+// 2, 202, 67; 8, 567, 215 (290 TFLOP/s). Relative error against 64 bits 8.6e-7,
+// 3.8e-7.
+constexpr float kSplitMax = 65504.0f, kSplitMin = 0x1p-13f;
+
+template <int W>
+struct SplitFlashSmem {
+    f16 k[2][2][64 * kKPitch];  // [buffer][h, l]
+    f16 v[2][2][64 * kVPitch];
+};
+
+// 8 floats as h and l chunks.
+__device__ __forceinline__ void split8(const float4 (&v)[2], u32x4& hi, u32x4& lo) {
+    const float f[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t hp = pk_f16(f[2 * i], f[2 * i + 1]);
+        asm("" : "+v"(hp));  // converted once, as a pair
+        const f16x2 h = u2h2(hp);
+        f16x2 l;
+        // a - h is exact in f32
+        l.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, f[2 * i] * 2048.0f));
+        l.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, f[2 * i + 1] * 2048.0f));
+        hi[i] = hp, lo[i] = h22u(l);
+    }
+}
+__device__ __forceinline__ float max8(const float4 (&v)[2]) {
+    return fmaxf(fmaxf(fmaxf(fabsf(v[0].x), fabsf(v[0].y)), fmaxf(fabsf(v[0].z), fabsf(v[0].w))),
+                 fmaxf(fmaxf(fabsf(v[1].x), fabsf(v[1].y)), fmaxf(fabsf(v[1].z), fabsf(v[1].w))));
+}
+// Buffer descriptor word 3 for raw (unstructured, stride 0) buffers on gfx950.
+constexpr int kRawBufferFlags = 0x00020000;
+__device__ __forceinline__ float4 buf_ld(__amdgpu_buffer_rsrc_t src, uint32_t voff, int soff) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
+}
+__device__ __forceinline__ bool split_unfit(float mx) { return mx > kSplitMax || (mx > 0.0f && mx < kSplitMin); }
+
+template <int W>
+__global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    float* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c, int token_major) {
+    constexpr int kThr = 64 * W, kPc = 64 * 8 / kThr;  // 8-float pieces per thread of a K or V tile
+    union Smem {
+        SplitFlashSmem<W> split;
+        F32FlashSmem f32;
+    };
+    __shared__ __align__(16) Smem smem;
+    __shared__ int unfit;
+    __shared__ uint32_t vmax[64];  // bits of the largest |V| per dim
+    SplitFlashSmem<W>& sm = smem.split;
+    // the f16 kernel's XCD-aware order
+    const int b = blockIdx.x;
+    const int slot = b / kXcds;
+    const int sh = (slot / qtiles) * kXcds + b % kXcds;
+    if (sh >= sh_count) return;  // workgroup-uniform, before any barrier
+    const int qt = slot % qtiles;
+    const int tid = threadIdx.x;
+    const int lane = lane_id();
+    const int wave = wave_in_block();
+    const int n = lane & 31, hh = lane >> 5;
+    const int64_t base = static_cast<int64_t>(sh) * t * kD;
+    const float* kb = k + base;
+    const float* vb = v + base;
+    const int qi = qt * 32 * W + wave * 32 + n;
+    const bool live = qt * 32 * W + wave * 32 < t;  // wave-uniform: some query below T
+    if (tid == 0) unfit = 0;
+    if (tid < 64) vmax[tid] = 0;
+
+    // staging: piece i of the thread is key row 8 W i + tid / 8, dims 8 (tid %
+    // 8) .. + 8; rows past the end read zeros (masked below)
+    const int prow = tid / 8, pd = 8 * (tid % 8);
+    const __amdgpu_buffer_rsrc_t krs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, t * kD * 4, kRawBufferFlags);
+    const __amdgpu_buffer_rsrc_t vrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, t * kD * 4, kRawBufferFlags);
+    const uint32_t voff0 = static_cast<uint32_t>((prow * kD + pd) * 4);
+    float4 kr[kPc][2], vr[kPc][2];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < kPc; i++) {
+            const int so = (k0 + 8 * W * i) * kD * 4;
+            kr[i][0] = buf_ld(krs, voff0, so), kr[i][1] = buf_ld(krs, voff0 + 16, so);
+            vr[i][0] = buf_ld(vrs, voff0, so), vr[i][1] = buf_ld(vrs, voff0 + 16, so);
+        }
+    };
+    bool bad = false;
+    float vm[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < kPc; i++) {
+            const int row = 8 * W * i + prow;
+            u32x4 h, l;
+            split8(kr[i], h, l);
+            st16(&sm.k[buf][0][row * kKPitch + pd], h);
+            st16(&sm.k[buf][1][row * kKPitch + pd], l);
+            // the row's eight threads are an aligned group of eight lanes
+            float mx = max8(kr[i]);
+            mx = fmaxf(mx, dpp<kQuadXor1>(mx));
+            mx = fmaxf(mx, dpp<kQuadXor2>(mx));
+            mx = fmaxf(mx, dpp<kRowHalfMirror>(mx));
+            bad = bad || split_unfit(mx);
+            split8(vr[i], h, l);
+            st16(&sm.v[buf][0][row * kVPitch + pd], h);
+            st16(&sm.v[buf][1][row * kVPitch + pd], l);
+            const float f[8] = {vr[i][0].x, vr[i][0].y, vr[i][0].z, vr[i][0].w,
+                                vr[i][1].x, vr[i][1].y, vr[i][1].z, vr[i][1].w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) vm[e] = fmaxf(vm[e], fabsf(f[e]));
+        }
+    };
+    load(0);
+
+    // Q^T as the B operand: lane (n, hh) holds dims 16 ks + 8 hh .. + 8 of its
+    // query (past T: row T - 1, not stored)
+    h8 qh[4], ql[4];
+    {
+        const float* qrow = q + base + static_cast<int64_t>(min(qi, t - 1)) * kD + 8 * hh;
+        float mx = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            const float4 f[2] = {ld_f32x4(qrow + 16 * ks), ld_f32x4(qrow + 16 * ks + 4)};
+            u32x4 h, l;
+            split8(f, h, l);
+            qh[ks] = as_h8(h), ql[ks] = as_h8(l);
+            mx = fmaxf(mx, max8(f));
+        }
+        bad = split_unfit(halves_max(mx));
+    }
+
+    f32x16 o[2] = {f32x16{}, f32x16{}}, ol[2] = {f32x16{}, f32x16{}};
+    float m = -INFINITY, l = 0.0f;
+    stage(0);
+    const int ntiles = static_cast<int>(ceil_div(t, 64));
+    __syncthreads();
+    for (int j = 0; j < ntiles; j++) {
+        const int cur = j & 1;
+        if (j + 1 < ntiles) load((j + 1) * 64);
+        if (live) {
+            f32x16 s[kKB], sl[kKB];
+            const f32x16 z = {};
+            const f16* a0 = sm.k[cur][0] + n * kKPitch + 8 * hh;
+            const f16* a1 = sm.k[cur][1] + n * kKPitch + 8 * hh;
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++) {
+                    const h8 kh = as_h8(ld16(a0 + 32 * kb2 * kKPitch + 16 * ks));
+                    const h8 kl = as_h8(ld16(a1 + 32 * kb2 * kKPitch + 16 * ks));
+                    s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[ks], ks ? s[kb2] : z, 0, 0, 0);
+                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[ks], ks ? sl[kb2] : z, 0, 0, 0);
+                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[ks], sl[kb2], 0, 0, 0);
+                }
+#pragma unroll
+            for (int kb2 = 0; kb2 < kKB; kb2++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[kb2][r] = fmaf(sl[kb2][r], 1.0f / 2048.0f, s[kb2][r]);
+            if ((j + 1) * 64 > t) mask_tail(s, j * 64, t, hh);
+            u32x4 ph[kKB][2], pl[kKB][2];
+            // the weights against reference ref, split, and their sum
+            auto weights = [&](float ref) {
+                float ps[2] = {0.0f, 0.0f};
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+#pragma unroll
+                    for (int w = 0; w < 8; w++) {
+                        float p[2];
+#pragma unroll
+                        for (int e = 0; e < 2; e++) {
+                            p[e] = __builtin_amdgcn_exp2f(fmaf(s[kb2][2 * w + e], c, -ref));
+                            ps[e] += p[e];
+                        }
+                        uint32_t hp = pk_f16(p[0], p[1]);
+                        asm("" : "+v"(hp));
+                        const f16x2 h = u2h2(hp);
+                        f16x2 lw;
+                        lw.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, p[0] * 2048.0f));
+                        lw.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, p[1] * 2048.0f));
+                        ph[kb2][w / 4][w % 4] = hp, pl[kb2][w / 4][w % 4] = h22u(lw);
+                    }
+                return ps[0] + ps[1];
+            };
+            // as in the f16 kernel: the tile's max only on the first tile and
+            // where a weight against the kept reference might pass 2^15
+            bool max_path = j == 0;
+            if (!max_path) {
+                const float ps = weights(m);
+                max_path = __any(!(ps <= kRowSumMax));
+                if (!max_path) l += ps;
+            }
+            if (max_path) {
+                float mx = s[0][0];
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[kb2][r]);
+                const float m_cand = fmaxf(m, halves_max(mx) * c);
+                const float m_new = m_cand > m + kLazyMax ? m_cand : m;
+                const float corr = __builtin_amdgcn_exp2f(m - m_new);
+                l = fmaf(l, corr, weights(m_new));
+                m = m_new;
+                rescale(o[0], o[1], corr);
+                rescale(ol[0], ol[1], corr);
+            }
+            const int lane16 = n & 15, c0 = n & 16;
+            const int voff = (4 * hh + lane16 / 4) * kVPitch + c0 + 4 * (lane16 % 4);
+#pragma unroll
+            for (int kb2 = 0; kb2 < kKB; kb2++)
+#pragma unroll
+                for (int kk = 0; kk < 2; kk++) {
+                    h8 a[2][2];  // [h, l][channel block]
+#pragma unroll
+                    for (int p = 0; p < 2; p++)
+#pragma unroll
+                        for (int mb = 0; mb < 2; mb++) {
+                            const f16* r0 = sm.v[cur][p] + voff + (32 * kb2 + 16 * kk) * kVPitch + 32 * mb;
+                            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)r0);
+                            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(r0 + 8 * kVPitch));
+                            const u32x2 wl = __builtin_bit_cast(u32x2, lo), wh = __builtin_bit_cast(u32x2, hi);
+                            u32x4 w;
+                            w[0] = wl[0], w[1] = wl[1], w[2] = wh[0], w[3] = wh[1];
+                            a[p][mb] = as_h8(w);
+                        }
+                    const h8 wh = as_h8(ph[kb2][kk]), wl = as_h8(pl[kb2][kk]);
+#pragma unroll
+                    for (int mb = 0; mb < 2; mb++) {
+                        o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][mb], wh, o[mb], 0, 0, 0);
+                        ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][mb], wl, ol[mb], 0, 0, 0);
+                        ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][mb], wh, ol[mb], 0, 0, 0);
+                    }
+                }
+        }
+        if (j + 1 < ntiles) stage(cur ^ 1);
+        __syncthreads();
+    }
+
+    // lanes 8 apart hold the same dims
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        float x = vm[e];
+#pragma unroll
+        for (int mask = 8; mask < 64; mask *= 2) x = fmaxf(x, xor_lanes(x, mask));
+        if (lane < 8) atomicMax(&vmax[pd + e], f2u(x));
+    }
+    if (bad) unfit = 1;
+    __syncthreads();
+    if (tid < 64 && split_unfit(u2f(vmax[tid]))) unfit = 1;
+    __syncthreads();
+    float lsum;
+    if (unfit == 0) {
+        lsum = halves_sum(l);
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[mb][r] = fmaf(ol[mb][r], 1.0f / 2048.0f, o[mb][r]);
+    } else {
+        lsum = flash_f32_body<W>(o, smem.f32, q + base, kb, vb, qi, t, c, tid, n, hh);
+    }
     if (qi >= t) return;  // after the last barrier
     float* orow = token_major
                       ? out + ((static_cast<int64_t>(sh / heads) * t + qi) * heads + sh % heads) * kD
                       : out + base + static_cast<int64_t>(qi) * kD;
+    const float inv = 1.0f / lsum;
 #pragma unroll
-    for (int db = 0; db < 2; db++)
+    for (int mb = 0; mb < 2; mb++)
 #pragma unroll
         for (int r4 = 0; r4 < 4; r4++) {
             u32x4 w;
 #pragma unroll
-            for (int e = 0; e < 4; e++) w[e] = f2u(o[db][4 * r4 + e] / l);
-            st16(orow + 32 * db + 8 * r4 + 4 * hh, w);
+            for (int e = 0; e < 4; e++) w[e] = f2u(o[mb][4 * r4 + e] * inv);
+            st16(orow + 32 * mb + 8 * r4 + 4 * hh, w);
         }
 }
 
@@ -754,8 +1019,6 @@ constexpr int kHD = 128;          // head dim
 constexpr int kHWaves = 4;
 constexpr int kHP = kHD / 16;     // 16-dim pieces
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float xor_lanes(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
 __global__ __launch_bounds__(64 * kHWaves) void attention_d128_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -873,6 +1136,19 @@ hs_status check_attention(const char* op, hs_dtype dt, const void* q, const void
     return HS_OK;
 }
 
+// False where the grid, or the byte offsets within a (frame, head), would not fit.
+template <int W>
+bool launch_split(hipStream_t st, const void* q, const void* k, const void* v, void* out, int sh, int h, int t,
+                  float scale, int token_major) {
+    const int qtiles = static_cast<int>(ceil_div(t, 32 * W));
+    const int64_t blocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * qtiles;
+    if (blocks >= (int64_t{1} << 31) / (64 * W) || t > (1 << 22)) return false;
+    flash_split_kernel<W><<<dim3(static_cast<uint32_t>(blocks)), dim3(64 * W), 0, st>>>(
+        static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+        static_cast<float*>(out), sh, h, t, qtiles, scale * 1.4426950408889634f, token_major);
+    return true;
+}
+
 hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const void* k,
                            const void* v, void* out, int s, int h, int t, int d, int token_major) {
     const int sh = s * h;
@@ -906,14 +1182,13 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
         }
     }
     if (dt == HS_F32 && d == kD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
-        const int qtiles = static_cast<int>(ceil_div(t, kF32Q));
-        const int64_t blocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * qtiles;
-        if (blocks < (int64_t{1} << 31) / kF32Threads) {
-            flash_f32_kernel<<<dim3(static_cast<uint32_t>(blocks)), dim3(kF32Threads), 0, st>>>(
-                static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
-                static_cast<float*>(out), sh, h, t, qtiles, scale * 1.4426950408889634f, token_major);
+        // 128 queries per workgroup while one per CU holds them all (16
+        // heads of 1374 tokens: 55 us against 63), 256 beyond (32 heads: 108
+        // against 67).
+        const bool few = static_cast<int64_t>(sh) * ceil_div(t, 128) <= num_cus();
+        if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
+                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
             return check_launch("attention");
-        }
     }
     if (dt == HS_F32 && d == kHD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
         const int qtiles = static_cast<int>(ceil_div(t, 16));

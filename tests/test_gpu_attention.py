@@ -402,3 +402,83 @@ def test_attention_global_blocks_sampled(ctx):
     vc = v[:, :, :1].expand(s, h, t, 64).contiguous()
     out = back(ctx.attention(q, k, vc)).astype(np.float32)
     f16_close(out, np.broadcast_to(back(vc).astype(np.float32), out.shape), "constant V")
+
+
+def _rel(got, want):
+    return (np.linalg.norm(got - want) / np.linalg.norm(want)).item()
+
+
+@pytest.mark.parametrize("s,h,t", [(1, 2, 1), (1, 3, 31), (1, 2, 64), (2, 2, 65), (1, 2, 127), (1, 1, 129),
+                                   (3, 5, 200), (1, 260, 40), (1, 300, 257), (2, 130, 300)])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_attention_f32_split_edges(ctx, s, h, t, spread):
+    """flash_split_kernel at the edges of its key tiles (64), query tiles (128
+    and, past 256 of those, 256), and wave-dead tails: f32 precision (2^-24
+    per rounding; the scores' spread of up to ~30 log2 units enters the
+    weights' relative error)."""
+    rng = np.random.default_rng(t)
+    q, k, v = (rng.standard_normal((s, h, t, 64)).astype(np.float32) for _ in range(3))
+    q *= np.float32(spread)
+    want = naive64(q, k, v)
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    assert _rel(got, want) < 1.2e-6
+    assert np.abs(got - want).max() < 1e-5 * max(1.0, spread)
+    merged = back(ctx.attention_merged(dev(q), dev(k), dev(v)))
+    assert_bit_exact(merged.reshape(s, t, h, 64).transpose(0, 2, 1, 3).copy(), got, "merged split")
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v", "vcol", "qrow", "krow"])
+@pytest.mark.parametrize("scale", [1e-8, 1e6])
+def test_attention_f32_split_ranges(ctx, what, scale):
+    """Values outside the f16 pair's range (a whole operand, one V column, one
+    query or key row) take the f32 instructions: the same relative error."""
+    rng = np.random.default_rng(4)
+    q, k, v = (rng.standard_normal((1, 3, 300, 64)).astype(np.float32) for _ in range(3))
+    if what == "q":
+        q *= np.float32(scale)
+        k *= np.float32(1 / scale)
+    elif what == "k":
+        k *= np.float32(scale)
+        q *= np.float32(1 / scale)
+    elif what == "v":
+        v *= np.float32(scale)
+    elif what == "vcol":
+        v[..., 17] *= np.float32(scale)
+    elif what == "qrow":
+        q[:, :, 150] *= np.float32(min(scale, 1e5))
+    else:
+        k[:, :, 299] *= np.float32(min(scale, 1e5))
+    want = naive64(q, k, v)
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    ok = np.isfinite(want)
+    assert ok.all() and np.isfinite(got).all()
+    if what in ("qrow", "krow") and scale > 1:
+        # scores of 1e5: their rounding alone moves weights by 1e5 x 2^-24
+        assert np.abs(got - want).max() < 0.1
+        rows = np.ones(300, bool)
+        if what == "qrow":
+            rows[150] = False
+            assert _rel(got[:, :, rows], want[:, :, rows]) < 1.2e-6
+    else:
+        err = np.abs(got - want).max(axis=(0, 1, 2)) / np.abs(want).max(axis=(0, 1, 2))
+        assert err.max() < 4e-6
+
+
+def test_attention_f32_split_special_values(ctx):
+    """Zero rows stay on the split path and exact; a NaN key or an infinite
+    value reaches what the float64 softmax gives it to."""
+    rng = np.random.default_rng(8)
+    q, k, v = (rng.standard_normal((1, 2, 200, 64)).astype(np.float32) for _ in range(3))
+    q[0, 0, 3] = 0
+    k[0, 0] = 0  # equal scores: the mean of V
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    assert np.abs(got[0, 0] - v[0, 0].astype(np.float64).mean(0)).max() < 1e-6
+    assert _rel(got, naive64(q, k, v)) < 1.2e-6
+    v[0, 1, 7, 5] = np.inf
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    assert np.isposinf(got[0, 1, :, 5]).all()
+    keep = np.arange(64) != 5
+    assert np.isfinite(got[0, 1][:, keep]).all() and np.isfinite(got[0, 0]).all()
+    k[0, 1, 9, 2] = np.nan
+    got = back(ctx.attention(dev(q), dev(k), dev(v)))
+    assert np.isnan(got[0, 1]).all() and np.isfinite(got[0, 0]).all()
