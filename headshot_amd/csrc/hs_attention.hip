@@ -725,8 +725,9 @@ __device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm
 //
 // Bounds: matrix and vector issue, 48 MFMAs and ~350 vector instructions per
 // wave and tile, which overlap little: two waves per SIMD in step. 16 heads of
-// 1374 tokens, us on the f32 matrix instructions and here: 1 sequence 111, 55;
-// 2, 202, 67; 8, 567, 215 (290 TFLOP/s). Relative error against 64 bits 8.6e-7,
+// 1374 tokens, us on the f32 matrix instructions and here: 1 sequence 111, 51;
+// 2, 197, 60; 8, 567, 210 (295 TFLOP/s); with operands read at their use, as the
+// compiler orders them, 55, 67, 215. Relative error against 64 bits 8.6e-7,
 // 3.8e-7.
 constexpr float kSplitMax = 65504.0f, kSplitMin = 0x1p-13f;
 
@@ -867,16 +868,34 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
             const f32x16 z = {};
             const f16* a0 = sm.k[cur][0] + n * kKPitch + 8 * hh;
             const f16* a1 = sm.k[cur][1] + n * kKPitch + 8 * hh;
+            // h operands are read a 16-dim slice ahead, l operands under the
+            // slice's h products
+            h8 kh[2][kKB], kl[kKB];
+            auto read_k = [&](h8(&dst)[kKB], const f16* src, int ks) {
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++)
+                for (int kb2 = 0; kb2 < kKB; kb2++) dst[kb2] = as_h8(ld16(src + 32 * kb2 * kKPitch + 16 * ks));
+            };
+            read_k(kh[0], a0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, kKB, 0);  // LDS reads
 #pragma unroll
-                for (int kb2 = 0; kb2 < kKB; kb2++) {
-                    const h8 kh = as_h8(ld16(a0 + 32 * kb2 * kKPitch + 16 * ks));
-                    const h8 kl = as_h8(ld16(a1 + 32 * kb2 * kKPitch + 16 * ks));
-                    s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[ks], ks ? s[kb2] : z, 0, 0, 0);
-                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[ks], ks ? sl[kb2] : z, 0, 0, 0);
-                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[ks], sl[kb2], 0, 0, 0);
-                }
+            for (int ks = 0; ks < 4; ks++) {
+                read_k(kl, a1, ks);
+                if (ks < 3) read_k(kh[(ks + 1) & 1], a0, ks + 1);
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+                    s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks & 1][kb2], qh[ks], ks ? s[kb2] : z, 0, 0, 0);
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks & 1][kb2], ql[ks], ks ? sl[kb2] : z, 0, 0, 0);
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[kb2], qh[ks], sl[kb2], 0, 0, 0);
+                if (ks < 3)
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kKB, 0);
+                else
+                    __builtin_amdgcn_sched_group_barrier(0x100, kKB, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 3 * kKB, 0);  // MFMAs
+            }
 #pragma unroll
             for (int kb2 = 0; kb2 < kKB; kb2++)
 #pragma unroll
@@ -930,31 +949,43 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
             }
             const int lane16 = n & 15, c0 = n & 16;
             const int voff = (4 * hh + lane16 / 4) * kVPitch + c0 + 4 * (lane16 % 4);
+            // 16 keys at a time, V's h operands read a group ahead, its l
+            // operands under the group's h products
+            h8 vh[2][2], vl[2];  // [channel block]
+            auto read_v = [&](h8(&dst)[2], const f16* src, int g) {
 #pragma unroll
-            for (int kb2 = 0; kb2 < kKB; kb2++)
-#pragma unroll
-                for (int kk = 0; kk < 2; kk++) {
-                    h8 a[2][2];  // [h, l][channel block]
-#pragma unroll
-                    for (int p = 0; p < 2; p++)
-#pragma unroll
-                        for (int mb = 0; mb < 2; mb++) {
-                            const f16* r0 = sm.v[cur][p] + voff + (32 * kb2 + 16 * kk) * kVPitch + 32 * mb;
-                            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)r0);
-                            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(r0 + 8 * kVPitch));
-                            const u32x2 wl = __builtin_bit_cast(u32x2, lo), wh = __builtin_bit_cast(u32x2, hi);
-                            u32x4 w;
-                            w[0] = wl[0], w[1] = wl[1], w[2] = wh[0], w[3] = wh[1];
-                            a[p][mb] = as_h8(w);
-                        }
-                    const h8 wh = as_h8(ph[kb2][kk]), wl = as_h8(pl[kb2][kk]);
-#pragma unroll
-                    for (int mb = 0; mb < 2; mb++) {
-                        o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][mb], wh, o[mb], 0, 0, 0);
-                        ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][mb], wl, ol[mb], 0, 0, 0);
-                        ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][mb], wh, ol[mb], 0, 0, 0);
-                    }
+                for (int mb = 0; mb < 2; mb++) {
+                    const f16* r0 = src + voff + 16 * g * kVPitch + 32 * mb;
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)r0);
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(r0 + 8 * kVPitch));
+                    const u32x2 wl = __builtin_bit_cast(u32x2, lo), wh = __builtin_bit_cast(u32x2, hi);
+                    u32x4 w;
+                    w[0] = wl[0], w[1] = wl[1], w[2] = wh[0], w[3] = wh[1];
+                    dst[mb] = as_h8(w);
                 }
+            };
+            read_v(vh[0], sm.v[cur][0], 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+            for (int g = 0; g < 2 * kKB; g++) {
+                read_v(vl, sm.v[cur][1], g);
+                if (g + 1 < 2 * kKB) read_v(vh[(g + 1) & 1], sm.v[cur][0], g + 1);
+                const h8 wh = as_h8(ph[g / 2][g % 2]), wl = as_h8(pl[g / 2][g % 2]);
+#pragma unroll
+                for (int mb = 0; mb < 2; mb++)
+                    o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[g & 1][mb], wh, o[mb], 0, 0, 0);
+#pragma unroll
+                for (int mb = 0; mb < 2; mb++)
+                    ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[g & 1][mb], wl, ol[mb], 0, 0, 0);
+#pragma unroll
+                for (int mb = 0; mb < 2; mb++)
+                    ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[mb], wh, ol[mb], 0, 0, 0);
+                if (g + 1 < 2 * kKB)
+                    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+                else
+                    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);  // MFMAs
+            }
         }
         if (j + 1 < ntiles) stage(cur ^ 1);
         __syncthreads();
@@ -1183,8 +1214,8 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
     }
     if (dt == HS_F32 && d == kD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
         // 128 queries per workgroup while one per CU holds them all (16
-        // heads of 1374 tokens: 55 us against 63), 256 beyond (32 heads: 108
-        // against 67).
+        // heads of 1374 tokens: 51 us against 60), 256 beyond (32 heads: 108
+        // against 64).
         const bool few = static_cast<int64_t>(sh) * ceil_div(t, 128) <= num_cus();
         if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
                 : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
