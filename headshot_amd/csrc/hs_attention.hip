@@ -49,17 +49,7 @@ constexpr int kXcds = 8;
 // ---------------------------------------------------------------------------
 // flash attention, f16, D = 64
 
-#ifndef HS_ATT_WAVES
-#define HS_ATT_WAVES 8  // waves (32 queries each) per workgroup
-#endif
 constexpr int kD = 64;
-constexpr int kWaves = HS_ATT_WAVES;
-constexpr int kThreads = 64 * kWaves;
-#ifndef HS_ATT_QB
-#define HS_ATT_QB 1  // 32-query blocks per wave
-#endif
-constexpr int kQB = HS_ATT_QB;
-constexpr int kBM = 32 * kQB * kWaves;  // queries per workgroup
 #ifndef HS_ATT_BN
 #define HS_ATT_BN 64  // keys per tile (a multiple of 32)
 #endif
@@ -87,13 +77,34 @@ constexpr int kKPitch = kD + HS_ATT_KPAD;
 constexpr int kVPitch = kD + HS_ATT_VPAD;
 static_assert(HS_ATT_KPAD % 8 == 0 && HS_ATT_VPAD % 8 == 0, "rows must stay 16-byte aligned");
 constexpr int kChunks = kBN * kD / 8;  // 16-byte chunks per K (or V) tile
-constexpr int kPer = (kChunks + kThreads - 1) / kThreads;
-static_assert(kChunks % kThreads == 0 || kThreads % kChunks == 0, "tile split");
 
-struct FlashSmem {
-    f16 k[2][kBN * kKPitch];
-    f16 v[2][kBN * kVPitch];
+// A workgroup's shape: KS groups of QW waves; a group's waves take 32 queries
+// each, every group the same QW x 32 queries over its own share of the key
+// tiles, staged in two buffers of its own.
+template <int QW, int KS>
+struct FlashShape {
+    static constexpr int kQW = QW, kKS = KS;
+    static constexpr int kThreads = 64 * QW * KS;
+    static constexpr int kBM = 32 * QW;                    // queries per workgroup
+    static constexpr int kPer = kChunks / (64 * QW);       // 16-byte chunks per thread of a tile
+    static_assert(kPer * 64 * QW == kChunks, "tile split");
+    struct Smem {
+        f16 k[KS][2][kBN * kKPitch];
+        f16 v[KS][2][kBN * kVPitch];
+    };
+    // half of the groups' outputs (32 floats a lane) and (m, l) at a time
+    struct Merge {
+        float o[KS > 1 ? KS / 2 * QW : 1][32][64];
+        float ml[KS > 1 ? KS / 2 * QW : 1][2][64];
+    };
+    union Lds {
+        Smem tiles;
+        Merge merge;
+    };
 };
+using FlashPlain = FlashShape<8, 1>;  // two workgroups per CU
+using FlashTwo = FlashShape<8, 2>;    // one per CU
+using FlashHalf = FlashShape<4, 2>;   // one per CU
 
 __device__ __forceinline__ h8 as_h8(u32x4 v) { return __builtin_bit_cast(h8, v); }
 
@@ -104,40 +115,39 @@ __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
 }
 
 // One thread's share of a 64-row K or V tile: 16-byte chunk c = tid + i *
-// kThreads is row c / 8, channels (c % 8) * 8 .. + 8.
+// threads (of its group) is row c / 8, channels (c % 8) * 8 .. + 8.
+template <int PER>
 struct TileChunks {
-    u32x4 c[kPer];
+    u32x4 c[PER];
 };
 
 // Loads rows [key0, key0 + 64) of one (frame, head); rows past the
 // sequence end are clamped to the last row (their scores are masked).
-__device__ __forceinline__ void load_rows(TileChunks& r, const f16* src, int key0, int t, int tid) {
+template <int PER>
+__device__ __forceinline__ void load_rows(TileChunks<PER>& r, const f16* src, int key0, int t, int tid) {
 #pragma unroll
-    for (int i = 0; i < kPer; i++) {
-        const int c = tid + i * kThreads;
-        if (kChunks % kThreads != 0 && c >= kChunks) break;
+    for (int i = 0; i < PER; i++) {
+        const int c = tid + i * (kChunks / PER);
         const int row = min(key0 + c / 8, t - 1);
         r.c[i] = ld16(src + static_cast<int64_t>(row) * kD + (c % 8) * 8);
     }
 }
 
 // Row-major into LDS with a padded pitch.
-template <int kPitch>
-__device__ __forceinline__ void store_rows(const TileChunks& r, f16* buf, int tid) {
+template <int kPitch, int PER>
+__device__ __forceinline__ void store_rows(const TileChunks<PER>& r, f16* buf, int tid) {
 #pragma unroll
-    for (int i = 0; i < kPer; i++) {
-        const int c = tid + i * kThreads;
-        if (kChunks % kThreads != 0 && c >= kChunks) break;
+    for (int i = 0; i < PER; i++) {
+        const int c = tid + i * (kChunks / PER);
         st16(&buf[(c / 8) * kPitch + (c % 8) * 8], r.c[i]);
     }
 }
 
-// S^T (keys x queries) of one tile for the wave's query blocks: s[b][kb]
-// holds keys [32 kb, 32 kb + 32) of the tile; register r of lane (n, hh) is
-// key 8 (r / 4) + 4 hh + r % 4 of its block, query n of query block b.
-// Each K operand read from LDS feeds the MFMAs of every query block.
-__device__ __forceinline__ void qk_scores(f32x16 (&s)[kQB][kKB], const f16* kbuf,
-                                          const h8 (&qa)[kQB][4], int n, int hh) {
+// S^T (keys x queries) of one tile for the wave's queries: s[kb] holds keys
+// [32 kb, 32 kb + 32) of the tile; register r of lane (n, hh) is key 8 (r /
+// 4) + 4 hh + r % 4 of its block, query n.
+__device__ __forceinline__ void qk_scores(f32x16 (&s)[kKB], const f16* kbuf, const h8 (&qa)[4], int n,
+                                          int hh) {
     const f16* a0 = kbuf + n * kKPitch + 8 * hh;
     const f32x16 z = {};
 #pragma unroll
@@ -145,9 +155,7 @@ __device__ __forceinline__ void qk_scores(f32x16 (&s)[kQB][kKB], const f16* kbuf
 #pragma unroll
         for (int kb = 0; kb < kKB; kb++) {
             const h8 kv = as_h8(ld16(a0 + 32 * kb * kKPitch + 16 * ks));
-#pragma unroll
-            for (int b = 0; b < kQB; b++)
-                s[b][kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qa[b][ks], ks ? s[b][kb] : z, 0, 0, 0);
+            s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qa[ks], ks ? s[kb] : z, 0, 0, 0);
         }
     }
 }
@@ -259,8 +267,8 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // channel c0 + i of 4 keys; two such reads give the 8 keys of one operand,
 // in the order the score accumulator holds P^T (keys 16 kk + 4 hh + j and
 // 16 kk + 8 + 4 hh + j of a 32-key block).
-__device__ __forceinline__ void pv_update(f32x16 (&o)[kQB][2], const f16* vbuf,
-                                          const u32x4 (&p)[kQB][kKB][2], int n, int hh) {
+__device__ __forceinline__ void pv_update(f32x16 (&o)[2], const f16* vbuf, const u32x4 (&p)[kKB][2], int n,
+                                          int hh) {
     const int lane16 = n & 15;  // lane within its 16-lane group
     const int c0 = n & 16;      // channel base of the group within a 32-channel block
     const f16* base = vbuf + (4 * hh + lane16 / 4) * kVPitch + c0 + 4 * (lane16 % 4);
@@ -279,11 +287,8 @@ __device__ __forceinline__ void pv_update(f32x16 (&o)[kQB][2], const f16* vbuf,
                 w[0] = wl[0], w[1] = wl[1], w[2] = wh[0], w[3] = wh[1];
                 a[mb] = as_h8(w);
             }
-#pragma unroll
-            for (int b = 0; b < kQB; b++) {
-                o[b][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_h8(p[b][kb2][kk]), o[b][0], 0, 0, 0);
-                o[b][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_h8(p[b][kb2][kk]), o[b][1], 0, 0, 0);
-            }
+            o[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], as_h8(p[kb2][kk]), o[0], 0, 0, 0);
+            o[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], as_h8(p[kb2][kk]), o[1], 0, 0, 0);
         }
 }
 
@@ -317,114 +322,135 @@ __device__ __forceinline__ void store_out(const f32x16& o0, const f32x16& o1, fl
 // b % kXcds, query tile qt0 + (b / kXcds) % QT.
 // TAIL: the launch of the partial last query tiles (qt0 = their index),
 // whose waves with every query past T only stage K and V.
-template <bool TAIL>
-__global__ __launch_bounds__(kThreads) void flash_f16_kernel(
+//
+// One workgroup per CU leaves two waves per SIMD, and a tile then takes nearly
+// as long as with four (1.36 us against 1.58). Where the grid is that small a
+// workgroup holds KS groups of waves instead, each over its own contiguous
+// share of the key tiles, whose (O, m, l) are merged through LDS in halves at
+// the end.
+template <bool TAIL, typename P>
+__global__ __launch_bounds__(P::kThreads) void flash_f16_kernel(
     const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v,
     f16* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c,
     int token_major, int qt0) {
-    __shared__ FlashSmem sm;
+    constexpr int kBM = P::kBM, kKS = P::kKS;
+    __shared__ __align__(16) typename P::Lds lds;
+    typename P::Smem& sm = lds.tiles;
     const int b = blockIdx.x;
     const int slot = b / kXcds;
     const int sh = (slot / qtiles) * kXcds + b % kXcds;
     if (sh >= sh_count) return;  // workgroup-uniform, before any barrier
     const int qt = qt0 + slot % qtiles;
-    const int tid = threadIdx.x;
     const int lane = lane_id();
-    const int wave = tid >> 6;
+    const int kg = kKS == 1 ? 0 : wave_in_block() / P::kQW;  // the wave's key group
+    const int wave = static_cast<int>(threadIdx.x >> 6) - kg * P::kQW;
+    const int tid = static_cast<int>(threadIdx.x) - kg * (64 * P::kQW);  // within the group
     const int n = lane & 31, hh = lane >> 5;
     const int64_t base = static_cast<int64_t>(sh) * t * kD;
     const f16* qb = q + base;
     const f16* kb = k + base;
     const f16* vb = v + base;
 
-    // Q^T as the B operand: lane (n, hh) of block b holds
-    // q[qi_b][16 ks + 8 hh .. + 8), qi_b = query n of the wave's block b.
-    int qi[kQB];
-    h8 qa[kQB][4];
+    // Q^T as the B operand: lane (n, hh) holds q[qi][16 ks + 8 hh .. + 8)
+    const int qi = qt * kBM + wave * 32 + n;
+    h8 qa[4];
+    const int qc = min(qi, t - 1);
 #pragma unroll
-    for (int b = 0; b < kQB; b++) {
-        qi[b] = qt * kBM + (wave * kQB + b) * 32 + n;
-        const int qc = min(qi[b], t - 1);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++)
-            qa[b][ks] = as_h8(ld16(qb + static_cast<int64_t>(qc) * kD + 16 * ks + 8 * hh));
-    }
+    for (int ks = 0; ks < 4; ks++) qa[ks] = as_h8(ld16(qb + static_cast<int64_t>(qc) * kD + 16 * ks + 8 * hh));
     // Q must have arrived before the tile loop: otherwise the compiler sinks
     // these loads into the loop's preheader and, unable to tell them from
     // the prefetch loads issued inside the loop, waits for the prefetch at
     // every tile's first MFMA.
 #pragma unroll
-    for (int b = 0; b < kQB; b++)
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) asm volatile("" ::"v"(qa[b][ks]));
+    for (int ks = 0; ks < 4; ks++) asm volatile("" ::"v"(qa[ks]));
 
-    f32x16 o[kQB][2];
-    float m[kQB], l[kQB];
-#pragma unroll
-    for (int b = 0; b < kQB; b++) {
-        o[b][0] = f32x16{}, o[b][1] = f32x16{};
-        m[b] = -INFINITY, l[b] = 0.0f;
-    }
+    f32x16 o[2] = {f32x16{}, f32x16{}};
+    float m = -INFINITY, l = 0.0f;
     const int ntiles = static_cast<int>(ceil_div(t, kBN));
+    // the group's tiles [j0, j1), `steps` for every group (the last ones may
+    // have fewer, or none)
+    const int steps = kKS == 1 ? ntiles : (ntiles + kKS - 1) / kKS;
+    const int j0 = kg * steps, j1 = min(j0 + steps, ntiles);
 
     // Double-buffered tiles: tile j + 1 is loaded into registers while tile
     // j computes from LDS, then written to the other buffer (last read in
     // iteration j - 1, which the barrier at its end closed).
-    TileChunks pk, pv;
-    load_rows(pk, kb, 0, t, tid);
-    load_rows(pv, vb, 0, t, tid);
-    store_rows<kKPitch>(pk, sm.k[0], tid);
-    store_rows<kVPitch>(pv, sm.v[0], tid);
+    TileChunks<P::kPer> pk, pv;
+    load_rows(pk, kb, j0 * kBN, t, tid);
+    load_rows(pv, vb, j0 * kBN, t, tid);
+    store_rows<kKPitch>(pk, sm.k[kg][0], tid);
+    store_rows<kVPitch>(pv, sm.v[kg][0], tid);
     __syncthreads();
-    for (int j = 0; j < ntiles; j++) {
-        const int cur = j & 1;
-        if (j + 1 < ntiles) {
+    for (int i = 0; i < steps; i++) {
+        const int j = j0 + i;
+        const int cur = i & 1;
+        if (i + 1 < steps) {
             load_rows(pk, kb, (j + 1) * kBN, t, tid);
             load_rows(pv, vb, (j + 1) * kBN, t, tid);
         }
-        if (!TAIL || qt * kBM + wave * kQB * 32 < t) {
-        f32x16 sc[kQB][kKB];
-        qk_scores(sc, sm.k[cur], qa, n, hh);
-        u32x4 p[kQB][kKB][2];
-#pragma unroll
-        for (int b = 0; b < kQB; b++) {
-            if ((j + 1) * kBN > t) mask_tail(sc[b], j * kBN, t, hh);
+        if ((!TAIL || qt * kBM + wave * 32 < t) && (kKS == 1 || j < j1)) {
+            f32x16 sc[kKB];
+            qk_scores(sc, sm.k[kg][cur], qa, n, hh);
+            u32x4 p[kKB][2];
+            if ((j + 1) * kBN > t) mask_tail(sc, j * kBN, t, hh);
             // After the first tile, weights against the kept reference; the
             // max path only when some lane's sum says a weight may exceed
             // 2^15 (a row sum above 2^15 means a weight above 2^10, more
             // than kLazyMax over m, so that path then moves m).
-            bool max_path = j == 0;
+            bool max_path = i == 0;
             if (!max_path) {
-                const float ps = weights_tile(sc[b], c, m[b], p[b]);
+                const float ps = weights_tile(sc, c, m, p);
                 max_path = __any(!(ps <= kRowSumMax));
-                if (!max_path) l[b] += ps;
+                if (!max_path) l += ps;
             }
             if (max_path) {
-                const float corr = softmax_tile(sc[b], c, m[b], l[b], p[b]);
-                rescale(o[b][0], o[b][1], corr);
+                const float corr = softmax_tile(sc, c, m, l, p);
+                rescale(o[0], o[1], corr);
             }
+            pv_update(o, sm.v[kg][cur], p, n, hh);
         }
-        pv_update(o, sm.v[cur], p, n, hh);
-        }
-        if (j + 1 < ntiles) {
-            store_rows<kKPitch>(pk, sm.k[cur ^ 1], tid);
-            store_rows<kVPitch>(pv, sm.v[cur ^ 1], tid);
+        if (i + 1 < steps) {
+            store_rows<kKPitch>(pk, sm.k[kg][cur ^ 1], tid);
+            store_rows<kVPitch>(pv, sm.v[kg][cur ^ 1], tid);
         }
         __syncthreads();
     }
 
+    // Merge the groups, upper half into lower half (a group without tiles
+    // has m = -inf, l = 0 and O = 0; group 0 has tiles). The tiles' LDS is free.
 #pragma unroll
-    for (int b = 0; b < kQB; b++) {
-        if (qi[b] >= t) continue;
-        f16* orow;
-        if (token_major) {
-            const int s = sh / heads, h = sh - s * heads;
-            orow = out + ((static_cast<int64_t>(s) * t + qi[b]) * heads + h) * kD;
-        } else {
-            orow = out + base + static_cast<int64_t>(qi[b]) * kD;
+    for (int half = kKS / 2; half >= 1; half /= 2) {
+        if (kg >= half && kg < 2 * half) {
+            const int w = (kg - half) * P::kQW + wave;
+#pragma unroll
+            for (int r = 0; r < 16; r++) lds.merge.o[w][r][lane] = o[0][r], lds.merge.o[w][16 + r][lane] = o[1][r];
+            lds.merge.ml[w][0][lane] = m, lds.merge.ml[w][1][lane] = l;
         }
-        store_out(o[b][0], o[b][1], l[b], orow, hh);
+        __syncthreads();
+        if (kg < half) {
+            const int w = kg * P::kQW + wave;
+            const float m1 = lds.merge.ml[w][0][lane], l1 = lds.merge.ml[w][1][lane];
+            const float mm = fmaxf(m, m1);
+            const float f0 = __builtin_amdgcn_exp2f(m - mm), f1 = __builtin_amdgcn_exp2f(m1 - mm);
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                o[0][r] = fmaf(o[0][r], f0, lds.merge.o[w][r][lane] * f1);
+                o[1][r] = fmaf(o[1][r], f0, lds.merge.o[w][16 + r][lane] * f1);
+            }
+            l = fmaf(l, f0, l1 * f1);
+            m = mm;
+        }
+        if (half > 1) __syncthreads();
     }
+    if (kg > 0 || qi >= t) return;
+    f16* orow;
+    if (token_major) {
+        const int s = sh / heads, h = sh - s * heads;
+        orow = out + ((static_cast<int64_t>(s) * t + qi) * heads + h) * kD;
+    } else {
+        orow = out + base + static_cast<int64_t>(qi) * kD;
+    }
+    store_out(o[0], o[1], l, orow, hh);
 }
 
 // ---------------------------------------------------------------------------
@@ -1187,28 +1213,47 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
     const bool flash_ok = dt == HS_F16 && d == kD && aligned16(q) && aligned16(k) && aligned16(v) &&
                           (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
     if (flash_ok) {
-        const int qtiles = static_cast<int>(ceil_div(t, kBM));
-        const int64_t blocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * qtiles;
-        if (blocks < (int64_t{1} << 31) / kThreads) {
-            const float c = scale * 1.4426950408889634f;  // scores enter exp2
+        const float c = scale * 1.4426950408889634f;  // scores enter exp2
+        auto grid = [&](int bm) { return static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * ceil_div(t, bm); };
+        if (grid(FlashPlain::kBM) < (int64_t{1} << 31) / FlashTwo::kThreads) {
+            const f16 *fq = static_cast<const f16*>(q), *fk = static_cast<const f16*>(k);
+            const f16* fv = static_cast<const f16*>(v);
+            f16* fo = static_cast<f16*>(out);
+            const int qtiles = static_cast<int>(ceil_div(t, FlashPlain::kBM));
+            const int64_t cus = num_cus();
+            // Key groups while one workgroup per CU holds the grid, with 128
+            // queries where they do, else 256. 16 heads, us with FlashPlain
+            // and here: 408 tokens 12.9, 9.4; 782 19.6, 13.2; 1386 29.3, 18.9;
+            // 2 x 1386 (192 workgroups of 256) 30.2, 27.9; 2772 53, 47. Two 4-wave
+            // groups with two workgroups per CU: 2 x 1386 35.6.
+            if (t > kBN && static_cast<int64_t>(sh) * ceil_div(t, FlashHalf::kBM) <= cus) {
+                flash_f16_kernel<false, FlashHalf><<<dim3(static_cast<uint32_t>(grid(FlashHalf::kBM))),
+                                                     dim3(FlashHalf::kThreads), 0, st>>>(
+                    fq, fk, fv, fo, sh, h, t, static_cast<int>(ceil_div(t, FlashHalf::kBM)), c, token_major, 0);
+                return check_launch("attention");
+            }
+            if (t > kBN && static_cast<int64_t>(sh) * qtiles <= cus) {
+                flash_f16_kernel<false, FlashTwo><<<dim3(static_cast<uint32_t>(grid(FlashTwo::kBM))),
+                                                    dim3(FlashTwo::kThreads), 0, st>>>(
+                    fq, fk, fv, fo, sh, h, t, qtiles, c, token_major, 0);
+                return check_launch("attention");
+            }
             // A partial last query tile runs as a launch of its own when
             // there are enough of them to fill the chip (two workgroups per
             // CU, e.g. 32 frames x 16 heads of 1374 tokens): its waves past
             // T then leave their SIMDs to the live ones. With fewer (one
             // long sequence) they stay in the main launch, where they
             // overlap the other tiles.
-            const bool split = t % kBM != 0 && qtiles > 1 && sh >= 2 * num_cus();
+            const bool split = t % FlashPlain::kBM != 0 && qtiles > 1 && sh >= 2 * cus;
             const int main_tiles = split ? qtiles - 1 : qtiles;
-            const int64_t mblocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * main_tiles;
-            flash_f16_kernel<false><<<dim3(static_cast<uint32_t>(mblocks)), dim3(kThreads), 0, st>>>(
-                static_cast<const f16*>(q), static_cast<const f16*>(k), static_cast<const f16*>(v),
-                static_cast<f16*>(out), sh, h, t, main_tiles, c, token_major, 0);
-            if (split) {
-                const int64_t tblocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds);
-                flash_f16_kernel<true><<<dim3(static_cast<uint32_t>(tblocks)), dim3(kThreads), 0, st>>>(
-                    static_cast<const f16*>(q), static_cast<const f16*>(k), static_cast<const f16*>(v),
-                    static_cast<f16*>(out), sh, h, t, 1, c, token_major, qtiles - 1);
-            }
+            const int64_t seqs = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds);
+            flash_f16_kernel<false, FlashPlain><<<dim3(static_cast<uint32_t>(seqs * main_tiles)),
+                                                  dim3(FlashPlain::kThreads), 0, st>>>(
+                fq, fk, fv, fo, sh, h, t, main_tiles, c, token_major, 0);
+            if (split)
+                flash_f16_kernel<true, FlashPlain><<<dim3(static_cast<uint32_t>(seqs)),
+                                                     dim3(FlashPlain::kThreads), 0, st>>>(
+                    fq, fk, fv, fo, sh, h, t, 1, c, token_major, qtiles - 1);
             return check_launch("attention");
         }
     }
