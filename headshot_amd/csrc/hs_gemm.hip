@@ -192,19 +192,11 @@ constexpr int kLnParamLoads = 4;            // 16-byte loads of ln_w / ln_b per 
 #ifndef HS_GEMM_LN_SLICES
 #define HS_GEMM_LN_SLICES 2  // k slices of a step over which the next stage is normalised
 #endif
-#ifndef HS_GEMM_LN_VALU
-#define HS_GEMM_LN_VALU 8  // vector instructions scheduled after each of those slices' MFMAs
-#endif
 #ifndef HS_GEMM_LN_FIRST
 #define HS_GEMM_LN_FIRST 1  // the first of those slices (the pieces are read at slice 0)
 #endif
-#ifndef HS_GEMM_LN_HINTS
-#define HS_GEMM_LN_HINTS 1  // interleave by scheduling groups (0: the compiler's order)
-#endif
 constexpr int kLnSlices = HS_GEMM_LN_SLICES;
 constexpr int kLnFirst = HS_GEMM_LN_FIRST;
-constexpr bool kLnHints = HS_GEMM_LN_HINTS != 0;
-constexpr int kLnValuPerMfma = HS_GEMM_LN_VALU;
 static_assert(kLnRows % kLnSlices == 0 && kLnFirst >= 0 && kLnFirst + kLnSlices < kBK / 16,
               "LayerNorm slices: the next stage's parameters load in a later slice");
 
@@ -246,10 +238,18 @@ __device__ __forceinline__ int ln_off(int i, int wave, int lane) {
 __device__ __forceinline__ u32x4 ln_piece(u32x4 v, f32x2 st, const float4 (&gb)[kLnParamLoads]) {
     const float g[8] = {gb[0].x, gb[0].y, gb[0].z, gb[0].w, gb[1].x, gb[1].y, gb[1].z, gb[1].w};
     const float b[8] = {gb[2].x, gb[2].y, gb[2].z, gb[2].w, gb[3].x, gb[3].y, gb[3].z, gb[3].w};
+    // x - mean as x * 1 - mean, a mixed-precision multiply-add on the f16
+    // half itself: the same value without the conversion
+    float one = 1.0f;
+    asm("" : "+s"(one));
+    const float neg = -st[0];
     float f[8];
-    unpack(v, f, f16{});
 #pragma unroll
-    for (int j = 0; j < 8; j++) f[j] = ln_affine(f[j], st[0], st[1], g[j], b[j]);
+    for (int j = 0; j < 4; j++) {
+        const f16x2 h = u2h2(v[j]);
+        f[2 * j] = as_f32(fmaf(fmaf(static_cast<float>(h.x), one, neg) * st[1], g[2 * j], b[2 * j]));
+        f[2 * j + 1] = as_f32(fmaf(fmaf(static_cast<float>(h.y), one, neg) * st[1], g[2 * j + 1], b[2 * j + 1]));
+    }
     return pack(f, f16{});
 }
 
@@ -519,34 +519,20 @@ __global__ __launch_bounds__(P::kThreads, P::kWavesPerEu) void gemm_f16_kernel(
                                      : "memory");
                     else
                         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                    // w[cur] is free: refill it with stage s + 2
+                    if constexpr (NORM) read_slice(p ^ 1, cur ^ 1, 0);
+                    // w[cur] is free: refill it with stage s + 2, behind the
+                    // reads and between the multiplies
                     if constexpr (ISSUE) issue_w(sm.w[cur], 2 * (s + 2) * kBK);
-                    if constexpr (NORM) {
-#pragma unroll
-                        for (int a = 0; a < 2; a++) A[p ^ 1][a] = ld_op(sm.w[cur ^ 1], wn + 32 * a + l32, hh);
-#pragma unroll
-                        for (int b = 0; b < kRB; b++) B[p ^ 1][b] = ld_op(sm.x[cur ^ 1], wm + 32 * b + l32, hh);
-                    }
                 }
 #pragma unroll
                 for (int a = 0; a < 2; a++)
 #pragma unroll
                     for (int b = 0; b < kRB; b++)
                         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[p][a], B[p][b], acc[a][b], 0, 0, 0);
-                if (NORM && !kLnHints) {
-                    // the scheduler's own order
-                } else if (NORM && ks == 0 && kLnFirst > 0) {
-                    // the operand and raw reads ahead of the multiplies
-                    __builtin_amdgcn_sched_group_barrier(0x100, 6 + kLnRows, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-                } else if (NORM && ks >= kLnFirst && ks < kLnFirst + kLnSlices) {
-                    // the LayerNorm's vector work between the multiplies
-                    __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // an MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x002, kLnValuPerMfma, 0);  // VALU
-                    }
+                if constexpr (NORM) {
+                    // the compiler's own order: groups that forced the
+                    // LayerNorm's vector work between the multiplies were
+                    // slower (a 21x37 frame block of 16: 513 us against 502)
                 } else {
                     __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);  // LDS reads
                     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);  // MFMAs
