@@ -581,3 +581,24 @@ def test_linear_f32_split_heads_and_prologue(ctx, s, t, h):
                     ctx.linear_qkv_heads(xn, w, b, s, t, h, qn=qn, kn=kn, rope=rope)):
         assert torch.equal(a, c)
     assert torch.equal(ctx.linear_ln_gelu(x, ln, w, b), ctx.linear_gelu(xn, w, b))
+
+
+@pytest.mark.parametrize("t,h,d,k,dtype", [(8, 16, 128, 2048, torch.float32), (1, 2, 128, 64, torch.float32),
+                                           (200, 4, 128, 96, torch.float32), (33, 3, 64, 100, torch.float32),
+                                           (40, 8, 32, 128, torch.float16), (7, 5, 24, 40, torch.float16),
+                                           (7, 1, 3, 40, torch.float16)])
+@pytest.mark.parametrize("with_bias", [True, False])
+def test_linear_qkv_heads_one_sequence(ctx, t, h, d, k, dtype, with_bias):
+    """One sequence without norms or RoPE, shapes the fused kernel does not
+    cover: one product and one split, equal to the three apart, contiguous."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t + k)
+    x = torch.randn((t, k), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((3 * h * d, k), generator=g, device="cuda") / k ** 0.5).to(dtype)
+    b = torch.randn(3 * h * d, generator=g, device="cuda") * 0.02 if with_bias else None
+    got = ctx.linear_qkv_heads(x, w, b, 1, t, h)
+    outs = tuple(torch.empty((1, h, t, d), device="cuda", dtype=dtype) for _ in range(3))
+    apart = ctx.linear_qkv_heads(x, w, b, 1, t, h, out=outs)  # given outputs: the three apart
+    for a, c in zip(got, apart):
+        assert a.shape == c.shape == (1, h, t, d) and a.is_contiguous() and a.data_ptr() % 16 == 0
+        assert torch.equal(a, c)
