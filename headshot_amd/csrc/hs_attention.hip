@@ -1215,7 +1215,7 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
     if (flash_ok) {
         const float c = scale * 1.4426950408889634f;  // scores enter exp2
         auto grid = [&](int bm) { return static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * ceil_div(t, bm); };
-        if (grid(FlashPlain::kBM) < (int64_t{1} << 31) / FlashTwo::kThreads) {
+        if (grid(FlashPlain::kBM) < (int64_t{1} << 31) / FlashPlain::kThreads) {
             const f16 *fq = static_cast<const f16*>(q), *fk = static_cast<const f16*>(k);
             const f16* fv = static_cast<const f16*>(v);
             f16* fo = static_cast<f16*>(out);
@@ -1263,10 +1263,12 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
         // against 64).
         const bool few = static_cast<int64_t>(sh) * ceil_div(t, 128) <= num_cus();
         if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
-                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
+                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major) ||
+                      launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major))
             return check_launch("attention");
     }
-    if (dt == HS_F32 && d == kHD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
+    if (dt == HS_F32 && d == kHD && sh <= 65535 && aligned16(q) && aligned16(k) && aligned16(v) &&
+        aligned16(out)) {
         const int qtiles = static_cast<int>(ceil_div(t, 16));
         const int64_t blocks = static_cast<int64_t>(sh) * qtiles;
         if (blocks < (int64_t{1} << 31) / (64 * kHWaves)) {

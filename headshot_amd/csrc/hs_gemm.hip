@@ -1136,7 +1136,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
 // 2048 14.2 (74.7), 2048 x 8192 26 (279), i.e. 2.0-4.7 TB/s of weights; at 100
 // rows 18 (74), 65 (75), 62 (280); above 128 rows wide outputs are faster in
 // tiles (200 rows, 8192 x 2048: 110 against 80).
-constexpr int kSkinnyRows = 128;
+constexpr int kSkinnyRows = 128, kSkinnyCols = 1 << 22;
 constexpr int kSkWaves = 16, kSkThreads = 64 * kSkWaves;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -1441,7 +1441,8 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
         (!LN || (aligned16(la.ln_w) && aligned16(la.ln_b)))) {
         // (a rule on M alone, so that one product summed in parts of its
         // columns, as q, k and v apart, takes the same order of k)
-        if (M <= kSkinnyRows)
+        // (nor would wider outputs fit a grid of few-row workgroups)
+        if (M <= kSkinnyRows && N <= kSkinnyCols)
             launch_skinny<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
         else
             launch_split<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);

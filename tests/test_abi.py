@@ -287,3 +287,13 @@ def test_tables_contract():
     _einval(L.hs_rope_tables(rope.periods().ctypes.data, -1, 3, s.ctypes.data, s.ctypes.data),
             "negative")
     assert L.hs_rope_tables(None, 0, 3, None, None) == _lib.HS_OK
+
+
+def test_attention_d128_group_limit():
+    """f32 head_dim 128 takes at most 65535 (frame, head) pairs, also where
+    the buffers' alignment fits the matrix-core kernel: refused before any
+    launch (fake addresses, far apart)."""
+    L = _lib.load()
+    big = [ctypes.c_void_p(0x10000000 * i) for i in range(1, 5)]
+    for f in (L.hs_attention, L.hs_attention_merged):
+        assert f(None, F32, *big, 65536, 1, 1, 128) == _lib.HS_EUNSUPPORTED
