@@ -5,7 +5,7 @@
 // accumulation in f32, plus the (S, H, T, D) -> (S*T, H*D) head merge.
 //
 // Fast path (f16, D = 64): flash attention on the matrix cores. A wave owns
-// 32 queries; a workgroup of kWaves waves shares 64-key K/V tiles staged in
+// 32 queries; a workgroup's 8 waves (FlashShape) share 64-key K/V tiles staged in
 // LDS (double-buffered, the next tile prefetched into registers while the
 // current one computes). The wave computes the transposed score block
 // S^T = K Q^T with v_mfma_f32_32x32x16_f16, so each lane holds one query's
