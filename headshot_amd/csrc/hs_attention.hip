@@ -5,7 +5,7 @@
 // accumulation in f32, plus the (S, H, T, D) -> (S*T, H*D) head merge.
 //
 // Fast path (f16, D = 64): flash attention on the matrix cores. A wave owns
-// 32 queries; a workgroup's 8 waves (FlashShape) share 64-key K/V tiles staged in
+// 32 queries; a workgroup's waves (FlashShape) share 64-key K/V tiles staged in
 // LDS (double-buffered, the next tile prefetched into registers while the
 // current one computes). The wave computes the transposed score block
 // S^T = K Q^T with v_mfma_f32_32x32x16_f16, so each lane holds one query's
@@ -78,33 +78,21 @@ constexpr int kVPitch = kD + HS_ATT_VPAD;
 static_assert(HS_ATT_KPAD % 8 == 0 && HS_ATT_VPAD % 8 == 0, "rows must stay 16-byte aligned");
 constexpr int kChunks = kBN * kD / 8;  // 16-byte chunks per K (or V) tile
 
-// A workgroup's shape: KS groups of QW waves; a group's waves take 32 queries
-// each, every group the same QW x 32 queries over its own share of the key
-// tiles, staged in two buffers of its own.
-template <int QW, int KS>
+// A workgroup's shape: QW waves of 32 queries each over the same key tiles. A
+// query's result does not depend on it.
+template <int QW>
 struct FlashShape {
-    static constexpr int kQW = QW, kKS = KS;
-    static constexpr int kThreads = 64 * QW * KS;
-    static constexpr int kBM = 32 * QW;                    // queries per workgroup
-    static constexpr int kPer = kChunks / (64 * QW);       // 16-byte chunks per thread of a tile
-    static_assert(kPer * 64 * QW == kChunks, "tile split");
+    static constexpr int kThreads = 64 * QW;
+    static constexpr int kBM = 32 * QW;               // queries per workgroup
+    static constexpr int kPer = kChunks / kThreads;   // 16-byte chunks per thread of a tile
+    static_assert(kPer * kThreads == kChunks, "tile split");
     struct Smem {
-        f16 k[KS][2][kBN * kKPitch];
-        f16 v[KS][2][kBN * kVPitch];
-    };
-    // half of the groups' outputs (32 floats a lane) and (m, l) at a time
-    struct Merge {
-        float o[KS > 1 ? KS / 2 * QW : 1][32][64];
-        float ml[KS > 1 ? KS / 2 * QW : 1][2][64];
-    };
-    union Lds {
-        Smem tiles;
-        Merge merge;
+        f16 k[2][kBN * kKPitch];
+        f16 v[2][kBN * kVPitch];
     };
 };
-using FlashPlain = FlashShape<8, 1>;  // two workgroups per CU
-using FlashTwo = FlashShape<8, 2>;    // one per CU
-using FlashHalf = FlashShape<4, 2>;   // one per CU
+using FlashPlain = FlashShape<8>;  // two workgroups per CU
+using FlashHalf = FlashShape<4>;   // four per CU
 
 __device__ __forceinline__ h8 as_h8(u32x4 v) { return __builtin_bit_cast(h8, v); }
 
@@ -115,7 +103,7 @@ __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
 }
 
 // One thread's share of a 64-row K or V tile: 16-byte chunk c = tid + i *
-// threads (of its group) is row c / 8, channels (c % 8) * 8 .. + 8.
+// threads is row c / 8, channels (c % 8) * 8 .. + 8.
 template <int PER>
 struct TileChunks {
     u32x4 c[PER];
@@ -322,29 +310,21 @@ __device__ __forceinline__ void store_out(const f32x16& o0, const f32x16& o1, fl
 // b % kXcds, query tile qt0 + (b / kXcds) % QT.
 // TAIL: the launch of the partial last query tiles (qt0 = their index),
 // whose waves with every query past T only stage K and V.
-//
-// One workgroup per CU leaves two waves per SIMD, and a tile then takes nearly
-// as long as with four (1.36 us against 1.58). Where the grid is that small a
-// workgroup holds KS groups of waves instead, each over its own contiguous
-// share of the key tiles, whose (O, m, l) are merged through LDS in halves at
-// the end.
 template <bool TAIL, typename P>
 __global__ __launch_bounds__(P::kThreads) void flash_f16_kernel(
     const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v,
     f16* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c,
     int token_major, int qt0) {
-    constexpr int kBM = P::kBM, kKS = P::kKS;
-    __shared__ __align__(16) typename P::Lds lds;
-    typename P::Smem& sm = lds.tiles;
+    constexpr int kBM = P::kBM;
+    __shared__ __align__(16) typename P::Smem sm;
     const int b = blockIdx.x;
     const int slot = b / kXcds;
     const int sh = (slot / qtiles) * kXcds + b % kXcds;
     if (sh >= sh_count) return;  // workgroup-uniform, before any barrier
     const int qt = qt0 + slot % qtiles;
     const int lane = lane_id();
-    const int kg = kKS == 1 ? 0 : wave_in_block() / P::kQW;  // the wave's key group
-    const int wave = static_cast<int>(threadIdx.x >> 6) - kg * P::kQW;
-    const int tid = static_cast<int>(threadIdx.x) - kg * (64 * P::kQW);  // within the group
+    const int tid = static_cast<int>(threadIdx.x);
+    const int wave = tid >> 6;
     const int n = lane & 31, hh = lane >> 5;
     const int64_t base = static_cast<int64_t>(sh) * t * kD;
     const f16* qb = q + base;
@@ -367,37 +347,32 @@ __global__ __launch_bounds__(P::kThreads) void flash_f16_kernel(
     f32x16 o[2] = {f32x16{}, f32x16{}};
     float m = -INFINITY, l = 0.0f;
     const int ntiles = static_cast<int>(ceil_div(t, kBN));
-    // the group's tiles [j0, j1), `steps` for every group (the last ones may
-    // have fewer, or none)
-    const int steps = kKS == 1 ? ntiles : (ntiles + kKS - 1) / kKS;
-    const int j0 = kg * steps, j1 = min(j0 + steps, ntiles);
 
     // Double-buffered tiles: tile j + 1 is loaded into registers while tile
     // j computes from LDS, then written to the other buffer (last read in
     // iteration j - 1, which the barrier at its end closed).
     TileChunks<P::kPer> pk, pv;
-    load_rows(pk, kb, j0 * kBN, t, tid);
-    load_rows(pv, vb, j0 * kBN, t, tid);
-    store_rows<kKPitch>(pk, sm.k[kg][0], tid);
-    store_rows<kVPitch>(pv, sm.v[kg][0], tid);
+    load_rows(pk, kb, 0, t, tid);
+    load_rows(pv, vb, 0, t, tid);
+    store_rows<kKPitch>(pk, sm.k[0], tid);
+    store_rows<kVPitch>(pv, sm.v[0], tid);
     __syncthreads();
-    for (int i = 0; i < steps; i++) {
-        const int j = j0 + i;
-        const int cur = i & 1;
-        if (i + 1 < steps) {
+    for (int j = 0; j < ntiles; j++) {
+        const int cur = j & 1;
+        if (j + 1 < ntiles) {
             load_rows(pk, kb, (j + 1) * kBN, t, tid);
             load_rows(pv, vb, (j + 1) * kBN, t, tid);
         }
-        if ((!TAIL || qt * kBM + wave * 32 < t) && (kKS == 1 || j < j1)) {
+        if (!TAIL || qt * kBM + wave * 32 < t) {
             f32x16 sc[kKB];
-            qk_scores(sc, sm.k[kg][cur], qa, n, hh);
+            qk_scores(sc, sm.k[cur], qa, n, hh);
             u32x4 p[kKB][2];
             if ((j + 1) * kBN > t) mask_tail(sc, j * kBN, t, hh);
             // After the first tile, weights against the kept reference; the
             // max path only when some lane's sum says a weight may exceed
             // 2^15 (a row sum above 2^15 means a weight above 2^10, more
             // than kLazyMax over m, so that path then moves m).
-            bool max_path = i == 0;
+            bool max_path = j == 0;
             if (!max_path) {
                 const float ps = weights_tile(sc, c, m, p);
                 max_path = __any(!(ps <= kRowSumMax));
@@ -407,42 +382,16 @@ __global__ __launch_bounds__(P::kThreads) void flash_f16_kernel(
                 const float corr = softmax_tile(sc, c, m, l, p);
                 rescale(o[0], o[1], corr);
             }
-            pv_update(o, sm.v[kg][cur], p, n, hh);
+            pv_update(o, sm.v[cur], p, n, hh);
         }
-        if (i + 1 < steps) {
-            store_rows<kKPitch>(pk, sm.k[kg][cur ^ 1], tid);
-            store_rows<kVPitch>(pv, sm.v[kg][cur ^ 1], tid);
+        if (j + 1 < ntiles) {
+            store_rows<kKPitch>(pk, sm.k[cur ^ 1], tid);
+            store_rows<kVPitch>(pv, sm.v[cur ^ 1], tid);
         }
         __syncthreads();
     }
 
-    // Merge the groups, upper half into lower half (a group without tiles
-    // has m = -inf, l = 0 and O = 0; group 0 has tiles). The tiles' LDS is free.
-#pragma unroll
-    for (int half = kKS / 2; half >= 1; half /= 2) {
-        if (kg >= half && kg < 2 * half) {
-            const int w = (kg - half) * P::kQW + wave;
-#pragma unroll
-            for (int r = 0; r < 16; r++) lds.merge.o[w][r][lane] = o[0][r], lds.merge.o[w][16 + r][lane] = o[1][r];
-            lds.merge.ml[w][0][lane] = m, lds.merge.ml[w][1][lane] = l;
-        }
-        __syncthreads();
-        if (kg < half) {
-            const int w = kg * P::kQW + wave;
-            const float m1 = lds.merge.ml[w][0][lane], l1 = lds.merge.ml[w][1][lane];
-            const float mm = fmaxf(m, m1);
-            const float f0 = __builtin_amdgcn_exp2f(m - mm), f1 = __builtin_amdgcn_exp2f(m1 - mm);
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                o[0][r] = fmaf(o[0][r], f0, lds.merge.o[w][r][lane] * f1);
-                o[1][r] = fmaf(o[1][r], f0, lds.merge.o[w][16 + r][lane] * f1);
-            }
-            l = fmaf(l, f0, l1 * f1);
-            m = mm;
-        }
-        if (half > 1) __syncthreads();
-    }
-    if (kg > 0 || qi >= t) return;
+    if (qi >= t) return;
     f16* orow;
     if (token_major) {
         const int s = sh / heads, h = sh - s * heads;
@@ -1214,28 +1163,25 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
                           (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
     if (flash_ok) {
         const float c = scale * 1.4426950408889634f;  // scores enter exp2
-        auto grid = [&](int bm) { return static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * ceil_div(t, bm); };
-        if (grid(FlashPlain::kBM) < (int64_t{1} << 31) / FlashPlain::kThreads) {
+        const int qtiles = static_cast<int>(ceil_div(t, FlashPlain::kBM));
+        const int64_t seqs = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds);
+        if (seqs * qtiles < (int64_t{1} << 31) / FlashPlain::kThreads) {
             const f16 *fq = static_cast<const f16*>(q), *fk = static_cast<const f16*>(k);
             const f16* fv = static_cast<const f16*>(v);
             f16* fo = static_cast<f16*>(out);
-            const int qtiles = static_cast<int>(ceil_div(t, FlashPlain::kBM));
             const int64_t cus = num_cus();
-            // Key groups while one workgroup per CU holds the grid, with 128
-            // queries where they do, else 256. 16 heads, us with FlashPlain
-            // and here: 408 tokens 12.9, 9.4; 782 19.6, 13.2; 1386 29.3, 18.9;
-            // 2 x 1386 (192 workgroups of 256) 30.2, 27.9; 2772 53, 47. Two 4-wave
-            // groups with two workgroups per CU: 2 x 1386 35.6.
-            if (t > kBN && static_cast<int64_t>(sh) * ceil_div(t, FlashHalf::kBM) <= cus) {
-                flash_f16_kernel<false, FlashHalf><<<dim3(static_cast<uint32_t>(grid(FlashHalf::kBM))),
+            const int half_tiles = static_cast<int>(ceil_div(t, FlashHalf::kBM));
+            // 128 queries per workgroup while one per CU holds them all: 16
+            // heads, us with 256 and here: 408 tokens 12.7, 9.6; 782 19.3,
+            // 14.9; 1386 29.1, 22.6; 2000 (250 workgroups) 40.0, 31.4.
+            // Past that two of 256 per CU share the tiles' loads better (2 x
+            // 1386 29.6, 31.8; 2772 53.2, 57.9). Splitting the keys over wave
+            // groups is faster still (1386 18.7) but sums a query in an order
+            // that follows the batch: not taken.
+            if (static_cast<int64_t>(sh) * half_tiles <= cus) {
+                flash_f16_kernel<false, FlashHalf><<<dim3(static_cast<uint32_t>(seqs * half_tiles)),
                                                      dim3(FlashHalf::kThreads), 0, st>>>(
-                    fq, fk, fv, fo, sh, h, t, static_cast<int>(ceil_div(t, FlashHalf::kBM)), c, token_major, 0);
-                return check_launch("attention");
-            }
-            if (t > kBN && static_cast<int64_t>(sh) * qtiles <= cus) {
-                flash_f16_kernel<false, FlashTwo><<<dim3(static_cast<uint32_t>(grid(FlashTwo::kBM))),
-                                                    dim3(FlashTwo::kThreads), 0, st>>>(
-                    fq, fk, fv, fo, sh, h, t, qtiles, c, token_major, 0);
+                    fq, fk, fv, fo, sh, h, t, half_tiles, c, token_major, 0);
                 return check_launch("attention");
             }
             // A partial last query tile runs as a launch of its own when
@@ -1246,7 +1192,6 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
             // overlap the other tiles.
             const bool split = t % FlashPlain::kBM != 0 && qtiles > 1 && sh >= 2 * cus;
             const int main_tiles = split ? qtiles - 1 : qtiles;
-            const int64_t seqs = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds);
             flash_f16_kernel<false, FlashPlain><<<dim3(static_cast<uint32_t>(seqs * main_tiles)),
                                                   dim3(FlashPlain::kThreads), 0, st>>>(
                 fq, fk, fv, fo, sh, h, t, main_tiles, c, token_major, 0);

@@ -487,19 +487,35 @@ def test_attention_f32_split_special_values(ctx):
 @pytest.mark.parametrize("s,h,t", [(1, 2, 65), (1, 2, 129), (1, 3, 193), (2, 16, 300), (1, 16, 2100),
                                    (1, 40, 1600), (1, 260, 300)])
 @pytest.mark.parametrize("spread", [1.0, 6.0])
-def test_attention_f16_key_groups(ctx, s, h, t, spread):
-    """f16 grids of at most one workgroup per CU split the keys over two wave
-    groups (4 or 8 query waves each; odd tile counts, a group one tile
-    short, a single tile more than a group) and merge; the last shape is past
-    both. Against the float64 softmax of the f16 values: weights and the
-    result round to f16."""
+def test_attention_f16_small_grids(ctx, s, h, t, spread):
+    """f16 grids of at most one 128-query workgroup per CU take four waves, the
+    others eight (the last shapes). Against the float64 softmax of the f16
+    values: weights and the result round to f16."""
     rng = np.random.default_rng(h * 1000 + t)
     q, k, v = (rng.standard_normal((s, h, t, 64)).astype(np.float16) for _ in range(3))
     q *= np.float16(spread)
-    # keys that rise along the sequence: the groups' maxima differ widely
+    # keys that rise along the sequence: the running max moves
     k[:, :, t // 2:] *= np.float16(1.5)
     got = back(ctx.attention(dev(q), dev(k), dev(v))).astype(np.float64)
     heads = [0, h - 1]
     want = naive64(q[:, heads].astype(np.float32), k[:, heads].astype(np.float32), v[:, heads].astype(np.float32))
     assert np.abs(got[:, heads] - want).max() < 4e-3
     assert _rel(got[:, heads], want) < 1e-3
+
+
+@pytest.mark.parametrize("t", [1, 33, 64, 65, 127, 129, 257, 1386])
+def test_attention_f16_alone_is_the_batch(ctx, t):
+    """A sequence's result does not follow the grid: alone (four waves per
+    workgroup), in a batch past one workgroup per CU (eight) and past two
+    (a partial last tile in a launch of its own) bit for bit the same."""
+    heads = 16
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t)
+    q, k, v = (torch.randn((33, heads, t, 64), generator=g, device="cuda").half() for _ in range(3))
+    q *= 4.0
+    whole = ctx.attention(q, k, v)
+    for s in (1, 2, 17):
+        part = ctx.attention(q[:s], k[:s], v[:s])
+        assert torch.equal(part, whole[:s]), s
+    one = ctx.attention(q[:1, :1].contiguous(), k[:1, :1].contiguous(), v[:1, :1].contiguous())
+    assert torch.equal(one[0, 0], whole[0, 0])
