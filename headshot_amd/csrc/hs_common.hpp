@@ -149,6 +149,29 @@ __device__ __forceinline__ u32x4 pack(const float (&f)[4], float) {
     return v;
 }
 
+// An f32 value as three bf16 ones, a = h + m + l with h = bf16(a), m = bf16(a -
+// h), l = a - h - m: 8 + 8 + 8 bits hold a's 24 and both differences are exact,
+// so nothing of a is lost while l's last bit is one bf16 has (|a| from 2^-110).
+// A product of two such sums is, to 2^-24 of itself, the six terms hh, hm, mh,
+// mm, hl, lh (the three left out: |m| <= 2^-8 |a|, |l| <= 2^-17 |a|).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    asm("" : "+v"(p));  // converted once, as a pair
+    return p;
+}
+
+// a and b split, each part's pair packed. (The differences as dot products
+// with (-1, 0) and (0, -1) are four instructions fewer and slower.)
+__device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pk_bf16(a, b);
+    const float ra = a - u2f(h << 16), rb = b - u2f(h & 0xFFFF0000u);
+    m = pk_bf16(ra, rb);
+    l = pk_bf16(ra - u2f(m << 16), rb - u2f(m & 0xFFFF0000u));
+}
+
 // Exact-erf GELU, gelu.wesl:18-38: 0.5*v*(1 + erf(v/sqrt(2))) with erf by
 // Abramowitz & Stegun 7.1.26, erf(z) = sign(z)*(1 - P(t)*t*exp(-z^2)),
 // t = 1/(1 + p*|z|). Evaluated in f32 from h = v/2 (exact), with the

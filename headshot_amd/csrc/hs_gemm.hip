@@ -30,7 +30,7 @@
 // S=32: 494 us against 523).
 //
 // f32 (N % 128 == 0, K % 32 == 0; every epilogue, with or without the LayerNorm
-// prologue): each operand as two f16 values on the f16 matrix cores
+// prologue): each operand as three bf16 values on the bf16 matrix cores
 // (gemm_split_kernel), or up to 128 rows a kernel that splits K over its waves
 // and streams the weights straight into registers (gemm_skinny_kernel).
 //
@@ -844,47 +844,48 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[2][kRB], const float* x,
 }
 
 // ---------------------------------------------------------------------------
-// f32 products on the f16 matrix cores (N % 128 == 0, K % 32 == 0, more rows
+// f32 products on the bf16 matrix cores (N % 128 == 0, K % 32 == 0, more rows
 // than gemm_skinny_kernel takes). The f32 matrix instructions run at a
-// sixteenth of the f16 rate; an f32 value is, to 2^-24 of itself, the sum of
-// two f16 values, a = h + l / 2048 with h = f16(a) and l = f16((a - h) 2048),
-// so that three f16 products with f32 accumulators
-//     sum(h_x h_w)  +  (sum(h_x l_w) + sum(l_x h_w)) / 2048
-// give the f32 product but for l_x l_w / 2^22 (below 2^-24 of |a_x a_w|) and
-// the two roundings of l. Every f16 product is exact in f32, and the chain of
-// accumulations is K / 16 long instead of K / 2, so the result is nearer the
-// 64-bit product than the f32 instructions' (DINO's q|k|v: 2.2e-7 against
-// 5.7e-7, fc2's 4096 terms 3.0e-7 against 8.1e-7).
+// sixteenth of the bf16 rate; an f32 value is the sum of three bf16 ones
+// (split3), a = h + m + l, and six products of those, every one exact in f32,
+//     sum(h h)  +  sum(m m + m h + h m + l h + h l)
+// give the f32 product to 2^-24 of each term, as one rounding of it would. The
+// second sum, 2^-8 of the first, has accumulators of its own, so the chain of
+// full-size roundings is K / 16 long instead of the f32 instructions' K / 2.
 //
-// l is held times 2048, in accumulators of its own, so both halves keep 11
-// bits for |a| from 2^-14 to 65504; smaller values lose absolute precision
-// only (2^-36). A row whose largest magnitude is above 65504 or below 2^-13
-// (all zeros apart) would lose more than 2^-23 of it: each workgroup tracks
-// its rows' maxima while it converts, and a tile with such a row (infinities
-// among them) is computed again on v_mfma_f32_32x32x2_f32.
+// The bf16 parts have f32's exponents, so this holds for every |a| from 2^-100
+// up. An output whose x or w row has a smaller nonzero element (from 2^-134 up;
+// below, f32 subnormals count as zero), and one that comes out infinite or NaN,
+// is computed again on v_mfma_f32_32x32x2_f32 (f32_block). That is decided
+// for each output by its own two rows, so no result depends on what shares its
+// tile.
 //
 // A workgroup of WM x WN waves computes 32 RB WM rows x 64 WN columns, a wave 32
-// RB x 64 as out^T blocks. K goes in stages of 32 through LDS, two buffers: a
-// stage row is 128 bytes, logical chunk 2 c holding h and 2 c + 1 l of floats 8
-// c .. + 8, at physical chunk ^ swz(row) (operand reads and these writes
-// conflict-free). The f32 pieces are prefetched into registers a stage ahead
-// and converted once per workgroup between the multiplies (~3 vector
-// instructions per element, 4.5 per MFMA).
-// Bounds: the sum of matrix and vector issue, which overlap little at two waves
-// per SIMD. At 10992 rows, q|k|v / proj / fc1 / fc2, us: 273 / 107 / 358 / 323
-// (242-285 TFLOP/s of f32 product) against 560 / 202 / 694 / 731 on the f32
-// matrix cores (94-133, peak 157); at 2748 rows 98 / 36 / 106 / 107 against 162 /
-// 67 / 199 / 247.
+// RB x 64 as out^T blocks. K goes in stages of 16 through LDS, two buffers of
+// three planes (h, m, l) of 32-byte rows: chunk c (8 floats) of row r at c ^ ((r
+// / 8) % 2), so sixteen rows' reads of a chunk and these writes cover the banks
+// once. The f32 pieces are prefetched into registers and converted once per
+// workgroup between the multiplies (6.5 vector instructions per element).
+// Bounds: matrix issue (six MFMAs where f16 has one) with the conversion
+// beside it. At 10992 rows, q|k|v / proj / fc1 / fc2, us: 390 / 140 / 500 / 486
+// (165-190 TFLOP/s of f32 product) against 586 / 198 / 690 / 722 on the f32
+// matrix cores; at 2748 rows 131 / 43 / 141 / 136 against 194 / 65 / 199 / 246.
+// With two f16 parts and three products they were 273 / 100 / 346 / 312, but
+// those parts keep no element below 2^-36 and only 22 bits of the others.
+// Relative error against 64 bits, q|k|v and fc2: 1.9e-7 and 4.0e-7; the f32
+// instructions 5.7e-7 and 1.15e-6. A 10992-row q|k|v with a row below 2^-100 in
+// every tile, all computed twice: 1.05 ms. 256 x 128 and 128 x 256 tiles by 8
+// waves: 478 and 471 us for q|k|v.
 template <int WM, int WN, int RB_>
 struct SplitTile {
     static constexpr int kWN = WN, kWaves = WM * WN, kThreads = 64 * kWaves, kRB = RB_;
-    static constexpr int kBM = 32 * RB_ * WM, kBN = 64 * WN, kBK = 32;
-    static constexpr int kPR = kThreads / 4;                                   // rows a pass of pieces covers
-    static constexpr int kXP = kBM / kPR, kWP = kBN / kPR, kPieces = kXP + kWP;  // 8-float pieces per thread
+    static constexpr int kBM = 32 * RB_ * WM, kBN = 64 * WN, kBK = 16;
+    static constexpr int kPR = kThreads / 4;                                     // rows a pass of pieces covers
+    static constexpr int kXP = kBM / kPR, kWP = kBN / kPR, kPieces = kXP + kWP;  // 4-float pieces per thread
     static_assert(kXP * kPR == kBM && kWP * kPR == kBN && kPR % 16 == 0, "pieces");
     struct Smem {
-        f16 x[2][kBM * 64];
-        f16 w[2][kBN * 64];
+        uint16_t x[2][3][kBM * kBK];
+        uint16_t w[2][3][kBN * kBK];
     };
     static constexpr size_t smem_bytes(int epi) {
         const size_t qkv = epi == EPI_QKV ? size_t{4} * kWaves * 32 * kRB * kQkvPitch : 0;
@@ -894,24 +895,11 @@ struct SplitTile {
 using SplitShape = SplitTile<2, 2, 2>;   // 128 x 128, two workgroups per CU
 using SplitEight = SplitTile<4, 2, 1>;   // 128 x 128 by 8 waves
 using SplitNarrow = SplitTile<2, 2, 1>;  // 64 x 128
-constexpr float kSplitMax = 65504.0f, kSplitMin = 0x1p-13f;
+constexpr int kSplitKs = 32;             // K is a multiple: stages go in pairs
 
-// 8 floats as h and l chunks; mx gathers their largest magnitude.
-__device__ __forceinline__ void split8(const u32x4 (&v)[2], u32x4& hi, u32x4& lo, float& mx) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float a = u2f(v[i / 2][2 * (i % 2)]), b = u2f(v[i / 2][2 * (i % 2) + 1]);
-        uint32_t hp = pk_f16(a, b);
-        asm("" : "+v"(hp));  // converted once, as a pair
-        const f16x2 h = u2h2(hp);
-        f16x2 l;
-        // a - h is exact in f32
-        l.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, a * 2048.0f));
-        l.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, b * 2048.0f));
-        hi[i] = hp, lo[i] = h22u(l);
-        mx = fmaxf(fmaxf(mx, fabsf(a)), fabsf(b));
-    }
-}
+// Twice the bf16 bits of 2^-100. 2 bits - kSmallest, mod 2^16, is then above the
+// value zero gives for the nonzero magnitudes below 2^-100 and for no others.
+constexpr uint32_t kSmallest = 0x1B00;
 
 __device__ __forceinline__ u32x4 buf_ld16(__amdgpu_buffer_rsrc_t src, uint32_t voff, int soff) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
@@ -922,9 +910,10 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
     const float* __restrict__ gamma, const float* res, float* out, int M, int N, int K,
     int tiles_n, int ntiles, LnArgs la, QkvArgs qa) {
-    constexpr int kRB = P::kRB, kXP = P::kXP, kWP = P::kWP;
+    constexpr int kRB = P::kRB, kXP = P::kXP, kPieces = P::kPieces;
     __shared__ __align__(16) unsigned char smem_raw[P::smem_bytes(EPI)];
-    __shared__ int out_of_range;
+    __shared__ uint8_t odd[P::kBM + P::kBN];  // x rows, then w rows, with an element below 2^-100
+    __shared__ int any_odd;
     typename P::Smem& sm = *reinterpret_cast<typename P::Smem*>(smem_raw);
     const int tid = threadIdx.x;
     const int lane = lane_id(), wave = wave_in_block();
@@ -941,7 +930,8 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     const int64_t n0 = static_cast<int64_t>(tile % tiles_n) * P::kBN;
     const int wm = (wave / P::kWN) * (32 * kRB);
     const int wn = (wave % P::kWN) * 64;
-    if (tid == 0) out_of_range = 0;
+    for (int i = tid; i < P::kBM + P::kBN; i += P::kThreads) odd[i] = 0;
+    if (tid == 0) any_odd = 0;
 
     const int xrows = static_cast<int>(min(static_cast<int64_t>(P::kBM), M - m0));
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -949,50 +939,65 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(w + n0 * K), 0, P::kBN * K * 4, kRawBufferFlags);
     // Pieces 0 .. kXP of the thread are x's, the rest w's: piece i is row kPR i +
-    // tid / 4 of its operand, floats 8 (tid % 4) .. + 8 of the stage (x rows
+    // tid / 4 of its operand, floats 4 (tid % 4) .. + 4 of the stage (x rows
     // past M read row M - 1; their outputs are masked).
     const int prow = tid / 4, pc = tid % 4;
-    uint32_t off[P::kPieces];
+    uint32_t off[kPieces];
     f32x2 lst[kXP];
 #pragma unroll
-    for (int i = 0; i < kXP; i++) {
-        const int row = static_cast<int>(min(m0 + P::kPR * i + prow, static_cast<int64_t>(M) - 1) - m0);
-        off[i] = static_cast<uint32_t>(row * K * 4 + 32 * pc);
-        if constexpr (LN) lst[i] = *reinterpret_cast<const f32x2*>(la.stats + 2 * (m0 + row));
+    for (int i = 0; i < kPieces; i++) {
+        if (i < kXP) {
+            const int row = static_cast<int>(min(m0 + P::kPR * i + prow, static_cast<int64_t>(M) - 1) - m0);
+            off[i] = static_cast<uint32_t>(row * K * 4 + 16 * pc);
+            if constexpr (LN) lst[i < kXP ? i : 0] = *reinterpret_cast<const f32x2*>(la.stats + 2 * (m0 + row));
+        } else {
+            off[i] = static_cast<uint32_t>((P::kPR * (i - kXP) + prow) * K * 4 + 16 * pc);
+        }
     }
-#pragma unroll
-    for (int i = 0; i < kWP; i++) off[kXP + i] = static_cast<uint32_t>((P::kPR * i + prow) * K * 4 + 32 * pc);
-    // halves offsets of a piece's h and l chunks (kPR rows on: the same swizzle)
-    const int dh = prow * 64 + 8 * ((2 * pc) ^ swz(prow)), dl = prow * 64 + 8 * ((2 * pc + 1) ^ swz(prow));
+    // halves offset of a piece within its plane (kPR rows on: the same swizzle)
+    const int dst = prow * 16 + 8 * ((pc >> 1) ^ ((prow >> 3) & 1)) + 4 * (pc & 1);
 
-    u32x4 raw[P::kPieces][2];
-    float mx[P::kPieces];
+    // the next stage's pieces and the LayerNorm parameters of their columns
+    u32x4 raw[kPieces];
+    float4 lw, lb;
+    uint32_t mx[kPieces];  // two 16-bit maxima of 2 bits(h) - kSmallest
 #pragma unroll
-    for (int i = 0; i < P::kPieces; i++) mx[i] = 0.0f;
-    const int nsteps = K / P::kBK;
+    for (int i = 0; i < kPieces; i++) mx[i] = 0;
+    uint32_t two = 0x00020002u, small = (0x10000u - kSmallest) * 0x00010001u;
+    asm("" : "+v"(two), "+v"(small));
+    const int nsteps = K / P::kBK;  // even
     auto load_piece = [&](int i, int s) {
-        const __amdgpu_buffer_rsrc_t src = i < kXP ? xr : wr;
-        raw[i][0] = buf_ld16(src, off[i], s * 128);
-        raw[i][1] = buf_ld16(src, off[i] + 16, s * 128);
-    };
-    // Piece i of stage s into buffer buf, as h and l.
-    auto store_piece = [&](int i, int s, int buf) {
+        raw[i] = buf_ld16(i < kXP ? xr : wr, off[i], s * 64);
         if constexpr (LN) {
-            if (i < kXP) {
-                // each element as hs_layernorm stores it
-                const int c = s * P::kBK + 8 * pc;
-                raw[i][0] = ln_quad(raw[i][0], lst[i < kXP ? i : 0], ld_f32x4(la.ln_w + c), ld_f32x4(la.ln_b + c));
-                raw[i][1] = ln_quad(raw[i][1], lst[i < kXP ? i : 0], ld_f32x4(la.ln_w + c + 4), ld_f32x4(la.ln_b + c + 4));
+            if (i == kXP - 1) {  // no x piece of the stage before needs them any more
+                const int c = s * P::kBK + 4 * pc;
+                lw = ld_f32x4(la.ln_w + c), lb = ld_f32x4(la.ln_b + c);
             }
         }
-        u32x4 h, l;
-        split8(raw[i], h, l, mx[i]);
-        f16* dst = (i < kXP ? sm.x[buf] + P::kPR * 64 * i : sm.w[buf] + P::kPR * 64 * (i - kXP));
-        st16(dst + dh, h);
-        st16(dst + dl, l);
+    };
+    // Piece i into buffer buf, as h, m and l.
+    auto store_piece = [&](int i, int buf) {
+        u32x4 v = raw[i];
+        if constexpr (LN) {
+            if (i < kXP) v = ln_quad(v, lst[i < kXP ? i : 0], lw, lb);  // as hs_layernorm stores it
+        }
+        u32x2 part[3];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            uint32_t h, m, l, t;
+            split3(u2f(v[2 * j]), u2f(v[2 * j + 1]), h, m, l);
+            part[0][j] = h, part[1][j] = m, part[2][j] = l;
+            asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t) : "v"(h), "v"(two), "v"(small));
+            asm("v_pk_max_u16 %0, %1, %2" : "=v"(mx[i]) : "v"(t), "v"(mx[i]));
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            uint16_t* plane = i < kXP ? sm.x[buf][q] + P::kPR * 16 * i : sm.w[buf][q] + P::kPR * 16 * (i - kXP);
+            *reinterpret_cast<u32x2*>(plane + dst) = part[q];
+        }
     };
 
-    // acc[a][b] (and the 1 / 2048 part, acl): register r of lane (l32, hh) is
+    // acc[a][b] (and the small products', acl): register r of lane (l32, hh) is
     // column wn + 32 a + 8 (r / 4) + 4 hh + r % 4, row wm + 32 b + l32
     f32x16 acc[2][kRB], acl[2][kRB];
 #pragma unroll
@@ -1000,122 +1005,141 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
 #pragma unroll
         for (int b = 0; b < kRB; b++) acc[a][b] = f32x16{}, acl[a][b] = f32x16{};
 
-    h8 Ah[2][2], Bh[2][kRB], Al[2], Bl[kRB];  // h operands of two slices, l of one
-    auto read_h = [&](int ks, int buf) {
-        const int ch = 2 * (2 * ks + hh);
+    // operands: h of two stages, m and l of one
+    u32x4 Ah[2][2], Bh[2][kRB], Am[2], Bm[kRB], Al[2], Bl[kRB];
+    const int op = l32 * 16 + 8 * (hh ^ ((l32 >> 3) & 1));
+    auto read_a = [&](u32x4(&d)[2], int q, int buf) {
 #pragma unroll
-        for (int a = 0; a < 2; a++) Ah[ks][a] = ld_op(sm.w[buf], wn + 32 * a + l32, ch);
-#pragma unroll
-        for (int b = 0; b < kRB; b++) Bh[ks][b] = ld_op(sm.x[buf], wm + 32 * b + l32, ch);
+        for (int a = 0; a < 2; a++) d[a] = ld16(sm.w[buf][q] + (wn + 32 * a) * 16 + op);
     };
-    auto read_l = [&](int ks, int buf) {
-        const int ch = 2 * (2 * ks + hh) + 1;
+    auto read_b = [&](u32x4(&d)[kRB], int q, int buf) {
 #pragma unroll
-        for (int b = 0; b < kRB; b++) Bl[b] = ld_op(sm.x[buf], wm + 32 * b + l32, ch);
-#pragma unroll
-        for (int a = 0; a < 2; a++) Al[a] = ld_op(sm.w[buf], wn + 32 * a + l32, ch);
+        for (int b = 0; b < kRB; b++) d[b] = ld16(sm.x[buf][q] + (wm + 32 * b) * 16 + op);
     };
-    // part 0 h_x h_w, 1 l_x h_w, 2 h_x l_w of slice ks
-    auto multiply = [&](int ks, int part) {
+    auto multiply = [&](f32x16(&c)[2][kRB], const u32x4(&A)[2], const u32x4(&B)[kRB]) {
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
-            for (int b = 0; b < kRB; b++) {
-                if (part == 0)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ks][a], Bh[ks][b], acc[a][b], 0, 0, 0);
-                else if (part == 1)
-                    acl[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ks][a], Bl[b], acl[a][b], 0, 0, 0);
-                else
-                    acl[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al[a], Bh[ks][b], acl[a][b], 0, 0, 0);
-            }
+            for (int b = 0; b < kRB; b++)
+                c[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A[a]),
+                                                                 __builtin_bit_cast(bf16x8, B[b]), c[a][b], 0, 0, 0);
     };
 #pragma unroll
-    for (int i = 0; i < P::kPieces; i++) load_piece(i, 0);
+    for (int i = 0; i < kPieces; i++) load_piece(i, 0);
 #pragma unroll
-    for (int i = 0; i < P::kPieces; i++) store_piece(i, 0, 0);
-    if (nsteps > 1) {
+    for (int i = 0; i < kPieces; i++) store_piece(i, 0);
 #pragma unroll
-        for (int i = 0; i < P::kPieces; i++) load_piece(i, 1);
-    }
+    for (int i = 0; i < kPieces; i++) load_piece(i, 1);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    read_h(0, 0);
-    // A stage's six groups of multiplies. In the first five, stage s + 1 is
+    // lgkmcnt(0) again, as an instruction the compiler knows: with scalar loads
+    // pending, as far as it can tell, it would wait for every read of a stage
+    // at the loop's top (395 us for q|k|v at 10992 rows against 390)
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    read_a(Ah[0], 0, 0);
+    read_b(Bh[0], 0, 0);
+    // A stage's six groups of multiplies. In the first four, stage s + 1 is
     // converted into the other buffer (last read before the barrier of the
-    // step before) and stage s + 2's pieces are loaded behind it; the barrier
-    // then opens stage s + 1, and its first h operands are read under the last
-    // group. NEXT: stage s + 1 exists.
-    auto step = [&](int s, auto next_c) {
+    // stage before) and stage s + 2's pieces are loaded behind it; the barrier then opens stage s + 1, and its h operands are read under the
+    // last group. cur = s % 2; NEXT: stage s + 1 exists.
+    auto stage = [&](int s, auto cur_c, auto next_c) {
         constexpr bool NEXT = decltype(next_c)::value;
-        const int cur = s & 1;
+        constexpr int cur = decltype(cur_c)::value;
         const int ld = s + 2 < nsteps ? s + 2 : s + 1;  // (past the end: not used)
         auto convert = [&](int i) {
-            if (NEXT && i < P::kPieces) {
-                store_piece(i, s + 1, cur ^ 1);
+            if (NEXT && i < kPieces) {
+                store_piece(i, cur ^ 1);
                 load_piece(i, ld);
             }
         };
         // A group's reads, then its MFMAs with the conversion's vector work
         // between them; its loads leave with it (left to the compiler they
-        // sank to the stage's end, a group before their use: 380 us for fc1
-        // at 10992 rows against 358).
-        auto group = [&](auto reads, auto conv) {
-            if constexpr (reads.value) __builtin_amdgcn_sched_group_barrier(0x100, 2 + kRB, 0);  // LDS reads
+        // sink to the stage's end, a group before their use).
+        auto group = [&](int reads, auto conv) {
+            if (reads == 1) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS reads
+            if (reads == 2) __builtin_amdgcn_sched_group_barrier(0x100, 2 + kRB, 0);
 #pragma unroll
             for (int q = 0; q < 2 * kRB; q++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
-                if constexpr (NEXT && conv.value) __builtin_amdgcn_sched_group_barrier(0x002, 16 / kRB, 0);  // VALU
+                if constexpr (NEXT && conv.value)
+                    __builtin_amdgcn_sched_group_barrier(0x002, 16 / kRB, 0);  // VALU
             }
             __builtin_amdgcn_sched_barrier(0);
         };
         constexpr std::true_type yes;
         constexpr std::false_type no;
-        read_l(0, cur);
+        read_a(Am, 1, cur);
+        read_b(Bm, 1, cur);
         convert(0);
-        multiply(0, 0);
-        group(yes, yes);
+        multiply(acc, Ah[cur], Bh[cur]);
+        group(2, yes);
         convert(1);
-        multiply(0, 1);
-        group(no, yes);
-        read_h(1, cur);
+        multiply(acl, Am, Bm);
+        group(0, yes);
         convert(2);
-        multiply(0, 2);
-        group(yes, yes);
-        read_l(1, cur);
+        multiply(acl, Am, Bh[cur]);
+        group(0, yes);
+        read_a(Al, 2, cur);
+        read_b(Bl, 2, cur);
         convert(3);
-        multiply(1, 0);
-        group(yes, yes);
-        multiply(1, 1);
-        group(no, no);
+        multiply(acl, Ah[cur], Bm);
+        group(2, yes);
+        multiply(acl, Al, Bh[cur]);
+        group(0, no);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if constexpr (NEXT) read_h(0, cur ^ 1);
-        multiply(1, 2);
-        group(next_c, no);
+        if constexpr (NEXT) {
+            read_a(Ah[cur ^ 1], 0, cur ^ 1);
+            read_b(Bh[cur ^ 1], 0, cur ^ 1);
+        }
+        multiply(acl, Ah[cur], Bl);
+        group(NEXT ? 2 : 0, no);
     };
-    static_assert(P::kPieces <= 4, "one piece per group of multiplies");
-    for (int s = 0; s + 1 < nsteps; s++) step(s, std::true_type{});
-    step(nsteps - 1, std::false_type{});
+    static_assert(kPieces <= 4, "one piece per group of multiplies");
+    constexpr std::integral_constant<int, 0> even;
+    constexpr std::integral_constant<int, 1> uneven;
+    for (int s = 0; s + 2 < nsteps; s += 2) {
+        stage(s, even, std::true_type{});
+        stage(s + 1, uneven, std::true_type{});
+    }
+    stage(nsteps - 2, even, std::true_type{});
+    stage(nsteps - 1, uneven, std::false_type{});
 
-    // a row's four threads are a quad
-    bool bad = false;
-    auto range = [&](float v) {
-        v = fmaxf(v, dpp<kQuadXor1>(v));
-        v = fmaxf(v, dpp<kQuadXor2>(v));
-        bad = bad || v > kSplitMax || (v > 0.0f && v < kSplitMin);
-    };
+    // rows with an element below 2^-100 (a row's four threads are a quad)
 #pragma unroll
-    for (int i = 0; i < P::kPieces; i++) range(mx[i]);
-    if (bad) out_of_range = 1;
+    for (int i = 0; i < kPieces; i++) {
+        if ((mx[i] & 0xFFFFu) > 0x10000u - kSmallest || (mx[i] >> 16) > 0x10000u - kSmallest) {
+            odd[(i < kXP ? P::kPR * i : P::kBM + P::kPR * (i - kXP)) + prow] = 1;
+            any_odd = 1;
+        }
+    }
     __syncthreads();  // also: every wave has left the main loop
-    if (out_of_range == 0) {
+    float bad = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < kRB; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                acc[a][b][r] += acl[a][b][r];
+                bad = fmaf(acc[a][b][r], 0.0f, bad);  // NaN once one is not finite
+            }
+    bool redo = !(bad == 0.0f);
+    if (any_odd != 0)
+        redo = redo || odd[P::kBM + wn + lane] != 0 || (lane < 32 * kRB && odd[wm + lane] != 0);
+    if (__any(redo)) {
+        f32x16 again[2][kRB];
+        f32_block<LN, kRB>(again, x, w, m0 + wm, n0 + wn, M, K, la, l32, hh);
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int b = 0; b < kRB; b++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[a][b][r] = fmaf(acl[a][b][r], 1.0f / 2048.0f, acc[a][b][r]);
-    } else {
-        f32_block<LN, kRB>(acc, x, w, m0 + wm, n0 + wn, M, K, la, l32, hh);
+                for (int r = 0; r < 16; r++) {
+                    const int row = wm + 32 * b + l32, col = wn + 32 * a + 8 * (r / 4) + 4 * hh + r % 4;
+                    if (odd[row] != 0 || odd[P::kBM + col] != 0 || !(fabsf(acc[a][b][r]) <= 3.4028235e38f))
+                        acc[a][b][r] = again[a][b][r];
+                }
     }
+    if constexpr (EPI == EPI_QKV) __syncthreads();  // the stages' LDS is free: see f32_epilogue
     f32_epilogue<EPI, kRB>(acc, reinterpret_cast<float*>(smem_raw), bias, gamma, res, out, m0 + wm, n0 + wn, M, N, wave, lane, qa);
 }
 
@@ -1352,7 +1376,7 @@ constexpr int kF32ColTile = 128;  // columns of an f32 tile: N is a multiple of 
 bool f32_fast(hs_dtype dt, int N, int K, const void* x, const void* w, const float* bias,
               const float* gamma, const void* out, const void* res) {
     // K <= 2^19 keeps a tile's byte offsets (128 rows x K x 4) in 32 bits
-    return dt == HS_F32 && N % kF32ColTile == 0 && K > 0 && K % SplitShape::kBK == 0 &&
+    return dt == HS_F32 && N % kF32ColTile == 0 && K > 0 && K % kSplitKs == 0 &&
            K <= (1 << 19) && aligned16(x) && aligned16(w) && (!bias || aligned16(bias)) &&
            (!gamma || aligned16(gamma)) && aligned16(out) && (!res || aligned16(res));
 }
@@ -1370,9 +1394,9 @@ void launch_split_as(hipStream_t st, const void* x, const void* w, const float* 
 }
 
 // 128 x 128 tiles by two 4-wave workgroups per CU; where one per CU holds
-// them all, by one of 8 waves (2748 rows, fc2: 107 us against 113), and where half
-// the CUs would, in 64 x 128 tiles (1374 rows, fc2: 85 us against 108 and 98).
-// Every shape sums k in one order.
+// them all, by one of 8 waves (2748 rows, fc2: 135 us against 152), and where half
+// the CUs would, in 64 x 128 tiles (1374 rows, fc2: 111 us against 148 and 123).
+// Every shape sums k in one order, and computes the same outputs again.
 template <int EPI, bool LN>
 void launch_split(hipStream_t st, const void* x, const void* w, const float* bias, const float* gamma,
                   const void* res, void* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
@@ -1484,7 +1508,7 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
     if constexpr (EPI == EPI_QKV) {
         return fail(HS_EUNSUPPORTED,
                     "%s: needs K %% %d == 0 (f16) or %% %d == 0 (f32) and 16-byte aligned buffers", op,
-                    kBK, SplitShape::kBK);
+                    kBK, kSplitKs);
     } else {
         const int tiles_n = static_cast<int>(ceil_div(N, kGT));
         const int64_t blocks = ceil_div(M, kGT) * tiles_n;
@@ -1727,7 +1751,7 @@ extern "C" hs_status hs_linear_ln_qkv_heads(hs_stream_t stream, hs_dtype dt, con
                                           nullptr, la))
         return fail(HS_EUNSUPPORTED,
                     "%s: needs K %% %d == 0 (f16) or %% %d == 0 (f32) and 16-byte aligned buffers", op,
-                    kBK, SplitShape::kBK);
+                    kBK, kSplitKs);
     hipStream_t st = static_cast<hipStream_t>(stream);
     rc = hs_layernorm_stats(st, dt, x, workspace, M, k, eps);
     if (rc != HS_OK) return rc;

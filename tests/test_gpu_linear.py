@@ -501,7 +501,7 @@ def _split_operands(m, n, k, seed, w_scale=1.0):
                                  (5000, 3072)])
 @pytest.mark.parametrize("k", [32, 64, 96, 1024])
 def test_linear_f32_split(ctx, m, n, k):
-    """f32 products as three f16 ones: closer to the float64 product than a
+    """f32 products as six bf16 ones: closer to the float64 product than a
     plain f32 chain of k / 2 terms is (relative 2-norm; 2^-24 per rounding, a
     chain's error grows with sqrt(k)), and rows and column parts of a call
     equal the same of a larger one."""
@@ -520,9 +520,7 @@ def test_linear_f32_split(ctx, m, n, k):
 @pytest.mark.parametrize("xs,ws", [(1e-3, 1.0), (200.0, 1e-2), (3000.0, 100.0), (1e-9, 1.0), (1.0, 1e-12),
                                    (1e6, 1.0), (1e20, 1e10)])
 def test_linear_f32_split_ranges(ctx, xs, ws):
-    """Magnitudes inside the f16 pair's range and, below 2^-13 or above 65504 a
-    row, outside it, where a tile is computed again in f32: the same relative
-    error everywhere."""
+    """Operands of any magnitude: the same relative error everywhere."""
     x, w, _ = _split_operands(300, 256, 512, 5)
     x *= xs
     w *= ws
@@ -555,6 +553,96 @@ def test_linear_f32_split_mixed_rows(ctx):
     mag = torch.nan_to_num(x.double(), 0, 0, 0).abs() @ torch.nan_to_num(w.double(), 0, 0, 0).abs().t().contiguous()
     bound = (mag + b.abs()) * 640 ** 0.5 * 2.0 ** -23 + 1e-45
     assert bool(((out - want).abs()[fin] <= bound[fin]).all())
+
+
+def test_linear_f32_split_keeps_every_bit(ctx):
+    """x times the identity is x, bit for bit, over rows whose elements span 2^-100
+    to 2^100, and with elements down to 2^-126, which are computed again."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(2)
+    x = torch.randn((300, 256), generator=g, device="cuda").clamp(-8, 8)
+    x = torch.where(x.abs() < 2.0 ** -10, torch.ones_like(x), x)
+    x *= torch.exp2(torch.randint(-90, 97, x.shape, generator=g, device="cuda").float())
+    x[0, :4] = torch.tensor([1.0, 1e-8, 1e-10, 1e-11])
+    x[1, ::3] = 0
+    x[130, 7], x[131, 8], x[132] = 1e-33, -(2.0 ** -126), 2.0 ** -101
+    x[140, 3], x[141, 4] = torch.finfo(torch.float32).max, -2.0 ** 127
+    eye = torch.eye(256, device="cuda")
+    assert torch.equal(ctx.linear(x, eye), x)
+    xt = x[:256].contiguous()
+    assert torch.equal(ctx.linear(eye, xt), xt.t())
+
+
+@pytest.mark.parametrize("s", [1e-3, 1e-6, 1e-8, 1e-11, 1e-20, 1e-29, 1e-36])
+def test_linear_f32_split_wide_rows(ctx, s):
+    """An ordinary element that the other operand ignores beside small ones:
+    the small ones' sum as precise as if they were alone (f32's precision is
+    relative, 2^-24 per rounding, over chains of k / 2 terms at most)."""
+    k = 512
+    small, other, b = _split_operands(300, 256, k, 3, k ** 0.5)
+    small, other = small * s, other.clone()
+    small[:, 0], other[:, 0] = 1, 0
+    for x, w in ((small, other), (other, small)):
+        want = x.double() @ w.double().t().contiguous()
+        err = (ctx.linear(x, w).double() - want).norm() / want.norm()
+        assert err.item() < 2.0 ** -24 * (1.5 + (k / 2) ** 0.5), (s, err.item())
+
+
+@pytest.mark.parametrize("c", [1 + 2.0 ** -11 - 3 * 2.0 ** -23, 1 + 2.0 ** -9 - 2.0 ** -23, 1 + 2.0 ** -8 + 2.0 ** -17 - 2.0 ** -23,
+                               2 - 2.0 ** -23])
+def test_linear_f32_split_equal_operands(ctx, c):
+    """Every product the same, on values whose parts are largest beside the
+    ones above them, so that nothing averages out: the three terms left out
+    (2^-24) and a rounding each of two k slices, their small products and the
+    final sum (2^-24 each)."""
+    x, w = torch.full((129, 32), c, device="cuda"), torch.full((128, 32), c, device="cuda")
+    want = 32 * (float(np.float32(c)) ** 2)
+    err = ((ctx.linear(x, w).double() - want).abs() / want).max().item()
+    assert err <= 5 * 2.0 ** -24, err
+
+
+def test_linear_f32_split_rows_do_not_see_each_other(ctx):
+    """An output follows its own x and w rows only, whatever shares its tile:
+    beside rows that are computed again (tiny, infinite, NaN, overflowing)
+    every other row keeps its bits, in tiles of 64 and of 128 rows, and the
+    fused q|k|v stays the parts' products."""
+    t, h, k = 1374, 16, 256  # 264 tiles of 128 rows fused, 64-row tiles for a third
+    x, w, b = _split_operands(t, 3 * h * 64, k, 7)
+    odd = x.clone()
+    rows = [70, 71, 200, 1373]
+    odd[70] *= 1e-36
+    odd[71, 5] = float("inf")
+    odd[200, 9] = float("nan")
+    odd[1373] = 3e38
+    ow = w.clone()
+    cols = [65, 1500]
+    ow[65, 3] = 1e-35
+    ow[1500, 3] = float("inf")
+    keep = torch.ones(t, dtype=torch.bool)
+    keep[rows] = False
+    wkeep = torch.ones(w.shape[0], dtype=torch.bool)
+    wkeep[cols] = False
+    part = slice(1024, 2048)
+    for n in (slice(0, 3072), part):
+        clean = ctx.linear(x, w[n], b[n])
+        assert torch.equal(ctx.linear(odd, w[n], b[n])[keep], clean[keep])
+        assert torch.equal(ctx.linear(x, ow[n], b[n])[:, wkeep[n]], clean[:, wkeep[n]])
+    whole = ctx.linear(odd, ow, b)
+    assert torch.equal(ctx.linear(odd, ow[part], b[part]).nan_to_num(7.0), whole[:, part].nan_to_num(7.0))
+    got = ctx.linear_qkv_heads(odd, ow, b, 1, t, h)
+    for i in range(3):
+        want = ctx.split_heads(ctx.linear(odd, ow[i * 1024:(i + 1) * 1024], b[i * 1024:(i + 1) * 1024]), 1, t, h, 64)
+        assert torch.equal(got[i].nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+def test_linear_f32_split_tiny_products(ctx):
+    """Products near the bottom of f32's range (2^-120; their small parts are
+    subnormal) keep f32's relative precision."""
+    x, w, _ = _split_operands(300, 256, 64, 9, 8.0)
+    x, w = x * 2.0 ** -58, w * 2.0 ** -58
+    want = x.double() @ w.double().t().contiguous()
+    err = ((ctx.linear(x, w).double() - want).norm() / want.norm()).item()
+    assert err < 2.0 ** -24 * (1.5 + 32 ** 0.5), err
 
 
 @pytest.mark.parametrize("s,t,h", [(1, 129, 4), (2, 700, 16), (3, 1400, 16)])
