@@ -770,20 +770,19 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
     if (tid < 64) vmax[tid] = 0;
 
     // staging: piece i of the thread is key row 8 W i + tid / 8, dims 8 (tid %
-    // 8) .. + 8; rows past the end read zeros (masked below)
+    // 8) .. + 8; keys past T read row T - 1 (masked below)
     const int prow = tid / 8, pd = 8 * (tid % 8);
     const __amdgpu_buffer_rsrc_t krs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, t * kD * 4, kRawBufferFlags);
     const __amdgpu_buffer_rsrc_t vrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, t * kD * 4, kRawBufferFlags);
-    const uint32_t voff0 = static_cast<uint32_t>((prow * kD + pd) * 4);
     float4 kr[kPc][2], vr[kPc][2];
     auto load = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < kPc; i++) {
-            const int so = (k0 + 8 * W * i) * kD * 4;
-            kr[i][0] = buf_ld(krs, voff0, so), kr[i][1] = buf_ld(krs, voff0 + 16, so);
-            vr[i][0] = buf_ld(vrs, voff0, so), vr[i][1] = buf_ld(vrs, voff0 + 16, so);
+            const uint32_t at = static_cast<uint32_t>((min(k0 + 8 * W * i + prow, t - 1) * kD + pd) * 4);
+            kr[i][0] = buf_ld(krs, at, 0), kr[i][1] = buf_ld(krs, at + 16, 0);
+            vr[i][0] = buf_ld(vrs, at, 0), vr[i][1] = buf_ld(vrs, at + 16, 0);
         }
     };
     bool bad = false;

@@ -484,6 +484,35 @@ def test_attention_f32_split_special_values(ctx):
     assert np.isnan(got[0, 1]).all() and np.isfinite(got[0, 0]).all()
 
 
+@pytest.mark.parametrize("t", [1, 31, 33, 65, 97, 200])
+@pytest.mark.parametrize("s", [1, 300])
+def test_attention_f32_split_reads_its_own_rows(ctx, t, s):
+    """Rows behind the last token (the next head's, and past the last head
+    memory that is not the call's) reach no result: with NaN and infinities
+    there every bit stays."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t)
+    size = s * t * 64
+
+    def guarded(fill):
+        bufs = [torch.full((size + 64 * 128,), fill, device="cuda") for _ in range(3)]
+        return bufs, [b[:size].view(s, 1, t, 64) for b in bufs]
+
+    src = [torch.randn((s, 1, t, 64), generator=g, device="cuda") for _ in range(3)]
+    outs = []
+    for fill in (0.0, float("nan"), float("inf")):
+        _, views = guarded(fill)
+        for a, b in zip(views, src):
+            a.copy_(b)
+        outs.append(ctx.attention(*views))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    if s > 1:  # the next head's rows
+        q, k, v = (a.clone() for a in src)
+        k[1::2] = float("nan")
+        v[1::2] = float("inf")
+        assert torch.equal(ctx.attention(q, k, v)[::2], outs[0][::2])
+
+
 @pytest.mark.parametrize("s,h,t", [(1, 2, 65), (1, 2, 129), (1, 3, 193), (2, 16, 300), (1, 16, 2100),
                                    (1, 40, 1600), (1, 260, 300)])
 @pytest.mark.parametrize("spread", [1.0, 6.0])
