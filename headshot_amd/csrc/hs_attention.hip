@@ -27,7 +27,7 @@
 // XCD, so its K/V stream through that XCD's L2.
 //
 // f32, D = 64 (16-byte aligned buffers): the same transposed flash scheme
-// with each f32 value as two f16 ones (flash_split_kernel).
+// with each f32 value as three bf16 ones (flash_split_kernel).
 //
 // f32, D = 128 (16-byte aligned buffers): attention_d128_kernel.
 //
@@ -148,7 +148,6 @@ __device__ __forceinline__ void qk_scores(f32x16 (&s)[kKB], const f16* kbuf, con
     }
 }
 
-// Keys at or past t score -inf (the partial last tile).
 // The two halves of the wave (lanes l and l ^ 32) exchanged with the gfx950
 // v_permlane32_swap: applied to two copies of v it leaves lane l holding
 // (v[l], v[l + 32]) for l < 32 and (v[l - 32], v[l]) above, so the pair's
@@ -169,6 +168,7 @@ __device__ __forceinline__ float halves_sum(float v) {
 
 __device__ __forceinline__ float xor_lanes(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
+// Keys at or past t score -inf (the partial last tile).
 __device__ __forceinline__ void mask_tail(f32x16 (&s)[kKB], int key0, int t, int hh) {
 #pragma unroll
     for (int kb = 0; kb < kKB; kb++)
@@ -681,76 +681,72 @@ __device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm
 }
 
 // ---------------------------------------------------------------------------
-// f32 flash attention, head_dim 64, on the f16 matrix cores. The f32 matrix
-// instructions run at a sixteenth of the f16 rate; an f32 value is, to 2^-24 of
-// itself, h + l / 2048 with h = f16(a) and l = f16((a - h) 2048), so each
-// product is three f16 products with f32 accumulators (h h in one set, h l
-// and l h in a second that counts 1 / 2048), l l (below 2^-24) left out. Queries
-// are split once, K and V as their tiles are staged, the softmax weights (f32;
-// the row sum adds them unsplit) where the f16 kernel rounds them. The rest is the f16 kernel: W waves of 32
-// queries over shared 64-key tiles, double-buffered (the next tile's rows in
-// registers while the current one computes), S^T = K Q^T, the lazy running
-// max, V^T through the transposing read, O^T += V^T P^T.
+// f32 flash attention, head_dim 64, on the bf16 matrix cores. The f32 matrix
+// instructions run at a sixteenth of the bf16 rate; each value goes in as three
+// bf16 ones (split3) and a product is six of theirs with f32 accumulators, to
+// 2^-24 of it as one f32 rounding. Queries are split once, K and V as their
+// tiles are staged, the softmax weights (f32; the row sum adds them unsplit)
+// where the f16 kernel rounds them. The five small products are summed ahead of
+// the large one in the scores, and in accumulators of their own in the output,
+// so they add no rounding of full size. The rest is the f16 kernel: W waves of
+// 32 queries over shared 64-key tiles, double-buffered (the next tile's rows in
+// registers while the current one computes), S^T = K Q^T, the lazy running max
+// (the reference is 2^kSplitShift below it, so a weight keeps its 24 bits down
+// to 2^-126 of the largest), V^T through the transposing read, O^T += V^T P^T.
 //
-// Both halves keep 11 bits for |a| from 2^-14 to 65504, smaller values an
-// absolute 2^-36. A query or key row, or a V column, whose largest magnitude is
-// above 65504 or below 2^-13 (all zeros apart) would lose more than 2^-23 of it:
-// the workgroup then computes its queries again on the f32 matrix
-// instructions (flash_f32_body).
+// A query above 2^50 in magnitude is computed again on the f32 matrix
+// instructions (flash_f32_body), and so are all queries of a (frame, head) with
+// such a key or value, or with a nonzero value below 2^-100, where bf16's last
+// part ends (from 2^-134 up; smaller ones count as zero; small queries and keys
+// move a score by less than 2^-60 only). A query's result follows its own row
+// and its head's K and V, and nothing else in its workgroup.
 //
-// Bounds: matrix and vector issue, 48 MFMAs and ~350 vector instructions per
-// wave and tile, which overlap little: two waves per SIMD in step. 16 heads of
-// 1374 tokens, us on the f32 matrix instructions and here: 1 sequence 111, 51;
-// 2, 197, 60; 8, 567, 210 (295 TFLOP/s); with operands read at their use, as the
-// compiler orders them, 55, 67, 215. Relative error against 64 bits 8.6e-7,
-// 3.8e-7.
-constexpr float kSplitMax = 65504.0f, kSplitMin = 0x1p-13f;
+// Bounds: matrix and vector issue, 96 MFMAs and ~600 vector instructions per
+// wave and tile, which overlap little: two waves per SIMD in step (one with 4
+// waves). 16 heads of 1374 tokens, us on the f32 matrix instructions and here: 1
+// sequence 109, 71; 2, 198, 91; 8, 565, 320 (193 TFLOP/s). With two f16 parts
+// and three products 51, 64, 212, but those keep no value or weight below
+// 2^-36. Relative error against 64 bits 8.7e-7 and 3.2e-7. Eight sequences with
+// such a value in every head, all computed twice: 950.
+constexpr float kSplitMax = 0x1p50f;
+constexpr float kSplitScale = 0x1p23f;
+constexpr uint32_t kSplitSmall = 0x1B00;  // twice the bf16 bits of 2^-100
 
-template <int W>
 struct SplitFlashSmem {
-    f16 k[2][2][64 * kKPitch];  // [buffer][h, l]
-    f16 v[2][2][64 * kVPitch];
+    uint16_t k[2][3][64 * kKPitch];  // [buffer][h, m, l]
+    uint16_t v[2][3][64 * kVPitch];
 };
 
-// 8 floats as h and l chunks.
-__device__ __forceinline__ void split8(const float4 (&v)[2], u32x4& hi, u32x4& lo) {
+// 8 floats as h, m and l chunks.
+__device__ __forceinline__ void split8(const float4 (&v)[2], u32x4 (&part)[3]) {
     const float f[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        uint32_t hp = pk_f16(f[2 * i], f[2 * i + 1]);
-        asm("" : "+v"(hp));  // converted once, as a pair
-        const f16x2 h = u2h2(hp);
-        f16x2 l;
-        // a - h is exact in f32
-        l.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, f[2 * i] * 2048.0f));
-        l.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, f[2 * i + 1] * 2048.0f));
-        hi[i] = hp, lo[i] = h22u(l);
+        uint32_t h, m, l;
+        split3(f[2 * i], f[2 * i + 1], h, m, l);
+        part[0][i] = h, part[1][i] = m, part[2][i] = l;
     }
 }
-__device__ __forceinline__ float max8(const float4 (&v)[2]) {
-    return fmaxf(fmaxf(fmaxf(fabsf(v[0].x), fabsf(v[0].y)), fmaxf(fabsf(v[0].z), fabsf(v[0].w))),
-                 fmaxf(fmaxf(fabsf(v[1].x), fabsf(v[1].y)), fmaxf(fabsf(v[1].z), fabsf(v[1].w))));
+__device__ __forceinline__ float max8(float mx, const float4 (&v)[2]) {
+    mx = fmaxf(fmaxf(mx, fabsf(v[0].x)), fabsf(v[0].y));
+    mx = fmaxf(fmaxf(mx, fabsf(v[0].z)), fabsf(v[0].w));
+    mx = fmaxf(fmaxf(mx, fabsf(v[1].x)), fabsf(v[1].y));
+    return fmaxf(fmaxf(mx, fabsf(v[1].z)), fabsf(v[1].w));
 }
-// Buffer descriptor word 3 for raw (unstructured, stride 0) buffers on gfx950.
-constexpr int kRawBufferFlags = 0x00020000;
-__device__ __forceinline__ float4 buf_ld(__amdgpu_buffer_rsrc_t src, uint32_t voff, int soff) {
-    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
-}
-__device__ __forceinline__ bool split_unfit(float mx) { return mx > kSplitMax || (mx > 0.0f && mx < kSplitMin); }
+__device__ __forceinline__ bf16x8 as_bf8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 template <int W>
-__global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
+__global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     float* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c, int token_major) {
     constexpr int kThr = 64 * W, kPc = 64 * 8 / kThr;  // 8-float pieces per thread of a K or V tile
     union Smem {
-        SplitFlashSmem<W> split;
+        SplitFlashSmem split;
         F32FlashSmem f32;
     };
     __shared__ __align__(16) Smem smem;
-    __shared__ int unfit;
-    __shared__ uint32_t vmax[64];  // bits of the largest |V| per dim
-    SplitFlashSmem<W>& sm = smem.split;
+    __shared__ int again;  // bit 0: every query of the workgroup, bit 1: some
+    SplitFlashSmem& sm = smem.split;
     // the f16 kernel's XCD-aware order
     const int b = blockIdx.x;
     const int slot = b / kXcds;
@@ -766,67 +762,63 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
     const float* vb = v + base;
     const int qi = qt * 32 * W + wave * 32 + n;
     const bool live = qt * 32 * W + wave * 32 < t;  // wave-uniform: some query below T
-    if (tid == 0) unfit = 0;
-    if (tid < 64) vmax[tid] = 0;
+    if (tid == 0) again = 0;
 
     // staging: piece i of the thread is key row 8 W i + tid / 8, dims 8 (tid %
     // 8) .. + 8; keys past T read row T - 1 (masked below)
     const int prow = tid / 8, pd = 8 * (tid % 8);
-    const __amdgpu_buffer_rsrc_t krs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, t * kD * 4, kRawBufferFlags);
-    const __amdgpu_buffer_rsrc_t vrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, t * kD * 4, kRawBufferFlags);
     float4 kr[kPc][2], vr[kPc][2];
     auto load = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < kPc; i++) {
-            const uint32_t at = static_cast<uint32_t>((min(k0 + 8 * W * i + prow, t - 1) * kD + pd) * 4);
-            kr[i][0] = buf_ld(krs, at, 0), kr[i][1] = buf_ld(krs, at + 16, 0);
-            vr[i][0] = buf_ld(vrs, at, 0), vr[i][1] = buf_ld(vrs, at + 16, 0);
+            const int64_t at = static_cast<int64_t>(min(k0 + 8 * W * i + prow, t - 1)) * kD + pd;
+            kr[i][0] = ld_f32x4(kb + at), kr[i][1] = ld_f32x4(kb + at + 4);
+            vr[i][0] = ld_f32x4(vb + at), vr[i][1] = ld_f32x4(vb + at + 4);
         }
     };
-    bool bad = false;
-    float vm[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float mx = 0.0f;      // largest |K| and |V| seen
+    uint32_t small = 0;   // largest 2 bits(h) - kSplitSmall of V, mod 2^16, in two halves
+    uint32_t two = 0x00020002u, less = (0x10000u - kSplitSmall) * 0x00010001u;
+    asm("" : "+v"(two), "+v"(less));
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < kPc; i++) {
             const int row = 8 * W * i + prow;
-            u32x4 h, l;
-            split8(kr[i], h, l);
-            st16(&sm.k[buf][0][row * kKPitch + pd], h);
-            st16(&sm.k[buf][1][row * kKPitch + pd], l);
-            // the row's eight threads are an aligned group of eight lanes
-            float mx = max8(kr[i]);
-            mx = fmaxf(mx, dpp<kQuadXor1>(mx));
-            mx = fmaxf(mx, dpp<kQuadXor2>(mx));
-            mx = fmaxf(mx, dpp<kRowHalfMirror>(mx));
-            bad = bad || split_unfit(mx);
-            split8(vr[i], h, l);
-            st16(&sm.v[buf][0][row * kVPitch + pd], h);
-            st16(&sm.v[buf][1][row * kVPitch + pd], l);
-            const float f[8] = {vr[i][0].x, vr[i][0].y, vr[i][0].z, vr[i][0].w,
-                                vr[i][1].x, vr[i][1].y, vr[i][1].z, vr[i][1].w};
+            u32x4 part[3];
+            split8(kr[i], part);
 #pragma unroll
-            for (int e = 0; e < 8; e++) vm[e] = fmaxf(vm[e], fabsf(f[e]));
+            for (int p = 0; p < 3; p++) st16(&sm.k[buf][p][row * kKPitch + pd], part[p]);
+            split8(vr[i], part);
+#pragma unroll
+            for (int p = 0; p < 3; p++) st16(&sm.v[buf][p][row * kVPitch + pd], part[p]);
+            mx = max8(max8(mx, kr[i]), vr[i]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t h = part[0][e];
+                uint32_t d;
+                asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(d) : "v"(h), "v"(two), "v"(less));
+                asm("v_pk_max_u16 %0, %1, %2" : "=v"(small) : "v"(d), "v"(small));
+            }
         }
     };
     load(0);
 
     // Q^T as the B operand: lane (n, hh) holds dims 16 ks + 8 hh .. + 8 of its
     // query (past T: row T - 1, not stored)
-    h8 qh[4], ql[4];
+    u32x4 qp[3][4];
+    bool bad_q;
     {
         const float* qrow = q + base + static_cast<int64_t>(min(qi, t - 1)) * kD + 8 * hh;
-        float mx = 0.0f;
+        float qmx = 0.0f;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             const float4 f[2] = {ld_f32x4(qrow + 16 * ks), ld_f32x4(qrow + 16 * ks + 4)};
-            u32x4 h, l;
-            split8(f, h, l);
-            qh[ks] = as_h8(h), ql[ks] = as_h8(l);
-            mx = fmaxf(mx, max8(f));
+            u32x4 part[3];
+            split8(f, part);
+            qp[0][ks] = part[0], qp[1][ks] = part[1], qp[2][ks] = part[2];
+            qmx = max8(qmx, f);
         }
-        bad = split_unfit(halves_max(mx));
+        bad_q = halves_max(qmx) > kSplitMax;
     }
 
     f32x16 o[2] = {f32x16{}, f32x16{}}, ol[2] = {f32x16{}, f32x16{}};
@@ -838,44 +830,46 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
         const int cur = j & 1;
         if (j + 1 < ntiles) load((j + 1) * 64);
         if (live) {
-            f32x16 s[kKB], sl[kKB];
+            f32x16 s[kKB];
             const f32x16 z = {};
-            const f16* a0 = sm.k[cur][0] + n * kKPitch + 8 * hh;
-            const f16* a1 = sm.k[cur][1] + n * kKPitch + 8 * hh;
-            // h operands are read a 16-dim slice ahead, l operands under the
-            // slice's h products
-            h8 kh[2][kKB], kl[kKB];
-            auto read_k = [&](h8(&dst)[kKB], const f16* src, int ks) {
+            const int koff = n * kKPitch + 8 * hh;
+            auto read_k = [&](u32x4(&dst)[kKB], int part, int ks) {
 #pragma unroll
-                for (int kb2 = 0; kb2 < kKB; kb2++) dst[kb2] = as_h8(ld16(src + 32 * kb2 * kKPitch + 16 * ks));
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+                    dst[kb2] = ld16(sm.k[cur][part] + koff + 32 * kb2 * kKPitch + 16 * ks);
             };
-            read_k(kh[0], a0, 0);
+            auto score = [&](const u32x4(&kk)[kKB], const u32x4& qq, bool first) {
+#pragma unroll
+                for (int kb2 = 0; kb2 < kKB; kb2++)
+                    s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(kk[kb2]), as_bf8(qq), first ? z : s[kb2], 0, 0, 0);
+            };
+            // The small products slice by slice (h read a slice ahead, m and l
+            // under the products before theirs), then h h.
+            u32x4 kh[2][kKB], km[kKB], kl[kKB];
+            read_k(kh[0], 0, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, kKB, 0);  // LDS reads
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) {
-                read_k(kl, a1, ks);
-                if (ks < 3) read_k(kh[(ks + 1) & 1], a0, ks + 1);
-#pragma unroll
-                for (int kb2 = 0; kb2 < kKB; kb2++)
-                    s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks & 1][kb2], qh[ks], ks ? s[kb2] : z, 0, 0, 0);
-#pragma unroll
-                for (int kb2 = 0; kb2 < kKB; kb2++)
-                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks & 1][kb2], ql[ks], ks ? sl[kb2] : z, 0, 0, 0);
-#pragma unroll
-                for (int kb2 = 0; kb2 < kKB; kb2++)
-                    sl[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[kb2], qh[ks], sl[kb2], 0, 0, 0);
-                if (ks < 3)
-                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kKB, 0);
-                else
-                    __builtin_amdgcn_sched_group_barrier(0x100, kKB, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 3 * kKB, 0);  // MFMAs
+                read_k(km, 1, ks);
+                read_k(kl, 2, ks);
+                read_k(kh[(ks + 1) & 1], 0, (ks + 1) & 3);  // after the last slice, slice 0 for h h
+                score(kh[ks & 1], qp[1][ks], ks == 0);
+                score(kh[ks & 1], qp[2][ks], false);
+                score(km, qp[1][ks], false);
+                score(km, qp[0][ks], false);
+                score(kl, qp[0][ks], false);
+                __builtin_amdgcn_sched_group_barrier(0x100, 3 * kKB, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 5 * kKB, 0);  // MFMAs
             }
 #pragma unroll
-            for (int kb2 = 0; kb2 < kKB; kb2++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) s[kb2][r] = fmaf(sl[kb2][r], 1.0f / 2048.0f, s[kb2][r]);
+            for (int ks = 0; ks < 4; ks++) {
+                if (ks < 3) read_k(kh[(ks + 1) & 1], 0, ks + 1);
+                score(kh[ks & 1], qp[0][ks], false);
+                if (ks < 3) __builtin_amdgcn_sched_group_barrier(0x100, kKB, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, kKB, 0);
+            }
             if ((j + 1) * 64 > t) mask_tail(s, j * 64, t, hh);
-            u32x4 ph[kKB][2], pl[kKB][2];
+            u32x4 wp[3][kKB][2];
             // the weights against reference ref, split, and their sum
             auto weights = [&](float ref) {
                 float ps[2] = {0.0f, 0.0f};
@@ -886,34 +880,31 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
                         float p[2];
 #pragma unroll
                         for (int e = 0; e < 2; e++) {
-                            p[e] = __builtin_amdgcn_exp2f(fmaf(s[kb2][2 * w + e], c, -ref));
+                            p[e] = kSplitScale * __builtin_amdgcn_exp2f(fmaf(s[kb2][2 * w + e], c, -ref));
                             ps[e] += p[e];
                         }
-                        uint32_t hp = pk_f16(p[0], p[1]);
-                        asm("" : "+v"(hp));
-                        const f16x2 h = u2h2(hp);
-                        f16x2 lw;
-                        lw.x = static_cast<f16>(fmaf(static_cast<float>(h.x), -2048.0f, p[0] * 2048.0f));
-                        lw.y = static_cast<f16>(fmaf(static_cast<float>(h.y), -2048.0f, p[1] * 2048.0f));
-                        ph[kb2][w / 4][w % 4] = hp, pl[kb2][w / 4][w % 4] = h22u(lw);
+                        uint32_t h, md, lo;
+                        split3(p[0], p[1], h, md, lo);
+                        wp[0][kb2][w / 4][w % 4] = h, wp[1][kb2][w / 4][w % 4] = md, wp[2][kb2][w / 4][w % 4] = lo;
                     }
                 return ps[0] + ps[1];
             };
             // as in the f16 kernel: the tile's max only on the first tile and
-            // where a weight against the kept reference might pass 2^15
+            // where a weight against the kept reference might pass 2^15 times
+            // the largest at it
             bool max_path = j == 0;
             if (!max_path) {
                 const float ps = weights(m);
-                max_path = __any(!(ps <= kRowSumMax));
+                max_path = __any(!(ps <= kRowSumMax * kSplitScale));
                 if (!max_path) l += ps;
             }
             if (max_path) {
-                float mx = s[0][0];
+                float sx = s[0][0];
 #pragma unroll
                 for (int kb2 = 0; kb2 < kKB; kb2++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[kb2][r]);
-                const float m_cand = fmaxf(m, halves_max(mx) * c);
+                    for (int r = 0; r < 16; r++) sx = fmaxf(sx, s[kb2][r]);
+                const float m_cand = fmaxf(m, halves_max(sx) * c);
                 const float m_new = m_cand > m + kLazyMax ? m_cand : m;
                 const float corr = __builtin_amdgcn_exp2f(m - m_new);
                 l = fmaf(l, corr, weights(m_new));
@@ -923,84 +914,79 @@ __global__ __launch_bounds__(64 * W, 2) void flash_split_kernel(
             }
             const int lane16 = n & 15, c0 = n & 16;
             const int voff = (4 * hh + lane16 / 4) * kVPitch + c0 + 4 * (lane16 % 4);
-            // 16 keys at a time, V's h operands read a group ahead, its l
-            // operands under the group's h products
-            h8 vh[2][2], vl[2];  // [channel block]
-            auto read_v = [&](h8(&dst)[2], const f16* src, int g) {
+            auto read_v = [&](u32x4(&dst)[2], int part, int g) {
 #pragma unroll
                 for (int mb = 0; mb < 2; mb++) {
-                    const f16* r0 = src + voff + 16 * g * kVPitch + 32 * mb;
+                    const uint16_t* r0 = sm.v[cur][part] + voff + 16 * g * kVPitch + 32 * mb;
                     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)r0);
                     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(r0 + 8 * kVPitch));
                     const u32x2 wl = __builtin_bit_cast(u32x2, lo), wh = __builtin_bit_cast(u32x2, hi);
-                    u32x4 w;
-                    w[0] = wl[0], w[1] = wl[1], w[2] = wh[0], w[3] = wh[1];
-                    dst[mb] = as_h8(w);
+                    dst[mb][0] = wl[0], dst[mb][1] = wl[1], dst[mb][2] = wh[0], dst[mb][3] = wh[1];
                 }
             };
-            read_v(vh[0], sm.v[cur][0], 0);
+            auto add = [&](f32x16(&acc)[2], const u32x4(&vv)[2], const u32x4& w) {
+#pragma unroll
+                for (int mb = 0; mb < 2; mb++)
+                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(vv[mb]), as_bf8(w), acc[mb], 0, 0, 0);
+            };
+            // 16 keys at a time, V's h read a group ahead, m and l under the
+            // products before theirs
+            u32x4 vh[2][2], vm[2], vl[2];  // [channel block]
+            read_v(vh[0], 0, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
 #pragma unroll
             for (int g = 0; g < 2 * kKB; g++) {
-                read_v(vl, sm.v[cur][1], g);
-                if (g + 1 < 2 * kKB) read_v(vh[(g + 1) & 1], sm.v[cur][0], g + 1);
-                const h8 wh = as_h8(ph[g / 2][g % 2]), wl = as_h8(pl[g / 2][g % 2]);
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++)
-                    o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[g & 1][mb], wh, o[mb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++)
-                    ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[g & 1][mb], wl, ol[mb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++)
-                    ol[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[mb], wh, ol[mb], 0, 0, 0);
+                read_v(vm, 1, g);
+                read_v(vl, 2, g);
+                if (g + 1 < 2 * kKB) read_v(vh[(g + 1) & 1], 0, g + 1);
+                const u32x4 wh = wp[0][g / 2][g % 2], wm = wp[1][g / 2][g % 2], wl = wp[2][g / 2][g % 2];
+                add(o, vh[g & 1], wh);
+                add(ol, vh[g & 1], wm);
+                add(ol, vh[g & 1], wl);
+                add(ol, vm, wm);
+                add(ol, vm, wh);
+                add(ol, vl, wh);
                 if (g + 1 < 2 * kKB)
-                    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
                 else
-                    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);  // MFMAs
+                    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);  // MFMAs
             }
         }
         if (j + 1 < ntiles) stage(cur ^ 1);
         __syncthreads();
     }
 
-    // lanes 8 apart hold the same dims
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        float x = vm[e];
-#pragma unroll
-        for (int mask = 8; mask < 64; mask *= 2) x = fmaxf(x, xor_lanes(x, mask));
-        if (lane < 8) atomicMax(&vmax[pd + e], f2u(x));
-    }
-    if (bad) unfit = 1;
+    const bool bad_kv = mx > kSplitMax || (small & 0xFFFFu) > 0x10000u - kSplitSmall ||
+                        (small >> 16) > 0x10000u - kSplitSmall;
+    if (bad_kv || bad_q) atomicOr(&again, (bad_kv ? 1 : 0) | (bad_q ? 2 : 0));
     __syncthreads();
-    if (tid < 64 && split_unfit(u2f(vmax[tid]))) unfit = 1;
-    __syncthreads();
-    float lsum;
-    if (unfit == 0) {
-        lsum = halves_sum(l);
-#pragma unroll
-        for (int mb = 0; mb < 2; mb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) o[mb][r] = fmaf(ol[mb][r], 1.0f / 2048.0f, o[mb][r]);
-    } else {
-        lsum = flash_f32_body<W>(o, smem.f32, q + base, kb, vb, qi, t, c, tid, n, hh);
-    }
-    if (qi >= t) return;  // after the last barrier
     float* orow = token_major
                       ? out + ((static_cast<int64_t>(sh / heads) * t + qi) * heads + sh % heads) * kD
                       : out + base + static_cast<int64_t>(qi) * kD;
-    const float inv = 1.0f / lsum;
+    auto store = [&](float lsum) {
+        const float inv = 1.0f / lsum;
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+                u32x4 w;
+#pragma unroll
+                for (int e = 0; e < 4; e++) w[e] = f2u(o[mb][4 * r4 + e] * inv);
+                st16(orow + 32 * mb + 8 * r4 + 4 * hh, w);
+            }
+    };
+    const bool redo = (again & 1) != 0 || bad_q;
+    const float lsum = halves_sum(l);
 #pragma unroll
     for (int mb = 0; mb < 2; mb++)
 #pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) {
-            u32x4 w;
-#pragma unroll
-            for (int e = 0; e < 4; e++) w[e] = f2u(o[mb][4 * r4 + e] * inv);
-            st16(orow + 32 * mb + 8 * r4 + 4 * hh, w);
-        }
+        for (int r = 0; r < 16; r++) o[mb][r] += ol[mb][r];
+    if (qi < t && !redo) store(lsum);
+    if (again != 0) {  // workgroup-uniform
+        const float l2 = flash_f32_body<W>(o, smem.f32, q + base, kb, vb, qi, t, c, tid, n, hh);
+        if (qi < t && redo) store(l2);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1141,13 +1127,13 @@ hs_status check_attention(const char* op, hs_dtype dt, const void* q, const void
     return HS_OK;
 }
 
-// False where the grid, or the byte offsets within a (frame, head), would not fit.
+// False where the grid would not fit.
 template <int W>
 bool launch_split(hipStream_t st, const void* q, const void* k, const void* v, void* out, int sh, int h, int t,
                   float scale, int token_major) {
     const int qtiles = static_cast<int>(ceil_div(t, 32 * W));
     const int64_t blocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * qtiles;
-    if (blocks >= (int64_t{1} << 31) / (64 * W) || t > (1 << 22)) return false;
+    if (blocks >= (int64_t{1} << 31) / (64 * W)) return false;
     flash_split_kernel<W><<<dim3(static_cast<uint32_t>(blocks)), dim3(64 * W), 0, st>>>(
         static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
         static_cast<float*>(out), sh, h, t, qtiles, scale * 1.4426950408889634f, token_major);
@@ -1203,12 +1189,11 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
     }
     if (dt == HS_F32 && d == kD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
         // 128 queries per workgroup while one per CU holds them all (16
-        // heads of 1374 tokens: 51 us against 60), 256 beyond (32 heads: 108
-        // against 64).
+        // heads of 1374 tokens: 71 us against 90), 256 beyond (32 heads: 140
+        // against 102).
         const bool few = static_cast<int64_t>(sh) * ceil_div(t, 128) <= num_cus();
         if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
-                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major) ||
-                      launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major))
+                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
             return check_launch("attention");
     }
     if (dt == HS_F32 && d == kHD && sh <= 65535 && aligned16(q) && aligned16(k) && aligned16(v) &&

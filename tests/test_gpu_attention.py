@@ -430,8 +430,8 @@ def test_attention_f32_split_edges(ctx, s, h, t, spread):
 @pytest.mark.parametrize("what", ["q", "k", "v", "vcol", "qrow", "krow"])
 @pytest.mark.parametrize("scale", [1e-8, 1e6])
 def test_attention_f32_split_ranges(ctx, what, scale):
-    """Values outside the f16 pair's range (a whole operand, one V column, one
-    query or key row) take the f32 instructions: the same relative error."""
+    """Operands, V columns, query and key rows of any magnitude: the same
+    relative error."""
     rng = np.random.default_rng(4)
     q, k, v = (rng.standard_normal((1, 3, 300, 64)).astype(np.float32) for _ in range(3))
     if what == "q":
@@ -482,6 +482,84 @@ def test_attention_f32_split_special_values(ctx):
     k[0, 1, 9, 2] = np.nan
     got = back(ctx.attention(dev(q), dev(k), dev(v)))
     assert np.isnan(got[0, 1]).all() and np.isfinite(got[0, 0]).all()
+
+
+@pytest.mark.parametrize("near,far,gap", [(1e-3, 6e4, 22.0), (1e-9, 1.0, 30.0), (1e-20, 1e-3, 60.0),
+                                          (1e-28, 1e2, 65.0)])
+@pytest.mark.parametrize("t", [200, 1374])
+def test_attention_f32_split_wide_values(ctx, near, far, gap, t):
+    """Large values under small weights beside small values under large ones:
+    each weight and each value enters with f32's relative precision. A score is
+    up to A = gap / ln 2 + 20 log2 units large; four accumulations of it and the
+    exponent's argument round it by 2^-24 of that each, which is 5 ln 2 2^-24 A
+    of the weight, below 2^-22 A (all weights are above 2^-126, where exp2
+    ends)."""
+    rng = np.random.default_rng(t)
+    q, k, v = (rng.standard_normal((1, 8, t, 64)).astype(np.float32) for _ in range(3))
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, :, ::2, 0] = -gap  # scores lower by gap
+    v *= np.float32(near)
+    v[:, :, ::2] *= np.float32(far / near)
+    want = naive64(q, k, v)
+    mag = naive64(q, k, np.abs(v))
+    err = np.abs(back(ctx.attention(dev(q), dev(k), dev(v))) - want) / mag
+    assert err.max() < 2.0 ** -22 * (gap / np.log(2) + 20), err.max()
+
+
+@pytest.mark.parametrize("s", [1e-2, 1e-4, 1e-6, 1e-9])
+@pytest.mark.parametrize("swap", [False, True])
+def test_attention_f32_split_wide_rows(ctx, s, swap):
+    """Keys (or queries) with one large element that the other operand ignores
+    and small ones that make the scores."""
+    rng = np.random.default_rng(3)
+    q, k, v = (rng.standard_normal((1, 3, 300, 64)).astype(np.float32) for _ in range(3))
+    a, b = (k, q) if swap else (q, k)
+    a *= np.float32(s)
+    a[..., 5] = 100.0
+    b *= np.float32(1 / s)
+    b[..., 5] = 0.0
+    assert _rel(back(ctx.attention(dev(q), dev(k), dev(v))), naive64(q, k, v)) < 1.2e-6
+
+
+def test_attention_f32_split_one_key_is_its_value(ctx):
+    """One token of score zero (weight one): every bit of its value, over
+    magnitudes of 2^-98 to 2^49, and past both ends, where it is computed
+    again."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    q, k, v = (torch.randn((40, 3, 1, 64), generator=g, device="cuda") for _ in range(3))
+    q.zero_()
+    v = torch.where(v.abs() < 0.5, torch.ones_like(v), v).clamp(-1.9, 1.9)
+    v *= torch.exp2(torch.randint(-97, 49, v.shape, generator=g, device="cuda").float())
+    v[3, 1, 0, 5], v[4, 2, 0, 6], v[5, 0, 0, 0] = 1e-35, 1e30, 0.0
+    assert torch.equal(ctx.attention(q, k, v), v)
+
+
+def test_attention_f32_split_queries_do_not_see_each_other(ctx):
+    """A query's result follows its own row and its head's keys and values:
+    beside queries that are computed again (huge, infinite, NaN) and in any
+    batch (128 and 256 queries per workgroup) it keeps its bits."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    q, k, v = (torch.randn((34, 8, 333, 64), generator=g, device="cuda") for _ in range(3))
+    whole = ctx.attention(q, k, v)
+    for n in (1, 2, 17):
+        assert torch.equal(ctx.attention(q[:n], k[:n], v[:n]), whole[:n]), n
+    odd = q.clone()
+    odd[0, :, 40] *= 1e20
+    odd[0, :, 300, 7] = float("inf")
+    odd[33, 3, 332, 1] = float("nan")
+    keep = torch.ones((34, 8, 333), dtype=torch.bool)
+    keep[0, :, 40] = keep[0, :, 300] = keep[33, 3, 332] = False
+    again = ctx.attention(odd, k, v)
+    assert torch.equal(again[keep], whole[keep])
+    one = ctx.attention(odd[:1], k[:1], v[:1])
+    assert torch.equal(one.nan_to_num(7.0), again[:1].nan_to_num(7.0))
+    v2 = v.clone()
+    v2[1, 2, 9, 3] = 1e-35  # head (1, 2) is computed again, the others not
+    heads = torch.ones((34, 8), dtype=torch.bool)
+    heads[1, 2] = False
+    assert torch.equal(ctx.attention(q, k, v2)[heads], whole[heads])
 
 
 @pytest.mark.parametrize("t", [1, 31, 33, 65, 97, 200])
