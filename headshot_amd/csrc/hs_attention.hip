@@ -892,10 +892,11 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
             // as in the f16 kernel: the tile's max only on the first tile and
             // where a weight against the kept reference might pass 2^15 times
             // the largest at it
-            bool max_path = j == 0;
+            bool own = j == 0, max_path = own;
             if (!max_path) {
                 const float ps = weights(m);
-                max_path = __any(!(ps <= kRowSumMax * kSplitScale));
+                own = !(halves_max(ps) <= kRowSumMax * kSplitScale);
+                max_path = __any(own);
                 if (!max_path) l += ps;
             }
             if (max_path) {
@@ -905,7 +906,9 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
 #pragma unroll
                     for (int r = 0; r < 16; r++) sx = fmaxf(sx, s[kb2][r]);
                 const float m_cand = fmaxf(m, halves_max(sx) * c);
-                const float m_new = m_cand > m + kLazyMax ? m_cand : m;
+                // (only for its own sums, so that a query does not follow the
+                // others of its wave)
+                const float m_new = own && m_cand > m + kLazyMax ? m_cand : m;
                 const float corr = __builtin_amdgcn_exp2f(m - m_new);
                 l = fmaf(l, corr, weights(m_new));
                 m = m_new;

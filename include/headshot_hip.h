@@ -337,7 +337,7 @@ hs_status hs_linear_ln_gelu_noalloc(hs_stream_t stream, hs_dtype dt, const void*
  * Softmax statistics and accumulation are f32. D is 64 (f32 or f16) or 128
  * (f32 only), as the reference's kernel variants; other combinations return
  * HS_EUNSUPPORTED. In f32 products keep f32's precision as in hs_linear. A
- * query's result depends on its own row and its sequence's k and v only. out
+ * sequence's result does not depend on the other sequences of the call. out
  * must not overlap q, k or v. */
 hs_status hs_attention(hs_stream_t stream, hs_dtype dt, const void* q, const void* k,
                        const void* v, void* out, int32_t s, int32_t h, int32_t t, int32_t d);

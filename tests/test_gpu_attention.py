@@ -555,6 +555,14 @@ def test_attention_f32_split_queries_do_not_see_each_other(ctx):
     assert torch.equal(again[keep], whole[keep])
     one = ctx.attention(odd[:1], k[:1], v[:1])
     assert torch.equal(one.nan_to_num(7.0), again[:1].nan_to_num(7.0))
+    # scores that rise along the keys move the running max of some queries only
+    rise = k * torch.linspace(0.5, 6, 333, device="cuda")[:, None]
+    mixed = q * torch.logspace(-2, 0.7, 333, device="cuda")[torch.randperm(333, generator=g, device="cuda")][:, None]
+    both = ctx.attention(mixed, rise, v)
+    for part in (0, 1):
+        some = mixed.clone()
+        some[:, :, part::2] = 0
+        assert torch.equal(ctx.attention(some, rise, v)[:, :, 1 - part::2], both[:, :, 1 - part::2])
     v2 = v.clone()
     v2[1, 2, 9, 3] = 1e-35  # head (1, 2) is computed again, the others not
     heads = torch.ones((34, 8), dtype=torch.bool)
