@@ -36,12 +36,20 @@ def _dt(t: torch.Tensor) -> int:
     raise AssertionError(f"storage must be f32 or f16, got {t.dtype}")
 
 
+# torch.cuda.current_stream() without building its Stream object and looking
+# the device index up through the environment (a large share of a launch's
+# host time: a register block of 7 launches takes 72 us a pass, 97 with it).
+# torch's own compiled code calls these two; a torch without them takes the
+# public call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    """The current device's current stream, as torch.cuda.current_stream()
-    gives it, without building its Stream object and looking the device index
-    up through the environment (a large share of a launch's host time: a
-    register block of 7 launches takes 72 us a pass, 97 so)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    """The current device's current stream as a hipStream_t."""
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 class _Ptr(int):

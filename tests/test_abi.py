@@ -297,3 +297,19 @@ def test_attention_d128_group_limit():
     big = [ctypes.c_void_p(0x10000000 * i) for i in range(1, 5)]
     for f in (L.hs_attention, L.hs_attention_merged):
         assert f(None, F32, *big, 65536, 1, 1, 128) == _lib.HS_EUNSUPPORTED
+
+
+def test_launch_stream_without_the_raw_call(monkeypatch):
+    """A torch without the raw stream call takes the public one."""
+    import torch
+
+    from headshot_amd import context
+
+    class Stream:
+        cuda_stream = 0x1234
+
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    for name in ("_raw_stream", "_raw_device"):
+        with monkeypatch.context() as m:
+            m.setattr(context, name, None)
+            assert context._stream() == 0x1234

@@ -659,3 +659,14 @@ def test_every_op_f16_matches_f32(ctx):
     a32, a16 = both(O.rvec_f16(8, rows * 8).reshape(rows, 8))
     c32, c16 = both(O.rvec_f16(9, rows * 24).reshape(rows, 24))
     close(ctx.concat_channels(a16, c16), ctx.concat_channels(a32, c32), 1e-6, "concat_channels")
+
+
+def test_launch_stream_is_the_current_stream(ctx):
+    """Launches go to torch's current stream, the default one and any other."""
+    from headshot_amd.context import _stream
+
+    side = torch.cuda.Stream()
+    assert _stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert _stream() == side.cuda_stream
+    assert _stream() == torch.cuda.current_stream().cuda_stream != side.cuda_stream
