@@ -361,7 +361,7 @@ class HipContext:
         = (sin, cos, prefix) or None) on q and k. Bit-identical to linear then
         qknorm_rope per third for 8, 16 or 32 heads (within one f16 ulp for
         other head counts); that sequence is what runs for shapes the fused
-        kernel does not cover (f32, head dim other than 64). Returns (q, k, v)."""
+        kernels do not cover (``_qkv_fused``). Returns (q, k, v)."""
         n3, k = w_qkv.shape
         assert n3 % (3 * h) == 0, "w_qkv rows must be 3 * H * d"
         d = n3 // (3 * h)

@@ -710,7 +710,6 @@ __device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm
 // such a value in every head, all computed twice: 950.
 constexpr float kSplitMax = 0x1p50f;
 constexpr float kSplitScale = 0x1p23f;
-constexpr uint32_t kSplitSmall = 0x1B00;  // twice the bf16 bits of 2^-100
 
 struct SplitFlashSmem {
     uint16_t k[2][3][64 * kKPitch];  // [buffer][h, m, l]
@@ -776,10 +775,9 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
             vr[i][0] = ld_f32x4(vb + at), vr[i][1] = ld_f32x4(vb + at + 4);
         }
     };
-    float mx = 0.0f;      // largest |K| and |V| seen
-    uint32_t small = 0;   // largest 2 bits(h) - kSplitSmall of V, mod 2^16, in two halves
-    uint32_t two = 0x00020002u, less = (0x10000u - kSplitSmall) * 0x00010001u;
-    asm("" : "+v"(two), "+v"(less));
+    float mx = 0.0f;  // largest |K| and |V| seen
+    const SplitSmall small;
+    uint32_t small_v = 0;
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < kPc; i++) {
@@ -793,12 +791,7 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
             for (int p = 0; p < 3; p++) st16(&sm.v[buf][p][row * kVPitch + pd], part[p]);
             mx = max8(max8(mx, kr[i]), vr[i]);
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t h = part[0][e];
-                uint32_t d;
-                asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(d) : "v"(h), "v"(two), "v"(less));
-                asm("v_pk_max_u16 %0, %1, %2" : "=v"(small) : "v"(d), "v"(small));
-            }
+            for (int e = 0; e < 4; e++) small.note(part[0][e], small_v);
         }
     };
     load(0);
@@ -960,8 +953,7 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
         __syncthreads();
     }
 
-    const bool bad_kv = mx > kSplitMax || (small & 0xFFFFu) > 0x10000u - kSplitSmall ||
-                        (small >> 16) > 0x10000u - kSplitSmall;
+    const bool bad_kv = mx > kSplitMax || SplitSmall::seen(small_v);
     if (bad_kv || bad_q) atomicOr(&again, (bad_kv ? 1 : 0) | (bad_q ? 2 : 0));
     __syncthreads();
     float* orow = token_major

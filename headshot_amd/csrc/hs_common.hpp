@@ -172,6 +172,25 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
     l = pk_bf16(ra - u2f(m << 16), rb - u2f(m & 0xFFFF0000u));
 }
 
+// Whether a nonzero value below 2^-100 was among those split, from their h: 2
+// bits(h) - kSplitSmall, mod 2^16, is above zero's for those magnitudes (from
+// 2^-134, where h rounds to zero) and for no others, so two instructions per
+// pair keep the largest.
+constexpr uint32_t kSplitSmall = 0x1B00;  // twice the bf16 bits of 2^-100
+
+struct SplitSmall {
+    uint32_t two = 0x00020002u, less = (0x10000u - kSplitSmall) * 0x00010001u;
+    __device__ __forceinline__ SplitSmall() { asm("" : "+v"(two), "+v"(less)); }
+    __device__ __forceinline__ void note(uint32_t h, uint32_t& largest) const {
+        uint32_t t;
+        asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t) : "v"(h), "v"(two), "v"(less));
+        asm("v_pk_max_u16 %0, %1, %2" : "=v"(largest) : "v"(t), "v"(largest));
+    }
+    static __device__ __forceinline__ bool seen(uint32_t largest) {
+        return (largest & 0xFFFFu) > 0x10000u - kSplitSmall || (largest >> 16) > 0x10000u - kSplitSmall;
+    }
+};
+
 // Exact-erf GELU, gelu.wesl:18-38: 0.5*v*(1 + erf(v/sqrt(2))) with erf by
 // Abramowitz & Stegun 7.1.26, erf(z) = sign(z)*(1 - P(t)*t*exp(-z^2)),
 // t = 1/(1 + p*|z|). Evaluated in f32 from h = v/2 (exact), with the

@@ -897,10 +897,6 @@ using SplitEight = SplitTile<4, 2, 1>;   // 128 x 128 by 8 waves
 using SplitNarrow = SplitTile<2, 2, 1>;  // 64 x 128
 constexpr int kSplitKs = 32;             // K is a multiple: stages go in pairs
 
-// Twice the bf16 bits of 2^-100. 2 bits - kSmallest, mod 2^16, is then above the
-// value zero gives for the nonzero magnitudes below 2^-100 and for no others.
-constexpr uint32_t kSmallest = 0x1B00;
-
 __device__ __forceinline__ u32x4 buf_ld16(__amdgpu_buffer_rsrc_t src, uint32_t voff, int soff) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, voff, soff, 0));
 }
@@ -960,11 +956,10 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     // the next stage's pieces and the LayerNorm parameters of their columns
     u32x4 raw[kPieces];
     float4 lw, lb;
-    uint32_t mx[kPieces];  // two 16-bit maxima of 2 bits(h) - kSmallest
+    const SplitSmall small;
+    uint32_t mx[kPieces];
 #pragma unroll
     for (int i = 0; i < kPieces; i++) mx[i] = 0;
-    uint32_t two = 0x00020002u, small = (0x10000u - kSmallest) * 0x00010001u;
-    asm("" : "+v"(two), "+v"(small));
     const int nsteps = K / P::kBK;  // even
     auto load_piece = [&](int i, int s) {
         raw[i] = buf_ld16(i < kXP ? xr : wr, off[i], s * 64);
@@ -984,11 +979,10 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
         u32x2 part[3];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            uint32_t h, m, l, t;
+            uint32_t h, m, l;
             split3(u2f(v[2 * j]), u2f(v[2 * j + 1]), h, m, l);
             part[0][j] = h, part[1][j] = m, part[2][j] = l;
-            asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t) : "v"(h), "v"(two), "v"(small));
-            asm("v_pk_max_u16 %0, %1, %2" : "=v"(mx[i]) : "v"(t), "v"(mx[i]));
+            small.note(h, mx[i]);
         }
 #pragma unroll
         for (int q = 0; q < 3; q++) {
@@ -1106,7 +1100,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     // rows with an element below 2^-100 (a row's four threads are a quad)
 #pragma unroll
     for (int i = 0; i < kPieces; i++) {
-        if ((mx[i] & 0xFFFFu) > 0x10000u - kSmallest || (mx[i] >> 16) > 0x10000u - kSmallest) {
+        if (SplitSmall::seen(mx[i])) {
             odd[(i < kXP ? P::kPR * i : P::kBM + P::kPR * (i - kXP)) + prow] = 1;
             any_odd = 1;
         }

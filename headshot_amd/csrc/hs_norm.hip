@@ -12,13 +12,12 @@
 // row counts beyond 2^22 workgroups): measured against persistent grids of
 // 2-8 workgroups per CU, which walk several row groups per wave, it is the
 // fastest at 44k rows, alone (69.5% of peak against 65.5%) and inside the
-// aggregator pass (72.1% against 69.7%).
+// aggregator pass (72.1% against 69.7%). CHUNKS is 1, 2, 4 or 8; 8 is the
+// camera head's f32 width of 2048 (8 rows in 2.8 us against the generic
+// path's 25).
 //
 // Narrow path (rows of 8 or 16 vectors, e.g. 64-wide f16 QK-norm rows):
 // several rows per wave, each reduced within its group of lanes.
-//
-// (1, 2, 4 or 8 chunks; 8 is the camera head's f32 width of 2048: 8 rows in
-// 2.8 us against the generic path's 25.)
 //
 // Generic path: any dim, one wave per row, strided over the row three
 // times (mean, variance, output) with the second and third reads served by
