@@ -1150,10 +1150,10 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
 // operands; its accumulators are columns 4 g .. + 4 of output row r. The
 // order of the sum depends on K only.
 //
-// At 8 rows (us, beside the 64 x 128 tiles): 2048 x 2048 8.4 (72.7), 8192 x
-// 2048 14.2 (74.7), 2048 x 8192 26 (279), i.e. 2.0-4.7 TB/s of weights; at 100
-// rows 18 (74), 65 (75), 62 (280); above 128 rows wide outputs are faster in
-// tiles (200 rows, 8192 x 2048: 110 against 80).
+// At 8 rows (us, beside the tiles of gemm_split_kernel): 2048 x 2048 8.5 (55),
+// 8192 x 2048 13.4 (53), 2048 x 8192 26 (200), i.e. 2.0-5.0 TB/s of weights; at
+// 128 rows 18 (53), 64 (55), 64 (198); above, wide outputs are faster in tiles
+// (200 rows, 8192 x 2048: 111 against 63).
 constexpr int kSkinnyRows = 128, kSkinnyCols = 1 << 22;
 constexpr int kSkWaves = 16, kSkThreads = 64 * kSkWaves;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
