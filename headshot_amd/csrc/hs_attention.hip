@@ -1158,7 +1158,9 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
             // 1386 29.6, 31.8; 2772 53.2, 57.9). Splitting the keys over wave
             // groups is faster still (1386 18.7) but sums a query in an order
             // that follows the batch: not taken.
-            if (static_cast<int64_t>(sh) * half_tiles <= cus) {
+            // (A sequence's tiles share one XCD: what counts is an XCD's CUs, and
+            // one head of 8000 tokens, 63 workgroups, is past them: 145, 157.)
+            if (seqs * half_tiles <= cus) {
                 flash_f16_kernel<false, FlashHalf><<<dim3(static_cast<uint32_t>(seqs * half_tiles)),
                                                      dim3(FlashHalf::kThreads), 0, st>>>(
                     fq, fk, fv, fo, sh, h, t, half_tiles, c, token_major, 0);
@@ -1186,7 +1188,8 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
         // 128 queries per workgroup while one per CU holds them all (16
         // heads of 1374 tokens: 71 us against 90), 256 beyond (32 heads: 140
         // against 102).
-        const bool few = static_cast<int64_t>(sh) * ceil_div(t, 128) <= num_cus();
+        // (counted by XCD, as above: one head of 8000 tokens 751 us against 490)
+        const bool few = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * ceil_div(t, 128) <= num_cus();
         if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
                 : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
             return check_launch("attention");
