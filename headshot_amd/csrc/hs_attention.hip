@@ -711,9 +711,10 @@ __device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm
 constexpr float kSplitMax = 0x1p50f;
 constexpr float kSplitScale = 0x1p23f;
 
+template <int ST>
 struct SplitFlashSmem {
-    uint16_t k[2][3][64 * kKPitch];  // [buffer][h, m, l]
-    uint16_t v[2][3][64 * kVPitch];
+    uint16_t k[ST][3][64 * kKPitch];  // [buffer][h, m, l]
+    uint16_t v[ST][3][64 * kVPitch];
 };
 
 // 8 floats as h, m and l chunks.
@@ -734,18 +735,20 @@ __device__ __forceinline__ float max8(float mx, const float4 (&v)[2]) {
 }
 __device__ __forceinline__ bf16x8 as_bf8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-template <int W>
-__global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
+// ST: buffers, 2, or 1 for sequences of one tile, whose workgroups then go two
+// to a CU.
+template <int W, int ST>
+__global__ __launch_bounds__(64 * W, (3 - ST) * W / 4) void flash_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     float* __restrict__ out, int sh_count, int heads, int t, int qtiles, float c, int token_major) {
     constexpr int kThr = 64 * W, kPc = 64 * 8 / kThr;  // 8-float pieces per thread of a K or V tile
     union Smem {
-        SplitFlashSmem split;
+        SplitFlashSmem<ST> split;
         F32FlashSmem f32;
     };
     __shared__ __align__(16) Smem smem;
     __shared__ int again;  // bit 0: every query of the workgroup, bit 1: some
-    SplitFlashSmem& sm = smem.split;
+    SplitFlashSmem<ST>& sm = smem.split;
     // the f16 kernel's XCD-aware order
     const int b = blockIdx.x;
     const int slot = b / kXcds;
@@ -817,11 +820,11 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
     f32x16 o[2] = {f32x16{}, f32x16{}}, ol[2] = {f32x16{}, f32x16{}};
     float m = -INFINITY, l = 0.0f;
     stage(0);
-    const int ntiles = static_cast<int>(ceil_div(t, 64));
+    const int ntiles = ST == 2 ? static_cast<int>(ceil_div(t, 64)) : 1;
     __syncthreads();
     for (int j = 0; j < ntiles; j++) {
-        const int cur = j & 1;
-        if (j + 1 < ntiles) load((j + 1) * 64);
+        const int cur = ST == 2 ? j & 1 : 0;
+        if (ST == 2 && j + 1 < ntiles) load((j + 1) * 64);
         if (live) {
             f32x16 s[kKB];
             const f32x16 z = {};
@@ -949,7 +952,7 @@ __global__ __launch_bounds__(64 * W, W / 4) void flash_split_kernel(
                 __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);  // MFMAs
             }
         }
-        if (j + 1 < ntiles) stage(cur ^ 1);
+        if (ST == 2 && j + 1 < ntiles) stage(cur ^ 1);
         __syncthreads();
     }
 
@@ -1123,13 +1126,13 @@ hs_status check_attention(const char* op, hs_dtype dt, const void* q, const void
 }
 
 // False where the grid would not fit.
-template <int W>
+template <int W, int ST>
 bool launch_split(hipStream_t st, const void* q, const void* k, const void* v, void* out, int sh, int h, int t,
                   float scale, int token_major) {
     const int qtiles = static_cast<int>(ceil_div(t, 32 * W));
     const int64_t blocks = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * qtiles;
     if (blocks >= (int64_t{1} << 31) / (64 * W)) return false;
-    flash_split_kernel<W><<<dim3(static_cast<uint32_t>(blocks)), dim3(64 * W), 0, st>>>(
+    flash_split_kernel<W, ST><<<dim3(static_cast<uint32_t>(blocks)), dim3(64 * W), 0, st>>>(
         static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
         static_cast<float*>(out), sh, h, t, qtiles, scale * 1.4426950408889634f, token_major);
     return true;
@@ -1185,13 +1188,16 @@ hs_status launch_attention(hipStream_t st, hs_dtype dt, const void* q, const voi
         }
     }
     if (dt == HS_F32 && d == kD && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
-        // 128 queries per workgroup while one per CU holds them all (16
-        // heads of 1374 tokens: 71 us against 90), 256 beyond (32 heads: 140
-        // against 102).
+        // One buffer, so two workgroups per CU, for sequences of one tile (4096
+        // heads of 33 tokens: 49 us against 95 with 8 waves and two buffers, 81
+        // on the f32 matrix instructions). Else 128 queries per workgroup while
+        // one per CU holds them all (16 heads of 1374 tokens: 71 us against 90),
+        // 256 beyond (32 heads: 140 against 102).
         // (counted by XCD, as above: one head of 8000 tokens 751 us against 490)
         const bool few = static_cast<int64_t>(kXcds) * ceil_div(sh, kXcds) * ceil_div(t, 128) <= num_cus();
-        if (few ? launch_split<4>(st, q, k, v, out, sh, h, t, scale, token_major)
-                : launch_split<8>(st, q, k, v, out, sh, h, t, scale, token_major))
+        if (t <= 64 ? launch_split<4, 1>(st, q, k, v, out, sh, h, t, scale, token_major)
+            : few   ? launch_split<4, 2>(st, q, k, v, out, sh, h, t, scale, token_major)
+                    : launch_split<8, 2>(st, q, k, v, out, sh, h, t, scale, token_major))
             return check_launch("attention");
     }
     if (dt == HS_F32 && d == kHD && sh <= 65535 && aligned16(q) && aligned16(k) && aligned16(v) &&

@@ -412,7 +412,8 @@ def _rel(got, want):
                                    (3, 5, 200), (1, 260, 40), (1, 300, 257), (2, 130, 300)])
 @pytest.mark.parametrize("spread", [1.0, 8.0])
 def test_attention_f32_split_edges(ctx, s, h, t, spread):
-    """flash_split_kernel at the edges of its key tiles (64), query tiles (128
+    """flash_split_kernel at the edges of its key tiles (64; up to there with
+    one buffer), query tiles (128
     and, past 256 of those, 256), and wave-dead tails: f32 precision (2^-24
     per rounding; the scores' spread of up to ~30 log2 units enters the
     weights' relative error)."""
