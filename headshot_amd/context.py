@@ -369,12 +369,14 @@ class HipContext:
         hd = h * d
         if not _qkv_fused(x.dtype, d, n3, k):
             if (s == 1 and qn is None and kn is None and rope is None and out is None
-                    and t * hd * x.element_size() % 16 == 0):
+                    and t * hd * x.element_size() % 16 == 0
+                    and (x.dtype == F16 or t <= 32 or t > 128 or n3 * -(-t // 32) <= 24576)):
                 # One sequence without norms or RoPE (the camera head): q | k |
                 # v of all heads is 3 H heads, so one product and one split
                 # give the three parts as contiguous, aligned views (8 tokens
                 # of width 2048: 17 us of kernels against 37, two launches for
-                # six; the block 117 us against 79).
+                # six; the block 117 us against 79). The last condition: the
+                # whole and the parts take the few-row kernel alike.
                 heads = self.split_heads(self.linear(x, w_qkv, b_qkv), 1, t, 3 * h, d)
                 return tuple(heads[:, i * h:(i + 1) * h] for i in range(3))
             outs = []

@@ -844,8 +844,8 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[2][kRB], const float* x,
 }
 
 // ---------------------------------------------------------------------------
-// f32 products on the bf16 matrix cores (N % 128 == 0, K % 32 == 0, more rows
-// than gemm_skinny_kernel takes). The f32 matrix instructions run at a
+// f32 products on the bf16 matrix cores (N % 128 == 0, K % 32 == 0, the calls
+// that few_rows does not give to gemm_skinny_kernel). The f32 matrix instructions run at a
 // sixteenth of the bf16 rate; an f32 value is the sum of three bf16 ones
 // (split3), a = h + m + l, and six products of those, every one exact in f32,
 //     sum(h h)  +  sum(m m + m h + h m + l h + h l)
@@ -1133,12 +1133,11 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
                         acc[a][b][r] = again[a][b][r];
                 }
     }
-    if constexpr (EPI == EPI_QKV) __syncthreads();  // the stages' LDS is free: see f32_epilogue
     f32_epilogue<EPI, kRB>(acc, reinterpret_cast<float*>(smem_raw), bias, gamma, res, out, m0 + wm, n0 + wn, M, N, wave, lane, qa);
 }
 
 // ---------------------------------------------------------------------------
-// few rows (f32, N % 128 == 0, K % 32 == 0, M <= kSkinnyRows):
+// few rows (f32, N % 128 == 0, K % 32 == 0, few_rows: up to 128):
 // what such a call cannot do without is the weights' way from memory, so the
 // work is split until every CU streams some of them. A workgroup of 16 waves
 // takes 16 CB output columns x 16 RB rows; its waves share K, wave v taking
@@ -1154,7 +1153,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
 // 8192 x 2048 13.4 (53), 2048 x 8192 26 (200), i.e. 2.0-5.0 TB/s of weights; at
 // 128 rows 18 (53), 64 (55), 64 (198); above, wide outputs are faster in tiles
 // (200 rows, 8192 x 2048: 111 against 63).
-constexpr int kSkinnyRows = 128, kSkinnyCols = 1 << 22;
+constexpr int kSkinnyRows = 128;
 constexpr int kSkWaves = 16, kSkThreads = 64 * kSkWaves;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -1403,6 +1402,23 @@ void launch_split(hipStream_t st, const void* x, const void* w, const float* bia
         launch_split_as<EPI, SplitShape, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
 }
 
+// Whether the few-row kernel takes a call: by its shape alone, and so that a
+// product summed in parts of its columns, as q, k and v apart, takes one route
+// with the whole where the whole is promised their bits (8, 16 or 32 heads, i.e.
+// up to 6144 columns). Wide outputs of more than 32 rows make too many
+// workgroups, each reading its weights again: 1024 deep, us here and in tiles:
+// 128 rows, 6144 columns 27, 30; 8192 35, 30; 16384 72, 36; 64 rows, 32768
+// columns 70, 48; 32 rows, 32768 columns 36, 43; q|k|v of 128 rows and 32 heads
+// 35, 34; 64 heads 68, 34.
+template <int EPI>
+bool few_rows(int M, int N) {
+    if (M > kSkinnyRows) return false;
+    if constexpr (EPI == EPI_QKV)
+        return N <= 6144 || N / 64 * ceil_div(M, 16) <= 512;
+    else
+        return N <= 2048 || M <= 32 || N * ceil_div(M, 32) <= 24576;
+}
+
 template <int EPI, int CB, int RB, bool LN>
 void launch_skinny_as(hipStream_t st, const float* x, const float* w, const float* bias, const float* gamma,
                       const float* res, float* out, int M, int N, int K, const LnArgs& la, const QkvArgs& qa) {
@@ -1457,10 +1473,7 @@ hs_status launch(hipStream_t st, hs_dtype dt, const void* x, const void* w, cons
                  const char* op, const QkvArgs& qa = QkvArgs{}, const LnArgs& la = LnArgs{}) {
     if (f32_fast(dt, N, K, x, w, bias, gamma, out, res) &&
         (!LN || (aligned16(la.ln_w) && aligned16(la.ln_b)))) {
-        // (a rule on M alone, so that one product summed in parts of its
-        // columns, as q, k and v apart, takes the same order of k)
-        // (nor would wider outputs fit a grid of few-row workgroups)
-        if (M <= kSkinnyRows && N <= kSkinnyCols)
+        if (few_rows<EPI>(M, N))
             launch_skinny<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);
         else
             launch_split<EPI, LN>(st, x, w, bias, gamma, res, out, M, N, K, la, qa);

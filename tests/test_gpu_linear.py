@@ -431,7 +431,7 @@ def test_linear_f16_tile_shapes_agree(ctx, n, k):
 def test_linear_f32_few_rows(ctx, m, n, k):
     """Up to 128 rows the weights stream through gemm_skinny_kernel (tiles of
     1 to 2 x 1 to 3 blocks of 16, K over 16 waves, some without a piece at
-    small k); 129 rows take the tiles. Every epilogue against float64: f32
+    small k); more, and wide outputs, take the tiles. Every epilogue against float64: f32
     sums of k products (error below k 2^-24 of the sum of magnitudes, which
     is about sqrt(k) of the result's scale), and the parts of a product's
     columns equal to the whole."""
@@ -485,6 +485,43 @@ def test_linear_f32_few_rows_heads_and_prologue(ctx, s, t, norm):
     for a, c in zip(fused, apart):
         assert torch.equal(a, c)
     assert torch.equal(ctx.linear_ln_gelu(x, ln, w, b), ctx.linear_gelu(ctx.layernorm(x, *ln), w, b))
+
+
+@pytest.mark.parametrize("m,n", [(32, 24704), (33, 12288), (33, 12416), (64, 12288), (65, 8192), (65, 8320),
+                                 (96, 8320), (97, 6144), (97, 6272), (128, 2048), (128, 6144), (128, 8192)])
+def test_linear_f32_few_rows_or_wide(ctx, m, n):
+    """Both sides of the line between the few-row kernel and the tiles, every
+    epilogue against float64 (sums of 64 products)."""
+    x, w, b = _split_operands(m, n, 64, m + n)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    gamma, res = (torch.randn(s, generator=g, device="cuda") for s in ((n,), (m, n)))
+    lin = x.double() @ w.double().t().contiguous() + b.double()
+    tol = (x.double().abs() @ w.double().abs().t().contiguous() + 1.0) * 16 * 2.0 ** -23
+    assert bool(((ctx.linear(x, w, b).double() - lin).abs() <= tol).all())
+    # A&S 7.1.26: 1.5e-7 absolute on erf, times |v| / 2
+    gel = torch.nn.functional.gelu(lin)
+    assert bool(((ctx.linear_gelu(x, w, b).double() - gel).abs() <= 1.2 * tol + 2e-7 * (1 + lin.abs())).all())
+    want = res.double() + gamma.double() * lin
+    assert bool(((ctx.linear_ls_residual(x, w, gamma, res, b).double() - want).abs() <= (1 + gamma.abs()) * tol).all())
+
+
+@pytest.mark.parametrize("t", [17, 32, 64, 65, 128])
+@pytest.mark.parametrize("h,d", [(16, 64), (32, 64), (44, 64), (40, 128)])
+def test_linear_f32_few_rows_fused_is_apart(ctx, t, h, d):
+    """q|k|v as one product and as three, over the line between the few-row
+    kernel and the tiles: the same bits for 8, 16 and 32 heads of 64 and for
+    heads of 128 without norms (one product and one split, or three)."""
+    k, hd = 64, h * d
+    x, w, b = _split_operands(t, 3 * hd, k, t + h)
+    got = ctx.linear_qkv_heads(x, w, b, 1, t, h)
+    for i in range(3):
+        part = ctx.linear(x, w[i * hd:(i + 1) * hd], b[i * hd:(i + 1) * hd])
+        want = ctx.split_heads(part, 1, t, h, d)
+        if h == 44:  # 64-wide heads past 32: promised to f32's rounding only
+            assert bool(((got[i] - want).abs() <= 2e-6 * (1 + want.abs())).all())
+        else:
+            assert torch.equal(got[i], want), i
 
 
 def _split_operands(m, n, k, seed, w_scale=1.0):
