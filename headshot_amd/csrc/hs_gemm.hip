@@ -31,7 +31,7 @@
 //
 // f32 (N % 128 == 0, K % 32 == 0; every epilogue, with or without the LayerNorm
 // prologue): each operand as three bf16 values on the bf16 matrix cores
-// (gemm_split_kernel), or up to 128 rows a kernel that splits K over its waves
+// (gemm_split_kernel), or for few rows a kernel that splits K over its waves
 // and streams the weights straight into registers (gemm_skinny_kernel).
 //
 // Generic path (the shapes neither covers): a tiled scalar kernel, f32
