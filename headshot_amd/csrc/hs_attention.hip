@@ -697,8 +697,7 @@ __device__ __forceinline__ float flash_f32_body(f32x16 (&o)[2], F32FlashSmem& sm
 // A query above 2^50 in magnitude is computed again on the f32 matrix
 // instructions (flash_f32_body), and so are all queries of a (frame, head) with
 // such a key or value, or with a nonzero value below 2^-100, where bf16's last
-// part ends (from 2^-134 up; smaller ones count as zero; small queries and keys
-// move a score by less than 2^-60 only). A query's result follows its own row
+// part ends (small queries and keys move a score by less than 2^-60 only). A query's result follows its own row
 // and its head's K and V, and nothing else in its workgroup.
 //
 // Bounds: matrix and vector issue, 96 MFMAs and ~600 vector instructions per
@@ -779,8 +778,7 @@ __global__ __launch_bounds__(64 * W, (3 - ST) * W / 4) void flash_split_kernel(
         }
     };
     float mx = 0.0f;  // largest |K| and |V| seen
-    const SplitSmall small;
-    uint32_t small_v = 0;
+    SplitSmall small;  // of V
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < kPc; i++) {
@@ -794,7 +792,7 @@ __global__ __launch_bounds__(64 * W, (3 - ST) * W / 4) void flash_split_kernel(
             for (int p = 0; p < 3; p++) st16(&sm.v[buf][p][row * kVPitch + pd], part[p]);
             mx = max8(max8(mx, kr[i]), vr[i]);
 #pragma unroll
-            for (int e = 0; e < 4; e++) small.note(part[0][e], small_v);
+            for (int e = 0; e < 2; e++) small.note(vr[i][e].x, vr[i][e].y), small.note(vr[i][e].z, vr[i][e].w);
         }
     };
     load(0);
@@ -956,7 +954,7 @@ __global__ __launch_bounds__(64 * W, (3 - ST) * W / 4) void flash_split_kernel(
         __syncthreads();
     }
 
-    const bool bad_kv = mx > kSplitMax || SplitSmall::seen(small_v);
+    const bool bad_kv = mx > kSplitMax || small.seen();
     if (bad_kv || bad_q) atomicOr(&again, (bad_kv ? 1 : 0) | (bad_q ? 2 : 0));
     __syncthreads();
     float* orow = token_major

@@ -172,23 +172,15 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
     l = pk_bf16(ra - u2f(m << 16), rb - u2f(m & 0xFFFF0000u));
 }
 
-// Whether a nonzero value below 2^-100 was among those split, from their h: 2
-// bits(h) - kSplitSmall, mod 2^16, is above zero's for those magnitudes (from
-// 2^-134, where h rounds to zero) and for no others, so two instructions per
-// pair keep the largest.
-constexpr uint32_t kSplitSmall = 0x1B00;  // twice the bf16 bits of 2^-100
-
+// Whether a nonzero value below 2^-100 is among those noted: 2 bits - 1, mod
+// 2^32, orders the magnitudes with zero last, so three instructions per pair
+// keep the least.
 struct SplitSmall {
-    uint32_t two = 0x00020002u, less = (0x10000u - kSplitSmall) * 0x00010001u;
-    __device__ __forceinline__ SplitSmall() { asm("" : "+v"(two), "+v"(less)); }
-    __device__ __forceinline__ void note(uint32_t h, uint32_t& largest) const {
-        uint32_t t;
-        asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t) : "v"(h), "v"(two), "v"(less));
-        asm("v_pk_max_u16 %0, %1, %2" : "=v"(largest) : "v"(t), "v"(largest));
+    uint32_t least = 0xFFFFFFFFu;
+    __device__ __forceinline__ void note(float a, float b) {
+        least = min(min(least, (f2u(a) << 1) - 1u), (f2u(b) << 1) - 1u);
     }
-    static __device__ __forceinline__ bool seen(uint32_t largest) {
-        return (largest & 0xFFFFu) > 0x10000u - kSplitSmall || (largest >> 16) > 0x10000u - kSplitSmall;
-    }
+    __device__ __forceinline__ bool seen() const { return least < 0x1B000000u - 1u; }  // twice 2^-100's bits
 };
 
 // Exact-erf GELU, gelu.wesl:18-38: 0.5*v*(1 + erf(v/sqrt(2))) with erf by

@@ -854,9 +854,8 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[2][kRB], const float* x,
 // full-size roundings is K / 16 long instead of the f32 instructions' K / 2.
 //
 // The bf16 parts have f32's exponents, so this holds for every |a| from 2^-100
-// up. An output whose x or w row has a smaller nonzero element (from 2^-134 up;
-// below, f32 subnormals count as zero), and one that comes out infinite or NaN,
-// is computed again on v_mfma_f32_32x32x2_f32 (f32_block). That is decided
+// up. An output whose x or w row has a smaller nonzero element, and one that
+// comes out infinite or NaN, is computed again on v_mfma_f32_32x32x2_f32 (f32_block). That is decided
 // for each output by its own two rows, so no result depends on what shares its
 // tile.
 //
@@ -865,7 +864,7 @@ __device__ __forceinline__ void f32_block(f32x16 (&acc)[2][kRB], const float* x,
 // three planes (h, m, l) of 32-byte rows: chunk c (8 floats) of row r at c ^ ((r
 // / 8) % 2), so sixteen rows' reads of a chunk and these writes cover the banks
 // once. The f32 pieces are prefetched into registers and converted once per
-// workgroup between the multiplies (6.5 vector instructions per element).
+// workgroup between the multiplies (7 vector instructions per element).
 // Bounds: matrix issue (six MFMAs where f16 has one) with the conversion
 // beside it. At 10992 rows, q|k|v / proj / fc1 / fc2, us: 390 / 140 / 500 / 486
 // (165-190 TFLOP/s of f32 product) against 586 / 198 / 690 / 722 on the f32
@@ -956,10 +955,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     // the next stage's pieces and the LayerNorm parameters of their columns
     u32x4 raw[kPieces];
     float4 lw, lb;
-    const SplitSmall small;
-    uint32_t mx[kPieces];
-#pragma unroll
-    for (int i = 0; i < kPieces; i++) mx[i] = 0;
+    SplitSmall small[kPieces];
     const int nsteps = K / P::kBK;  // even
     auto load_piece = [&](int i, int s) {
         raw[i] = buf_ld16(i < kXP ? xr : wr, off[i], s * 64);
@@ -982,7 +978,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
             uint32_t h, m, l;
             split3(u2f(v[2 * j]), u2f(v[2 * j + 1]), h, m, l);
             part[0][j] = h, part[1][j] = m, part[2][j] = l;
-            small.note(h, mx[i]);
+            small[i].note(u2f(v[2 * j]), u2f(v[2 * j + 1]));
         }
 #pragma unroll
         for (int q = 0; q < 3; q++) {
@@ -1100,7 +1096,7 @@ __global__ __launch_bounds__(P::kThreads, 2) void gemm_split_kernel(
     // rows with an element below 2^-100 (a row's four threads are a quad)
 #pragma unroll
     for (int i = 0; i < kPieces; i++) {
-        if (SplitSmall::seen(mx[i])) {
+        if (small[i].seen()) {
             odd[(i < kXP ? P::kPR * i : P::kBM + P::kPR * (i - kXP)) + prow] = 1;
             any_odd = 1;
         }

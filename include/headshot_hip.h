@@ -224,11 +224,10 @@ hs_status hs_copy_row_blocks(hs_stream_t stream, const void* src, int64_t src_ro
  * shaders/linear.wesl): out (m, n) = x (m, k) @ w (n, k)^T + bias (n),
  * accumulated in f32, stored in dt. bias (f32) may be NULL. out must not
  * overlap x or w. In f32 each product keeps f32's precision (2^-24 of itself,
- * whatever the other elements of its rows), for elements from 2^-134 in
- * magnitude up; an output depends on its own rows of x and w only, and on m
- * and n only by the order of its sum, which is one for calls of up to 32
- * rows, and of up to 128 with n <= 2048 or n * ceil(m / 32) <= 24576, and
- * another for the rest. */
+ * whatever the other elements of its rows); an output depends on its own rows
+ * of x and w only, and on m and n only by the order of its sum, which is one
+ * for calls of up to 32 rows, and of up to 128 with n <= 2048 or n * ceil(m /
+ * 32) <= 24576, and another for the rest. */
 hs_status hs_linear(hs_stream_t stream, hs_dtype dt, const void* x, const void* w,
                     const float* bias, void* out, int64_t m, int32_t n, int32_t k);
 

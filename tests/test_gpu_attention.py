@@ -533,6 +533,7 @@ def test_attention_f32_split_one_key_is_its_value(ctx):
     v = torch.where(v.abs() < 0.5, torch.ones_like(v), v).clamp(-1.9, 1.9)
     v *= torch.exp2(torch.randint(-97, 49, v.shape, generator=g, device="cuda").float())
     v[3, 1, 0, 5], v[4, 2, 0, 6], v[5, 0, 0, 0] = 1e-35, 1e30, 0.0
+    v[6, 0, 0, 1], v[7, 0, 0, 2] = 1e-39, 2.0 ** -149
     assert torch.equal(ctx.attention(q, k, v), v)
 
 

@@ -594,7 +594,8 @@ def test_linear_f32_split_mixed_rows(ctx):
 
 def test_linear_f32_split_keeps_every_bit(ctx):
     """x times the identity is x, bit for bit, over rows whose elements span 2^-100
-    to 2^100, and with elements down to 2^-126, which are computed again."""
+    to 2^100, and with smaller elements, subnormals among them, which are
+    computed again."""
     g = torch.Generator(device="cuda")
     g.manual_seed(2)
     x = torch.randn((300, 256), generator=g, device="cuda").clamp(-8, 8)
@@ -603,6 +604,7 @@ def test_linear_f32_split_keeps_every_bit(ctx):
     x[0, :4] = torch.tensor([1.0, 1e-8, 1e-10, 1e-11])
     x[1, ::3] = 0
     x[130, 7], x[131, 8], x[132] = 1e-33, -(2.0 ** -126), 2.0 ** -101
+    x[133, 9], x[134, 10], x[135] = 1e-39, 2.0 ** -149, 3e-41
     x[140, 3], x[141, 4] = torch.finfo(torch.float32).max, -2.0 ** 127
     eye = torch.eye(256, device="cuda")
     assert torch.equal(ctx.linear(x, eye), x)
